@@ -38,6 +38,14 @@ int mj_sample_top_k(const float* logits, int64_t ld_logits, int64_t b, int64_t v
                     float temperature, const float* noise, int32_t* token, int32_t* top_idx,
                     float* top_val, void* stream);
 
+/* mj_sample_top_k with a workspace (16-byte aligned, of mj_sample_draw_workspace_bytes bytes), in which
+ * the rows are first cut into segments that many workgroups select from at the same time; same results.
+ * workspace == NULL draws without segments.  Calls may overlap only if they use distinct workspaces. */
+int mj_sample_draw_workspace_bytes(int64_t b, int64_t vocab, int k, size_t* bytes);
+int mj_sample_draw(const float* logits, int64_t ld_logits, int64_t b, int64_t vocab, int k, float temperature,
+                   const float* noise, int32_t* token, int32_t* top_idx, float* top_val,
+                   void* workspace, size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

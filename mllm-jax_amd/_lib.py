@@ -19,7 +19,7 @@ FLAG_DW_BF16 = 1 << 3
 EXPORTS = ("mj_grpo_version", "mj_grpo_last_error", "mj_grpo_workspace_bytes", "mj_grpo_forward",
            "mj_grpo_forward_backward", "mj_grpo_backward", "mj_grpo_forward_noalloc", "mj_grpo_set_trace", "mj_grpo_forward_backward_value",
            "mj_grpo_value_workspace_bytes", "mj_value_head_forward", "mj_grpo_sequence_entropy", "mj_grpo_scale_gradients",
-           "mj_grpo_group_advantages", "mj_grpo_advantages", "mj_grpo_gae", "mj_rmsnorm_forward", "mj_sample_logits", "mj_sample_top_k", "mj_rmsnorm_workspace_bytes", "mj_rmsnorm_backward")
+           "mj_grpo_group_advantages", "mj_grpo_advantages", "mj_grpo_gae", "mj_rmsnorm_forward", "mj_sample_logits", "mj_sample_top_k", "mj_sample_draw", "mj_sample_draw_workspace_bytes", "mj_rmsnorm_workspace_bytes", "mj_rmsnorm_backward")
 
 KERNEL_NAMES = ("k_logits_stats", "k_finalize", "k_dz", "k_dhidden", "k_dhidden_reduce", "k_dw",
                 "k_reduce_loss", "k_scale_hidden", "k_rescue")
@@ -85,6 +85,8 @@ def load() -> C.CDLL:
     lib.mj_grpo_gae.argtypes = [fp, fp, fp, fp, fp, i64, i64, f32, f32, C.c_int, f32, f32, vp]
     lib.mj_sample_logits.argtypes = [vp, i64, vp, i64, fp, i64, i64, i64, i64, f32, vp]
     lib.mj_sample_top_k.argtypes = [fp, i64, i64, i64, C.c_int, f32, fp, ip, ip, fp, vp]
+    lib.mj_sample_draw_workspace_bytes.argtypes = [i64, i64, C.c_int, C.POINTER(sz)]
+    lib.mj_sample_draw.argtypes = [fp, i64, i64, i64, C.c_int, f32, fp, ip, ip, fp, vp, sz, vp]
     lib.mj_rmsnorm_forward.argtypes = [vp, i64, fp, vp, i64, fp, i64, i64, f32, vp]
     lib.mj_rmsnorm_workspace_bytes.argtypes = [i64, i64, C.POINTER(sz)]
     lib.mj_rmsnorm_backward.argtypes = [vp, i64, vp, i64, fp, vp, i64, fp, C.c_int, i64, i64, f32, vp, sz, vp]

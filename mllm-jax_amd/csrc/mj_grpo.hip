@@ -19,6 +19,7 @@
 namespace {
 
 using namespace mj::host;
+static_assert(mj::kSegMax == mj::host::kDrawSegment, "a segment's elements fit the registers of its workgroup");
 static_assert(mj::kValueRows == mj::host::kValueRows, "the plan sizes the value head's partial rows");
 
 // ---- launch tracing (mj_grpo_set_trace): a callback before and after every kernel launch
@@ -587,6 +588,17 @@ int mj_sample_logits(const void* hidden, int64_t ld_hidden, const void* lm_head,
   mj::LogitsRowsArgs a;
   a.w = (const __bf16*)lm_head; a.hid = (const __bf16*)hidden; a.ld_w = ld_w; a.ld_hid = ld_hidden;
   a.V = (int)vocab; a.n = (int)b; a.H = (int)h; a.cap = softcap; a.out = logits; a.ld_out = ld_logits;
+  hipStream_t st = (hipStream_t)stream;
+  // One or two rows go to the vector ALUs: 57.7 -> 51.0 us at 1 x 896 x 151936, 60.0 -> 52.8 at two rows, 184 -> 177
+  // at 1 x 4096 x 128256, 18.7 -> 14.8 at 1 x 904 x 32008.  With four rows their multiply-adds show (57 against
+  // 60 us at the first shape, but 219 against 207 at 3584 x 152064 and 24 against 18 at the last).
+  if (b <= 2) {
+    const unsigned grid = (unsigned)((vocab + 255) / 256);
+    a.units = a.items = 0;
+    if (b == 1) mj::k_logits_few<1><<<grid, 64 * mj::kFewWaves, 0, st>>>(a);
+    else mj::k_logits_few<2><<<grid, 64 * mj::kFewWaves, 0, st>>>(a);
+    return check_launch("k_logits_few");
+  }
   // Batch-row tile and vocab columns per work item: the fewest rounds of resident workgroups (one
   // per CU) whose items are <= 256 columns wide.  Measured at 3584 x 152064: the 128-row tile beats
   // both a 64-row tile with two workgroups per CU (0.25 against 0.23 ms at 64 rows) and, past 128
@@ -594,9 +606,10 @@ int mj_sample_logits(const void* hidden, int64_t ld_hidden, const void* lm_head,
   int bn;
   int64_t tiles_n, tile_rows;
   sample_tiles(b, vocab, &bn, &tiles_n, &tile_rows);
-  a.tile_rows = (int)tile_rows;
-  const mj::TileMap map = mj::TileMap::pick_shape((int)((vocab + tile_rows - 1) / tile_rows), (int)tiles_n, 1, 1);
-  hipStream_t st = (hipStream_t)stream;
+  a.units = (int)((vocab + mj::kRowUnit - 1) / mj::kRowUnit);
+  a.items = (int)((vocab + tile_rows - 1) / tile_rows);
+  if (a.items > a.units) a.items = a.units;
+  const mj::TileMap map = mj::TileMap::pick_shape(a.items, (int)tiles_n, 1, 1);
   if (bn == 128) {
     if ((rc = enable_lds(mj::k_logits_rows<BM, 128>))) return rc;
     mj::k_logits_rows<BM, 128><<<map.items(), mj::kThreads, mj::GemmTN<BM, 128>::kLdsBytes, st>>>(a, map);
@@ -607,8 +620,16 @@ int mj_sample_logits(const void* hidden, int64_t ld_hidden, const void* lm_head,
   return check_launch("k_logits_rows");
 }
 
-int mj_sample_top_k(const float* logits, int64_t ld_logits, int64_t b, int64_t vocab, int k, float temperature,
-                    const float* noise, int32_t* token, int32_t* top_idx, float* top_val, void* stream) {
+int mj_sample_draw_workspace_bytes(int64_t b, int64_t vocab, int k, size_t* bytes) {
+  if (b <= 0 || vocab <= 0 || b > (1 << 24) || vocab > (1 << 30) || k < 1 || k > mj::kTopKMax)
+    return fail(MJ_GRPO_ERR_SHAPE, "sample_draw: bad shape b=%lld vocab=%lld k=%d", (long long)b, (long long)vocab, k);
+  if (bytes) *bytes = draw_segments(b, vocab).bytes(b, k);
+  return MJ_GRPO_OK;
+}
+
+int mj_sample_draw(const float* logits, int64_t ld_logits, int64_t b, int64_t vocab, int k, float temperature,
+                   const float* noise, int32_t* token, int32_t* top_idx, float* top_val,
+                   void* workspace, size_t workspace_bytes, void* stream) {
   if (!logits || !token) return fail(MJ_GRPO_ERR_NULL, "sample_top_k: logits/token is NULL");
   if (b <= 0 || vocab <= 0 || b > (1 << 24) || vocab > (1 << 30) || ld_logits < vocab)
     return fail(MJ_GRPO_ERR_SHAPE, "sample_top_k: bad shape b=%lld vocab=%lld ld=%lld", (long long)b, (long long)vocab, (long long)ld_logits);
@@ -617,8 +638,26 @@ int mj_sample_top_k(const float* logits, int64_t ld_logits, int64_t b, int64_t v
   mj::TopKArgs a;
   a.logits = logits; a.ld = ld_logits; a.V = (int)vocab; a.k = k; a.t = temperature; a.noise = noise;
   a.token = token; a.top_idx = top_idx; a.top_val = top_val;
+  a.words = nullptr; a.counts = nullptr; a.segs = a.seg_len = 0;
+  if (workspace != nullptr) {
+    const DrawSegments g = draw_segments(b, vocab);
+    if (workspace_bytes < g.bytes(b, k))
+      return fail(MJ_GRPO_ERR_WORKSPACE, "sample_draw: workspace too small: %zu < %zu bytes", workspace_bytes, g.bytes(b, k));
+    if (misaligned(workspace)) return fail(MJ_GRPO_ERR_ALIGN, "sample_draw: the workspace must be 16-byte aligned");
+    if (g.segs > 0) {
+      a.segs = g.segs; a.seg_len = g.seg_len;
+      a.words = (uint64_t*)workspace;
+      a.counts = (uint32_t*)((char*)workspace + g.counts_at(b, k));
+      mj::k_topk_segments<<<(unsigned)(b * g.segs), mj::kSegThreads, 0, (hipStream_t)stream>>>(a);
+    }
+  }
   mj::k_topk_sample<<<(unsigned)b, 1024, 0, (hipStream_t)stream>>>(a);
   return check_launch("k_topk_sample");
+}
+
+int mj_sample_top_k(const float* logits, int64_t ld_logits, int64_t b, int64_t vocab, int k, float temperature,
+                    const float* noise, int32_t* token, int32_t* top_idx, float* top_val, void* stream) {
+  return mj_sample_draw(logits, ld_logits, b, vocab, k, temperature, noise, token, top_idx, top_val, nullptr, 0, stream);
 }
 
 }  // extern "C"

@@ -1322,22 +1322,27 @@ struct LogitsRowsArgs {
   float cap;             // final-logit softcap, 0 = off
   float* out;            // [n, ld_out]
   int64_t ld_out;
-  int tile_rows;         // vocab columns per work item: a multiple of 8, <= BM
+  int units, items;      // the vocabulary in units of kRowUnit columns, spread evenly over `items` work items
 };
 
 // A decode batch is a few rows against the whole vocabulary matrix: the product is bound by reading
 // W once.  BN follows the batch (128 or 256 rows, so the MFMA work per slice does not outlast its
-// loads) and a work item covers `tile_rows` <= BM vocab columns, chosen on the host so that the
-// items fill whole rounds of the resident workgroups; the columns of the 256-wide tile past
-// tile_rows are neither loaded (the operand's row limit) nor stored.
+// loads) and a work item covers at most BM vocab columns, as many items as the host chose to fill whole
+// rounds of the resident workgroups; the columns of the 256-wide tile past the item's are neither loaded
+// (the operand's row limit) nor stored.  Items begin at multiples of kRowUnit columns: an item's piece of
+// a k-row is 400 bytes or so out of 300 KB, and a piece that starts in the middle of a 64-byte sector is
+// fetched with the neighbour's bytes around it (128 x 3584 x 152064 in 200-column items: 253 us; in items
+// of 192 and 224 columns: 245).
+constexpr int kRowUnit = 32;
 template <int BM, int BN>
 __global__ __launch_bounds__(kThreads) void k_logits_rows(LogitsRowsArgs p, TileMap map) {
   using G = GemmTN<BM, BN, kKRow, kRowK, (BN < 256 ? 2 : 1)>;   // the narrow tiles wait on memory: three slices in flight
   extern __shared__ __attribute__((aligned(16))) char smem[];
   int tm, tn, split;
   if (!map.tile(blockIdx.x, tm, tn, split)) return;
-  const int m0 = tm * p.tile_rows, n0 = tn * BN;
-  const int m1 = min(p.V, m0 + p.tile_rows);
+  const int base = p.units / p.items, wide = p.units - base * p.items;      // the first `wide` items take one unit more
+  const int m0 = (tm * base + min(tm, wide)) * kRowUnit, n0 = tn * BN;
+  const int m1 = min(p.V, m0 + (base + (tm < wide ? 1 : 0)) * kRowUnit);
   G g;
   g.run(p.w + m0, m1 - m0, p.ld_w, p.hid + (int64_t)n0 * p.ld_hid, p.n - n0, p.ld_hid, p.H, smem);
   const int lane = threadIdx.x & 63;
@@ -1368,12 +1373,87 @@ __global__ __launch_bounds__(kThreads) void k_logits_rows(LogitsRowsArgs p, Tile
   }
 }
 
+// The same product for one or two batch rows.  A matrix tile is 128 rows wide whatever the batch, and a
+// small model's k loop (14 slices at hidden 896) is over before a tile's pipeline has filled.  With NB <= 2
+// the products are few enough for the vector ALUs, so W streams straight into registers: a
+// workgroup owns 256 columns, a wavefront every fourth group of sixteen k-rows of them (lanes 0..31 the even rows,
+// lanes 32..63 the odd ones, 16 bytes each; the next group requested before the current one is used), hidden
+// comes through the constant cache, and the sums of the wavefronts and of their halves meet in the LDS.
+constexpr int kFewWaves = 4;
+template <int NB>
+__global__ __launch_bounds__(64 * kFewWaves) void k_logits_few(LogitsRowsArgs p) {
+  __shared__ __attribute__((aligned(16))) float part[2 * kFewWaves][256];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l31 = lane & 31, odd = lane >> 5;
+  const int col0 = blockIdx.x * 256;
+  const bool inside = col0 + l31 * 8 < p.V;                      // V % 8 == 0
+  const uint32_t ld2 = (uint32_t)p.ld_w * 2;
+  const uint32_t voff = inside ? (uint32_t)l31 * 16 + odd * ld2 : kOob;
+  float acc[NB][8];
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[b][j] = 0.f;
+  const int groups = (p.H + 15) >> 4;
+  auto load = [&](int g, u32x4 (&w)[8]) {                         // rows past the last: rejected, zeros
+    const int left = min(p.H - g * 16, 16);
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc((const char*)(p.w + (int64_t)g * 16 * p.ld_w + col0), left > 0 ? left * (int64_t)ld2 - col0 * 2 : 0);
+#pragma unroll
+    for (int r = 0; r < 8; ++r) w[r] = __builtin_amdgcn_raw_buffer_load_b128(rs, voff, (uint32_t)(2 * r) * ld2, 0);
+  };
+  typedef const __attribute__((address_space(4))) u32x4* const_quads;
+  auto use = [&](int g, const u32x4 (&w)[8]) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      // sixteen hidden values of row b (clamped: a row past n is computed and not stored, so are k-rows past H)
+      const const_quads x = (const_quads)(uintptr_t)(p.hid + (int64_t)min(b, p.n - 1) * p.ld_hid);
+      const u32x4 x0 = x[2 * g], x1 = x[min(2 * g + 1, (p.H >> 3) - 1)];
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        const uint32_t pair = r < 4 ? x0[r] : x1[r - 4];
+        const float h = __uint_as_float(odd ? (pair & 0xffff0000u) : (pair << 16));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          acc[b][2 * j] = fmaf(__uint_as_float(w[r][j] << 16), h, acc[b][2 * j]);
+          acc[b][2 * j + 1] = fmaf(__uint_as_float(w[r][j] & 0xffff0000u), h, acc[b][2 * j + 1]);
+        }
+      }
+    }
+  };
+  u32x4 wa[8], wb[8];
+  load(wave, wa);
+  for (int g = wave; g < groups; g += 2 * kFewWaves) {
+    load(g + kFewWaves, wb);
+    use(g, wa);
+    load(g + 2 * kFewWaves, wa);
+    if (g + kFewWaves < groups) use(g + kFewWaves, wb);
+  }
+  const float inv_cap = p.cap > 0.f ? 1.f / p.cap : 0.f;
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    if (b > 0) __syncthreads();
+    float* mine = &part[wave * 2 + odd][l31 * 8];
+    *(f32x4*)mine = f32x4{acc[b][0], acc[b][1], acc[b][2], acc[b][3]};
+    *(f32x4*)(mine + 4) = f32x4{acc[b][4], acc[b][5], acc[b][6], acc[b][7]};
+    __syncthreads();
+    if (b < p.n && col0 + tid < p.V) {
+      float z = 0.f;
+#pragma unroll
+      for (int q = 0; q < 2 * kFewWaves; ++q) z += part[q][tid];
+      if (p.cap > 0.f) z = softcap_apply(z, p.cap, inv_cap);
+      p.out[(int64_t)b * p.ld_out + col0 + tid] = z;
+    }
+  }
+}
+
 // Top-k + categorical draw per row (MLLM_JAX/sample/sanple_utils.py:35-53): the k largest of
 // logits / t in the IEEE total order (-0 below +0, NaN largest, as XLA's sort comparators order
 // floats; ties: lower index first, like jax.lax.top_k), then argmax_j(top_j + noise_j) where
-// noise holds the caller's Gumbel samples -- what jax.random.categorical evaluates.  One
-// workgroup per row: an 8-bit-per-pass radix select over order-preserving keys finds the k-th
-// largest key, elements above it are collected in any order, elements equal to it in index order.
+// noise holds the caller's Gumbel samples -- what jax.random.categorical evaluates.  With a workspace:
+// k_topk_segments over pieces of the rows, then k_topk_sample over their lists; without one,
+// k_topk_sample alone.  Rows with too many near-equal values around the k-th take a radix select over
+// order-preserving keys: elements above the k-th largest key are collected in any order, elements equal
+// to it in index order.
 constexpr int kTopKMax = 64;
 struct TopKArgs {
   const float* logits;   // [b, ld]
@@ -1384,6 +1464,9 @@ struct TopKArgs {
   int32_t* token;        // [b]
   int32_t* top_idx;      // [b, k] or null
   float* top_val;        // [b, k] or null (logits / t, descending)
+  int segs, seg_len;     // k_topk_segments: pieces of a row and their length (a multiple of 4)
+  uint64_t* words;       // [b, segs, k] each segment's largest, descending; null: no segment pass was run
+  uint32_t* counts;      // [b, segs] how many of the k words are there; kSegOverflow: too many near-equal values
 };
 
 MJ_DEV uint32_t topk_key(float f) {   // larger float <=> larger key; -0 and +0 differ only in sign bit order
@@ -1395,8 +1478,135 @@ MJ_DEV float topk_unkey(uint32_t key) {
   return __uint_as_float((key & 0x80000000u) ? (key ^ 0x80000000u) : ~key);
 }
 
+// One 64-bit word per element whose order is (key descending, index ascending); never 0.
+MJ_DEV uint64_t topk_word(float x, float t, int i) { return ((uint64_t)topk_key(x / t) << 32) | (uint32_t)~i; }
+
+MJ_DEV float nan_max(float a, float b) { return __builtin_elementwise_maximum(a, b); }   // a NaN if either is one
+
+// The k largest of one segment of a row.  One workgroup for a whole row leaves a decode batch of a few
+// sequences on a few CUs, each of them streaming 0.6 MB twice: with segments of 16384 elements a row of
+// 152064 logits is 10 workgroups, the elements stay in registers (8 quads per thread) and are read once.
+// What is left to pay is instructions, so the work per element is a share of its quad's maximum and of one
+// comparison; everything else happens to the few quads that matter, behind an LDS pool.
+// Threshold: the threads form 64 groups of eight; at least k elements reach the k-th largest of the 64 group
+// maxima, `tau`, and few more do (about 100 for k = 50).  x -> key(x / t) is non-decreasing, so the k-th
+// largest key is at least key(tau / t), and an element whose key reaches it has x >= tau up to the rounding
+// of the two quotients: x >= tau_lo, a few ulps below tau.  Elements not below tau_lo (NaNs included:
+// their key is the largest) are ranked by their exact keys.  Groups without elements or with a NaN count as
+// -inf, which only lowers tau; a pool that overflows is reported to k_topk_sample.
+constexpr int kSegThreads = 512, kSegUnits = 8, kSegMax = kSegThreads * kSegUnits * 4, kSegPool = 512;
+constexpr uint32_t kSegOverflow = 0xffffffffu;
+__global__ __launch_bounds__(kSegThreads, 8) void k_topk_segments(TopKArgs p) {
+  __shared__ __attribute__((aligned(16))) float s_max[64];
+  __shared__ __attribute__((aligned(16))) f32x4 s_quad[kSegPool];
+  __shared__ int s_at[kSegPool];                 // row index of the quad's first element, top bits: elements to skip
+  __shared__ __attribute__((aligned(16))) uint64_t pool[kSegPool];
+  __shared__ uint32_t s_quads, s_pool;
+  __shared__ float s_tau;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int r = blockIdx.x / p.segs, seg = blockIdx.x - r * p.segs;
+  const int i0 = min(seg * p.seg_len, p.V), len = min(p.seg_len, p.V - i0);      // len >= 4
+  const float* base = p.logits + (int64_t)r * p.ld + i0;
+  const __amdgpu_buffer_rsrc_t rs = make_rsrc(base, (int64_t)len * 4);
+  // Quad u of the thread starts at element 4 (512 u + tid) of the segment.  Past the end the loads return
+  // zeros; a quad across the end (V % 4 elements of the last segment) is read from len - 4 on instead and
+  // its leading elements, which belong to the quad in front, are skipped.
+  f32x4 x[kSegUnits];
+#pragma unroll
+  for (int u = 0; u < kSegUnits; ++u) x[u] = load_b128(rs, (uint32_t)min((u * kSegThreads + tid) * 4, len - 4) * 4, 0);
+  float m[kSegUnits], mx = -__builtin_inff();
+#pragma unroll
+  for (int u = 0; u < kSegUnits; ++u) {
+    m[u] = nan_max(nan_max(x[u][0], x[u][1]), nan_max(x[u][2], x[u][3]));
+    if ((u * kSegThreads + tid) * 4 + 4 > len) m[u] = -__builtin_inff();    // past or across the end: not a witness for tau
+    mx = nan_max(mx, m[u]);
+  }
+#pragma unroll
+  for (int o = 1; o < 8; o <<= 1) mx = nan_max(mx, __shfl_xor(mx, o));
+  if ((tid & 7) == 0) s_max[tid >> 3] = mx == mx ? mx : -__builtin_inff();
+  if (tid == 0) { s_quads = 0; s_pool = 0; }
+  __syncthreads();
+  if (tid < 64) {
+    const float mine = s_max[lane];
+    int above = 0;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      const f32x4 o = *(const f32x4*)(s_max + 4 * q);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) above += o[j] > mine ? 1 : 0;
+    }
+    float tau = above < p.k ? mine : __builtin_inff();      // the k largest are among these
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) tau = fminf(tau, __shfl_xor(tau, o));
+    if (lane == 0) s_tau = tau;
+  }
+  __syncthreads();
+  const float tau = s_tau;
+  const float tau_lo = tau - fmaxf(fabsf(tau) * 0x1p-20f, 0x1p-100f);
+  // Quads with an element that is not below tau_lo; places by ballots and one LDS atomic per wavefront.
+  uint64_t hit[kSegUnits];
+  int count = 0;
+#pragma unroll
+  for (int u = 0; u < kSegUnits; ++u) {
+    const int e = (u * kSegThreads + tid) * 4;
+    hit[u] = __ballot(e < len && (!(m[u] < tau_lo) || e + 4 > len));
+    count += __popcll(hit[u]);
+  }
+  uint32_t first = 0;
+  if (lane == 0 && count > 0) first = atomicAdd(&s_quads, (uint32_t)count);
+  uint32_t at = __builtin_amdgcn_readfirstlane(first);
+#pragma unroll
+  for (int u = 0; u < kSegUnits; ++u) {
+    const uint32_t slot = at + __builtin_amdgcn_mbcnt_hi((uint32_t)(hit[u] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)hit[u], 0));
+    if (((hit[u] >> lane) & 1) && slot < (uint32_t)kSegPool) {
+      const int e = (u * kSegThreads + tid) * 4, s = min(e, len - 4);
+      s_quad[slot] = x[u];
+      s_at[slot] = s | ((e - s) << 28);
+    }
+    at += __popcll(hit[u]);
+  }
+  __syncthreads();
+  const uint32_t quads = s_quads;
+  // their elements, one per thread, with the exact key
+  for (uint32_t q = tid; q < min(quads, (uint32_t)kSegPool) * 4; q += kSegThreads) {
+    const float v = ((const float*)s_quad)[q];
+    const int s = s_at[q >> 2], j = (int)(q & 3);
+    const bool ok = !(v < tau_lo) && j >= (s >> 28);
+    const uint64_t b = __ballot(ok);
+    uint32_t f = 0;
+    if (ok) {
+      const int leader = __builtin_ctzll(b);
+      if (lane == leader) f = atomicAdd(&s_pool, (uint32_t)__popcll(b));
+      f = __shfl(f, leader) + __builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0));
+      if (f < (uint32_t)kSegPool) pool[f] = topk_word(v, p.t, i0 + (s & 0xfffffff) + j);
+    }
+  }
+  __syncthreads();
+  const uint32_t pooled = s_pool;
+  const bool over = quads > (uint32_t)kSegPool || pooled > (uint32_t)kSegPool;
+  if (tid == 0) p.counts[blockIdx.x] = over ? kSegOverflow : min(pooled, (uint32_t)p.k);
+  if (over) return;
+  const uint32_t padded = (pooled + 7u) & ~7u;
+  if ((uint32_t)tid >= pooled && (uint32_t)tid < padded) pool[tid] = 0ull;
+  __syncthreads();
+  if ((uint32_t)tid < pooled) {
+    const uint64_t mine = pool[tid];
+    int above = 0;
+    for (uint32_t q = 0; q < padded; q += 8) {
+      uint64_t other[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) other[j] = pool[q + j];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) above += other[j] > mine ? 1 : 0;
+    }
+    if (above < p.k) p.words[(int64_t)blockIdx.x * p.k + above] = mine;
+  }
+}
+
 constexpr int kTopKPool = 4096;
 
+// Draws for one row: orders the k largest (from the segments' lists when k_topk_segments ran, from the
+// row itself otherwise), adds the noise and takes the first maximum.
 __global__ __launch_bounds__(1024) void k_topk_sample(TopKArgs p) {
   __shared__ __attribute__((aligned(16))) uint32_t hist[4096];
   uint64_t* ranked_word = (uint64_t*)hist;      // the common path's pool; the histogram paths start by clearing hist
@@ -1405,10 +1615,12 @@ __global__ __launch_bounds__(1024) void k_topk_sample(TopKArgs p) {
   __shared__ uint32_t s_scan[1024];
   __shared__ uint32_t s_prefix, s_need, s_cnt, s_pool, s_wave[16], s_base;
   __shared__ float s_gmax[64];
+  __shared__ uint64_t s_tau_word;
   __shared__ float c_val[kTopKMax], o_val[kTopKMax];
   __shared__ int c_idx[kTopKMax], o_idx[kTopKMax];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const float* row = p.logits + (int64_t)blockIdx.x * p.ld;
+  const float noise = p.noise != nullptr && tid < p.k ? p.noise[(int64_t)blockIdx.x * p.k + tid] : 0.f;
 
   // Walks the row once, 16 bytes per lane where the row's address allows it, eight loads in flight
   // per lane (the row comes from L2 or beyond: latency, not bandwidth, is what one workgroup sees).
@@ -1445,23 +1657,62 @@ __global__ __launch_bounds__(1024) void k_topk_sample(TopKArgs p) {
   // A pool that overflows (rows of near-equal values) takes the histogram paths below instead.
   constexpr int kRankPool = 1024;
   if (tid == 0) s_pool = 0;
-  float mx = -__builtin_inff();
-  for_each([&](int, float x) { mx = fmaxf(mx, x); });
+  if (p.words != nullptr) {
+    // The segments' lists hold the top k.  A list's word number ceil(k / segs) - 1 is reached by that
+    // many words of the list, so at least k words reach the smallest of these over the lists: the words
+    // that do -- a few more than k -- are ranked below.  (An incomplete list counts as 0: all qualify.)
+    const uint64_t* words = p.words + (int64_t)blockIdx.x * p.segs * p.k;
+    const uint32_t* counts = p.counts + (int64_t)blockIdx.x * p.segs;
+    if (wave == 0) {
+      const uint32_t place = (uint32_t)((p.k + p.segs - 1) / p.segs);
+      uint64_t tau = ~0ull;
+      bool full = false;
+      for (int q = lane; q < p.segs; q += 64) {
+        const uint32_t c = counts[q];
+        full |= c == kSegOverflow;
+        const uint64_t w = c >= place && c != kSegOverflow ? words[(int64_t)q * p.k + place - 1] : 0ull;
+        tau = w < tau ? w : tau;
+      }
 #pragma unroll
-  for (int o = 1; o < 16; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-  if ((lane & 15) == 0) s_gmax[wave * 4 + (lane >> 4)] = mx;
-  __syncthreads();
-  float tau = s_gmax[lane];
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) tau = fminf(tau, __shfl_xor(tau, o));
-  const float tau_lo = tau - fmaxf(fabsf(tau) * 0x1p-20f, 0x1p-100f);
-  for_each([&](int i, float x) {
-    if (!(x < tau_lo)) {
-      const uint32_t slot = atomicAdd(&s_pool, 1u);
-      // one 64-bit word per element whose order is (key descending, index ascending); never 0
-      if (slot < (uint32_t)kRankPool) ranked_word[slot] = ((uint64_t)topk_key(x / p.t) << 32) | (uint32_t)~i;
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint64_t other = __shfl_xor((unsigned long long)tau, o);
+        tau = other < tau ? other : tau;
+      }
+      if (__any(full) && lane == 0) s_pool = kRankPool + 1;      // the histogram paths take the row
+      if (lane == 0) s_tau_word = tau;
     }
-  });
+    const int total = p.segs * p.k;
+    auto word = [&](int q) -> uint64_t {         // 0: no such word
+      const int seg = q / p.k;
+      return q < total && (uint32_t)(q - seg * p.k) < min(counts[seg], (uint32_t)p.k) ? words[q] : 0ull;
+    };
+    const uint64_t first = word(tid);            // requested before the barrier; usually all there is
+    __syncthreads();
+    const uint64_t tau = s_tau_word;
+    for (int q = tid; q < total; q += 1024) {
+      const uint64_t w = q == tid ? first : word(q);
+      if (w == 0ull || w < tau) continue;
+      const uint32_t slot = atomicAdd(&s_pool, 1u);
+      if (slot < (uint32_t)kRankPool) ranked_word[slot] = w;
+    }
+  } else {
+    float mx = -__builtin_inff();
+    for_each([&](int, float x) { mx = fmaxf(mx, x); });
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    if ((lane & 15) == 0) s_gmax[wave * 4 + (lane >> 4)] = mx;
+    __syncthreads();
+    float tau = s_gmax[lane];
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) tau = fminf(tau, __shfl_xor(tau, o));
+    const float tau_lo = tau - fmaxf(fabsf(tau) * 0x1p-20f, 0x1p-100f);
+    for_each([&](int i, float x) {
+      if (!(x < tau_lo)) {
+        const uint32_t slot = atomicAdd(&s_pool, 1u);
+        if (slot < (uint32_t)kRankPool) ranked_word[slot] = topk_word(x, p.t, i);
+      }
+    });
+  }
   __syncthreads();
   const uint32_t ranked = s_pool;
   __syncthreads();                       // every thread has read s_pool before the paths below reset it
@@ -1672,22 +1923,24 @@ __global__ __launch_bounds__(1024) void k_topk_sample(TopKArgs p) {
   if (tid < p.k) {
     if (p.top_idx != nullptr) p.top_idx[(int64_t)blockIdx.x * p.k + tid] = o_idx[tid];
     if (p.top_val != nullptr) p.top_val[(int64_t)blockIdx.x * p.k + tid] = o_val[tid];
-    // the k noise values in one go (c_val is free again): the scan below then stays inside the LDS
-    if (p.noise != nullptr) c_val[tid] = o_val[tid] + p.noise[(int64_t)blockIdx.x * p.k + tid];
+    if (p.noise != nullptr) c_val[tid] = o_val[tid] + noise;
   }
   __syncthreads();
-  if (tid == 0) {
+  if (wave == 0) {
+    // the first maximum wins, like argmax; a NaN in front stays, one behind it is never chosen
     int best = 0;
     if (p.noise != nullptr) {
-      float sc[kTopKMax];
+      float v = lane < p.k ? c_val[lane] : -__builtin_inff();
+      if (v != v) v = lane == 0 ? __builtin_inff() : -__builtin_inff();
+      best = lane;
 #pragma unroll
-      for (int j = 0; j < kTopKMax; ++j) sc[j] = c_val[j];
-      float bs = sc[0];
-#pragma unroll
-      for (int j = 1; j < kTopKMax; ++j)
-        if (j < p.k && sc[j] > bs) { bs = sc[j]; best = j; }      // first maximum wins, like argmax
+      for (int o = 1; o < 64; o <<= 1) {
+        const float ov = __shfl_xor(v, o);
+        const int oi = __shfl_xor(best, o);
+        if (ov > v || (ov == v && oi < best)) { v = ov; best = oi; }
+      }
     }
-    p.token[blockIdx.x] = o_idx[best];
+    if (lane == 0) p.token[blockIdx.x] = o_idx[best];
   }
 }
 

@@ -9,6 +9,7 @@ threefry stream.  No CPU fallback exists.
 """
 from __future__ import annotations
 
+import ctypes as C
 from typing import Optional, Union
 
 import torch
@@ -72,11 +73,15 @@ def top_k_sampling_batched(rng: Union[torch.Generator, torch.Tensor, None], logi
     token = torch.empty(b, dtype=torch.int32, device=lg.device)
     idx = torch.empty((b, k), dtype=torch.int32, device=lg.device) if return_top_k else None
     val = torch.empty((b, k), dtype=torch.float32, device=lg.device) if return_top_k else None
+    lib = _lib.load()
+    need = C.c_size_t()
+    _lib.check(lib.mj_sample_draw_workspace_bytes(b, v, int(k), C.byref(need)))
+    ws = torch.empty(need.value, dtype=torch.uint8, device=lg.device)
     with torch.cuda.device(lg.device):
-        _lib.check(_lib.load().mj_sample_top_k(
+        _lib.check(lib.mj_sample_draw(
             lg.data_ptr(), lg.stride(0), b, v, int(k), float(t), None if noise is None else noise.data_ptr(),
             token.data_ptr(), None if idx is None else idx.data_ptr(), None if val is None else val.data_ptr(),
-            torch.cuda.current_stream(lg.device).cuda_stream))
+            ws.data_ptr(), ws.numel(), torch.cuda.current_stream(lg.device).cuda_stream))
     return (token, idx, val) if return_top_k else token
 
 

@@ -148,3 +148,47 @@ def test_near_equal_logits_overflow_the_pool_and_take_the_slow_path():
     np.testing.assert_array_equal(idx.cpu().numpy(), ri)
     np.testing.assert_array_equal(val.cpu().numpy(), rv)
     np.testing.assert_array_equal(tok.cpu().numpy(), rt)
+
+
+@pytest.mark.parametrize("v,ld", [(4096, 4096), (16381, 16384), (16384, 16387), (16385, 16392), (32769, 32769), (49153, 49160)])
+def test_rows_cut_into_segments_draw_like_whole_rows(v, ld):
+    """Vocabularies either side of a segment's 16384 elements, rows that are not 16-byte aligned, the
+    largest values at the segments' ends, NaNs, ties across segments and a row whose ties overflow a
+    segment's pool: bit for bit the oracle's choice."""
+    import mllm_jax_amd as M
+    dev = torch.device("cuda:0")
+    rng = np.random.default_rng(v)
+    k = 64
+    x = rng.normal(0, 1, size=(6, ld)).astype(np.float32)
+    x[1, [0, v - 1, v // 2, min(16383, v - 1)]] = 9.0
+    x[2, v - 3:v] = np.float32(7.0)
+    x[2, v:] = 99.0                                                  # padding of the row: never looked at
+    x[3, rng.integers(0, v, 70)] = np.nan
+    x[4, ::97] = 5.0                                                 # more than k equal maxima, spread over the segments
+    x[5] = 1.0
+    noise = rng.gumbel(size=(6, k)).astype(np.float32)
+    lg = torch.tensor(x, device=dev)[:, :v]
+    tok, idx, val = M.top_k_sampling_batched(torch.tensor(noise), lg, k=k, t=0.9, return_top_k=True)
+    rt, ri, rv = O.top_k_sample(x[:, :v], k=k, t=0.9, noise=noise)
+    np.testing.assert_array_equal(idx.cpu().numpy(), ri)
+    np.testing.assert_array_equal(val.cpu().numpy().view(np.uint32), rv.view(np.uint32))
+    rows = [0, 1, 2, 4, 5]                                           # what argmax makes of NaN scores is not at issue here
+    np.testing.assert_array_equal(tok.cpu().numpy()[rows], rt[rows])
+
+
+@pytest.mark.parametrize("b,h,v,cap", [(1, 8, 8, None), (1, 24, 264, 30.0), (2, 56, 1000, None), (2, 72, 256, 10.0), (1, 136, 2008, None),
+                                       (2, 904, 5000, None)])
+def test_one_or_two_rows_on_the_vector_alus(b, h, v, cap):
+    """k_logits_few: odd counts of 8-row groups, columns either side of a workgroup's 256, softcap; a row
+    pitch of W and of hidden past their lengths.  The bound is float32 summation: h products of at most
+    0.2 * 4 * 4 in magnitude, one rounding of 2^-24 of the partial sum each."""
+    import mllm_jax_amd as M
+    dev = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(h + v)
+    hid = torch.randn(b, h + 8, generator=g).to(torch.bfloat16)
+    w = (0.2 * torch.randn(h, v + 16, generator=g)).to(torch.bfloat16)
+    w[:, v:] = float("nan")                                          # padding: never looked at
+    hid[:, h:] = float("nan")
+    out = M.last_position_logits(hid.to(dev)[:, :h], w.to(dev)[:, :v], cap)
+    ref = O.lm_head_logits(hid[:, :h].float().numpy(), w[:, :v].float().numpy(), cap)
+    np.testing.assert_allclose(out.cpu().numpy(), ref, rtol=1e-5, atol=h * 3.2 * 2.0 ** -24 * 4)
