@@ -534,15 +534,18 @@ int mj_grpo_advantages(int mode, const float* rewards, const int32_t* group_ids,
   if (!rewards || !advantages || (mode != mj::kAdvGlobal && !group_ids))
     return fail(MJ_GRPO_ERR_NULL, "rewards/group_ids/advantages is NULL");
   if (b <= 0 || b > (1 << 16)) return fail(MJ_GRPO_ERR_SHAPE, "batch must be in [1, 65536] (got %lld)", (long long)b);
-  // the grouped estimators walk the batch once per sample (a batch is hundreds of sequences)
+  // the grouped estimators walk the batch once or twice per sample (a batch is hundreds of sequences)
   if (mode != mj::kAdvGlobal && b > (1 << 13))
     return fail(MJ_GRPO_ERR_SHAPE, "grouped advantage estimators take at most 8192 sequences (got %lld)", (long long)b);
   if (!(eps > 0.f)) return fail(MJ_GRPO_ERR_UNSUPPORTED, "eps must be > 0");
   if (mode == mj::kAdvDapo && !(alpha >= 0.f)) return fail(MJ_GRPO_ERR_UNSUPPORTED, "alpha must be >= 0");
   mj::AdvArgs a;
-  a.rewards = rewards; a.group_ids = group_ids; a.adv = advantages; a.b = (int)b; a.mode = mode; a.whiten = whiten;
-  a.eps = eps; a.alpha = alpha; a.clip = clip_range;
-  mj::k_advantages<<<1, 1024, 0, (hipStream_t)stream>>>(a);
+  const bool whitened = mode == mj::kAdvRloo && whiten != 0;
+  a.rewards = rewards; a.group_ids = group_ids; a.adv = advantages; a.b = (int)b; a.mode = mode;
+  a.eps = eps; a.alpha = alpha; a.clip = whitened ? 0.f : clip_range;
+  const int per = mode == mj::kAdvGlobal ? mj::kAdvThreads : mj::kAdvThreads / mj::kAdvLanes;   // samples per workgroup
+  mj::k_advantages<<<(unsigned)((b + per - 1) / per), mj::kAdvThreads, 0, (hipStream_t)stream>>>(a);
+  if (whitened) mj::k_whiten<<<1, 1024, 0, (hipStream_t)stream>>>(advantages, (int)b, eps, clip_range);
   return check_launch("k_advantages");
 }
 
@@ -561,7 +564,7 @@ int mj_grpo_gae(const float* rewards, const float* values, const float* completi
   a.rewards = rewards; a.values = values; a.mask = completion_mask; a.adv = advantages; a.ret = returns;
   a.b = (int)b; a.t = (int)t; a.gamma = gamma; a.lambda = gae_lambda;
   hipStream_t st = (hipStream_t)stream;
-  mj::k_gae_scan<<<(unsigned)((b + 255) / 256), 256, 0, st>>>(a);
+  mj::k_gae_scan<<<(unsigned)((b + 3) / 4), 256, 0, st>>>(a);
   if (normalize || clip_range > 0.f)
     mj::k_gae_normalize<<<1, 1024, 0, st>>>(advantages, completion_mask, b * t, normalize, eps, clip_range);
   return check_launch("gae kernels");

@@ -95,3 +95,40 @@ def test_argument_errors_mirror_the_reference():
         M.compute_gae_advantages(rewards=_d(R5), values=_d(np.zeros((5, 3), np.float32)), completion_mask=_d(np.zeros((5, 4), np.float32)))
     with pytest.raises(RuntimeError):
         M.compute_global_normalized_advantages(rewards=torch.tensor(R5))
+
+
+@pytest.mark.parametrize("t", [3, 4, 255, 256, 257, 513, 1024])
+@pytest.mark.parametrize("gamma,lam", [(1.0, 0.95), (1.0, 1.0), (0.9, 0.0)])
+def test_gae_blocks_of_256_tokens(t, gamma, lam):
+    """Sequence lengths either side of a lane's four tokens and of a 256-token block; completions that end
+    in the last block, in an earlier one, in the middle of a lane's tokens, or nowhere."""
+    import mllm_jax_amd as M
+    rng = np.random.default_rng(t)
+    b = 7
+    r = rng.standard_normal(b).astype(np.float32)
+    v = rng.standard_normal((b, t)).astype(np.float32)
+    end = np.array([t, t - 1, max(t // 2, 1), 1, 0, max(t - 255, 1), max(t - 257, 1)])
+    m = ((np.arange(t)[None] >= end[:, None] // 3) & (np.arange(t)[None] < end[:, None])).astype(np.float32)
+    adv, ret = M.compute_gae_advantages(rewards=_d(r), values=_d(v), completion_mask=_d(m), gamma=gamma, gae_lambda=lam,
+                                        normalize=False)
+    ra, rr = O.gae_advantages(r, v, m, gamma, lam, False, 1e-4, None)
+    # both walk up to t float32 steps; each adds a rounding of 2^-24 of a running value of a few sigma
+    tol = dict(rtol=1e-5, atol=max(1e-5, t * 2.0 ** -24 * 8))
+    np.testing.assert_allclose(ret.cpu().numpy(), rr, **tol)
+    np.testing.assert_allclose(adv.cpu().numpy(), ra, **tol)
+
+
+@pytest.mark.parametrize("b", [15, 16, 17, 255, 257, 1039])
+def test_batches_across_workgroups(b):
+    """Batch sizes either side of a workgroup's samples; one group, singletons, and ragged groups."""
+    import mllm_jax_amd as M
+    rng = np.random.default_rng(b)
+    r = rng.standard_normal(b).astype(np.float32)
+    for gid in (np.zeros(b, np.int32), np.arange(b, dtype=np.int32), rng.integers(0, max(b // 7, 1), b).astype(np.int32)):
+        kw = dict(rtol=1e-5, atol=1e-5)
+        np.testing.assert_allclose(M.compute_grpo_advantages_by_group_id(rewards=_d(r), group_ids=_d(gid)).cpu().numpy(),
+                                   O.grpo_advantages(r, gid), **kw)
+        np.testing.assert_allclose(M.compute_rloo_advantages_by_group_id(rewards=_d(r), group_ids=_d(gid), whiten=b > 16, clip_range=1.0).cpu().numpy(),
+                                   O.rloo_advantages(r, gid, whiten=b > 16, clip_range=1.0), **kw)
+        np.testing.assert_allclose(M.compute_dapo_advantages_by_group_id(rewards=_d(r), group_ids=_d(gid), clip_range=0.9).cpu().numpy(),
+                                   O.dapo_advantages(r, gid, clip_range=0.9), **kw)
