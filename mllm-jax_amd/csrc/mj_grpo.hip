@@ -668,6 +668,7 @@ int mj_sample_top_k(const float* logits, int64_t ld_logits, int64_t b, int64_t v
 // ----------------------------------------------------------------------------- RMSNorm
 namespace {
 constexpr int kNormMaxH = 8192;
+bool norm_streams(int64_t n, int64_t h) { return n * h * 2 > (32ll << 20); }   // see mj_norm_kernels.hpp
 int norm_grid(int64_t n) {   // workgroups of the backward (one row at a time each, rows with this stride): four per CU
   return (int)(n < 1024 ? n : 1024);
 }
@@ -696,8 +697,9 @@ int mj_rmsnorm_forward(const void* x, int64_t ld_x, const float* scale, void* y,
   a.x = (const uint16_t*)x; a.scale = scale; a.y = (uint16_t*)y; a.rstd = rstd;
   a.ld_x = ld_x; a.ld_y = ld_y; a.n = (int)n; a.H = (int)h; a.eps = eps;
   const unsigned grid = (unsigned)((n + 3) / 4);
-  if (h <= 4096) mj::k_rmsnorm_fwd<8><<<grid, 256, 0, (hipStream_t)stream>>>(a);
-  else mj::k_rmsnorm_fwd<16><<<grid, 256, 0, (hipStream_t)stream>>>(a);
+  auto kernel = norm_streams(n, h) ? (h <= 4096 ? mj::k_rmsnorm_fwd<8, true> : mj::k_rmsnorm_fwd<16, true>)
+                                   : (h <= 4096 ? mj::k_rmsnorm_fwd<8, false> : mj::k_rmsnorm_fwd<16, false>);
+  kernel<<<grid, 256, 0, (hipStream_t)stream>>>(a);
   return check_launch("k_rmsnorm_fwd");
 }
 
@@ -722,9 +724,10 @@ int mj_rmsnorm_backward(const void* dy, int64_t ld_dy, const void* x, int64_t ld
   a.dy = (const uint16_t*)dy; a.x = (const uint16_t*)x; a.scale = scale; a.dx = (uint16_t*)dx;
   a.part = (float*)workspace; a.ld_dy = ld_dy; a.ld_x = ld_x; a.ld_dx = ld_dx; a.n = (int)n; a.H = (int)h; a.eps = eps;
   hipStream_t st = (hipStream_t)stream;
-  if (h <= 2048) mj::k_rmsnorm_bwd<1><<<grid, 256, 0, st>>>(a);
-  else if (h <= 4096) mj::k_rmsnorm_bwd<2><<<grid, 256, 0, st>>>(a);
-  else mj::k_rmsnorm_bwd<4><<<grid, 256, 0, st>>>(a);
+  auto kernel = norm_streams(n, h)
+                    ? (h <= 2048 ? mj::k_rmsnorm_bwd<1, true> : h <= 4096 ? mj::k_rmsnorm_bwd<2, true> : mj::k_rmsnorm_bwd<4, true>)
+                    : (h <= 2048 ? mj::k_rmsnorm_bwd<1, false> : h <= 4096 ? mj::k_rmsnorm_bwd<2, false> : mj::k_rmsnorm_bwd<4, false>);
+  kernel<<<grid, 256, 0, st>>>(a);
   if ((rc = check_launch("k_rmsnorm_bwd"))) return rc;
   mj::k_rmsnorm_dscale<<<(unsigned)((h + 63) / 64), 256, 0, st>>>((const float*)workspace, grid, (int)h, dscale,
                                                                   accumulate_dscale);

@@ -93,3 +93,30 @@ def test_norm_feeds_the_fused_loss_end_to_end():
     assert _rel(xd.grad.float().cpu().numpy(), dxr) <= 3e-2      # two bf16 roundings in the chain
     assert _rel(sd.grad.cpu().numpy(), dsr) <= 2e-2
     assert _rel(wd.grad.float().cpu().numpy(), ref["d_lm_head"]) <= 2e-2
+
+
+@pytest.mark.parametrize("n,h", [(8193, 2048), (4099, 4096), (2051, 8192), (4667, 3600)])
+def test_matrices_larger_than_the_l2s_stream(n, h):
+    """Just past 32 MB the accesses carry the non-temporal hint: rows are those of a small call bit for
+    bit (a row's arithmetic does not depend on the matrix), dscale is the float64 column sum."""
+    import mllm_jax_amd as M
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(h)
+    x = torch.randn(n, h, generator=g, device=dev).to(torch.bfloat16)
+    dy = torch.randn(n, h, generator=g, device=dev).to(torch.bfloat16)
+    s = 1.0 + 0.2 * torch.randn(h, generator=g, device=dev)
+    assert n * h * 2 > 32 << 20
+
+    def run(x, dy):
+        x, sc = x.clone().requires_grad_(), s.clone().requires_grad_()
+        y = M.rms_norm(x, sc)
+        return (y.detach(), *torch.autograd.grad(y, [x, sc], dy))
+
+    y, dx, ds = run(x, dy)
+    for rows in (slice(0, 70), slice(n // 2, n // 2 + 70), slice(n - 70, n)):
+        ys, dxs, _ = run(x[rows], dy[rows])
+        assert torch.equal(y[rows], ys) and torch.equal(dx[rows], dxs)
+    xd = x.double()
+    ref = (dy.double() * xd * torch.rsqrt((xd * xd).mean(-1, keepdim=True) + 1e-6)).sum(0)
+    # n float32 products and additions per column, in 1024 partial sums of a few rows: about sqrt(n) 2^-24 of the terms' norm
+    assert float((ds.double() - ref).norm() / ref.norm()) < 1e-5
