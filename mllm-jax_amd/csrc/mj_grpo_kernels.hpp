@@ -137,14 +137,9 @@ MJ_DEV uint32_t pack_f16(float a, float b) {   // clamped to the finite half ran
 // The lanes l and l + 32 hold rows 4..7 of the same groups for the same token; after exchanging
 // one half with the partner each lane owns eight CONSECUTIVE vocab entries and stores them with
 // one 16-byte access (`voff` carries the lane's 16 bytes of the 32).
-template <bool HALF>
 MJ_DEV void store_rows8(const float (&v)[8], __amdgpu_buffer_rsrc_t rs, uint32_t voff, uint32_t soff) {
-  uint32_t a0, a1, b0, b1;
-  if (HALF) {
-    a0 = pack_f16(v[0], v[1]); a1 = pack_f16(v[2], v[3]); b0 = pack_f16(v[4], v[5]); b1 = pack_f16(v[6], v[7]);
-  } else {
-    a0 = pack_bf16(v[0], v[1]); a1 = pack_bf16(v[2], v[3]); b0 = pack_bf16(v[4], v[5]); b1 = pack_bf16(v[6], v[7]);
-  }
+  const uint32_t a0 = pack_bf16(v[0], v[1]), a1 = pack_bf16(v[2], v[3]);
+  const uint32_t b0 = pack_bf16(v[4], v[5]), b1 = pack_bf16(v[6], v[7]);
   // v_permlane32_swap: the first operand of lanes 32..63 <-> the second operand of lanes 0..31
   const auto s0 = __builtin_amdgcn_permlane32_swap(a0, b0, false, false);
   const auto s1 = __builtin_amdgcn_permlane32_swap(a1, b1, false, false);
@@ -152,10 +147,10 @@ MJ_DEV void store_rows8(const float (&v)[8], __amdgpu_buffer_rsrc_t rs, uint32_t
   __builtin_amdgcn_raw_buffer_store_b128(out, rs, voff, soff, 0);
 }
 
-// One 256 x 256 tile: logits^T [vocab x tokens] = W^T * hidden^T on MFMA, then the epilogue of MODE
-// (kStatsMax, kStatsGrad; kStatsExp has a tile of its own, logits_tile16).
-template <int BM, int BN, int MODE, bool CAP>
-MJ_DEV void logits_tile(const LogitsArgs& p, int tm, int tn, char* smem, int tid) {
+// One 256 x 256 tile: logits^T [vocab x tokens] = W^T * hidden^T on MFMA, then the epilogue of kStatsGrad
+// (the other two modes have a tile of their own, logits_tile16).
+template <int BM, int BN, bool CAP>
+MJ_DEV void logits_tile_grad(const LogitsArgs& p, int tm, int tn, char* smem, int tid) {
   using G = GemmTN<BM, BN, kKRow, kRowK>;
   const int m0 = tm * BM, n0 = tn * BN;
   G g;
@@ -182,7 +177,6 @@ MJ_DEV void logits_tile(const LogitsArgs& p, int tm, int tn, char* smem, int tid
     // Softcap (CAP: a kernel of its own, so that the uncapped one carries none of this).  While every
     // logit of the block is small against the cap -- checked per wavefront -- tanh is its odd series
     // to u^7 (|u| <= 0.25: error below 1e-7 of u, five multiply-adds instead of an exp and a reciprocal).
-    static_assert(MODE != kStatsExp, "kStatsExp runs on logits_tile16");
     if (CAP) {
       float big = 0.f;
 #pragma unroll
@@ -231,72 +225,15 @@ MJ_DEV void logits_tile(const LogitsArgs& p, int tm, int tn, char* smem, int tid
     // where this lane's eight-entry groups go: token row, then the lane's half of a 16-entry span
     const bool store = p.zt != nullptr && (t0 + ni * 32) < zt_cols;   // tokens past the live ones are never read
     const uint32_t voff = (uint32_t)((ni * 32 + l31) * ldz2 + (vwave + lhi * 8) * 2);
-    // Rows of tokens that cannot carry a gradient (mask 0; in kStatsGrad: dloss/dlogp 0) are not
-    // written at all: the backward products know them from the dead-token bits and do not read them.
+    // Rows of tokens that cannot carry a gradient (dloss/dlogp 0) are not written at all: the backward
+    // products know them from the dead-token bits and do not read them.
     bool keep = true;
-    if (store) keep = MODE == kStatsGrad ? (col < p.n && p.g[col] != 0.f) : (col < p.n && p.mask[col] != 0.f);
+    if (store) keep = col < p.n && p.g[col] != 0.f;
     auto group_off = [&](int mi, int qp) {      // kOob when the lane's eight entries lie past V (V % 8 == 0)
       return (keep && (vwave + mi * 32 + qp * 16 + lhi * 8) < p.V) ? voff : kOob;
     };
 
-    if (MODE == kStatsMax) {
-      float mx = kNegBig;
-#pragma unroll
-      for (int mi = 0; mi < G::MI; ++mi)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, g.acc[mi][ni][r]);
-      mx = fmaxf(mx, __shfl_xor(mx, 32));
-      float l = 0.f, s = 0.f;
-      const float mxl = mx * kLog2e;
-#pragma unroll
-      for (int mi = 0; mi < G::MI; ++mi)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float z = g.acc[mi][ni][r];
-          const float e = __builtin_amdgcn_exp2f(fmaf(z, kLog2e, -mxl));
-          l += e;
-          s = fmaf(e, z, s);
-        }
-      l += __shfl_xor(l, 32);
-      s += __shfl_xor(s, 32);
-      float lt = 0.f;
-      if (p.inv_t != 1.f) {
-        // The reference takes the log-prob from softmax(z) but the entropy from softmax(z / T)
-        // (train_modules/__init__.py:124-126, :136): a second pair of sums, only when T != 1.
-        asm volatile("");
-        const float kt = kLog2e * p.inv_t, mxt = mx * kt;
-        s = 0.f;
-#pragma unroll
-        for (int mi = 0; mi < G::MI; ++mi)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const float z = g.acc[mi][ni][r];
-            const float e = __builtin_amdgcn_exp2f(fmaf(z, kt, -mxt));
-            lt += e;
-            s = fmaf(e, z, s);
-          }
-        lt += __shfl_xor(lt, 32);
-        s += __shfl_xor(s, 32);
-      }
-      if (lhi == 0) {
-        const int64_t o = (int64_t)(tm * 2 + wm) * p.ld_p + col;
-        p.pm[o] = mx;
-        p.pl[o] = l;
-        p.ps[o] = s;
-        if (p.inv_t != 1.f) p.plt[o] = lt;
-      }
-      if (store) {
-#pragma unroll
-        for (int mi = 0; mi < G::MI; ++mi)
-#pragma unroll
-          for (int qp = 0; qp < 2; ++qp) {
-            float v[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = g.acc[mi][ni][qp * 8 + j];
-            store_rows8<true>(v, zrs, group_off(mi, qp), (uint32_t)(mi * 32 + qp * 16) * 2);
-          }
-      }
-    } else {   // kStatsGrad
+    {
       const float lse2 = col < p.n ? p.lse[col] * kLog2e : 0.f;
       const float gneg = col < p.n ? -p.g[col] : 0.f;
       if (store) {
@@ -311,7 +248,7 @@ MJ_DEV void logits_tile(const LogitsArgs& p, int tm, int tn, char* smem, int tid
               const float d = gneg * __builtin_amdgcn_exp2f(fmaf(z, kLog2e, -lse2));
               v[j] = CAP ? d * (1.f - z * z * inv_cap2) : d;
             }
-            store_rows8<false>(v, zrs, group_off(mi, qp), (uint32_t)(mi * 32 + qp * 16) * 2);
+            store_rows8(v, zrs, group_off(mi, qp), (uint32_t)(mi * 32 + qp * 16) * 2);
           }
       }
     }
@@ -344,7 +281,15 @@ MJ_DEV float sum_rows16(float x) {
   return __uint_as_float(q[0]) + __uint_as_float(q[1]);
 }
 
-// The kStatsExp tile on the chained 16 x 16 x 32 engine (GemmTN16).  A lane holds, for the token
+MJ_DEV float max_rows16(float x) {
+  const uint32_t a = __float_as_uint(x);
+  const auto p = __builtin_amdgcn_permlane16_swap(a, a, false, false);
+  const uint32_t b = __float_as_uint(fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1])));
+  const auto q = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  return fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
+}
+
+// The kStatsExp and kStatsMax tile on the chained 16 x 16 x 32 engine (GemmTN16).  A lane holds, for the token
 // ni*16 + lane%16, the four vocab rows mi*16 + (lane/16)*4 + 0..3 of each of the eight blocks mi.
 // Two blocks at a time, the lanes l and l + 16 exchange one packed half (v_permlane16_swap) so that
 // each owns eight CONSECUTIVE vocab entries of one block and stores them with one 16-byte access.
@@ -353,10 +298,14 @@ MJ_DEV float sum_rows16(float x) {
 // the two stages: requested in the epilogue they cost a memory round trip per tile (2.6 us of a
 // tile's 95 at 16384 x 3584 x 152064).
 constexpr int kTileExtraLds = 2048;
-template <int BM, int BN, bool CAP>
+template <int BM, int BN, int MODE, bool CAP>
 MJ_DEV void logits_tile16(const LogitsArgs& p, int tm, int tn, char* smem, int tid) {
   using G = GemmTN16<BM, BN, kKRow, kRowK>;
   static_assert(BN == kThreads, "one token of the tile per thread");
+  static_assert(MODE != kStatsGrad, "kStatsGrad runs on logits_tile_grad");
+  // CAP: the epilogue's logits are in units of log2 in kStatsExp, in natural units in kStatsMax
+  constexpr float kUnit = MODE == kStatsExp ? kLog2e : 1.f;
+  constexpr float kToLog2 = CAP && MODE == kStatsExp ? 1.f : kLog2e;
   const int m0 = tm * BM, n0 = tn * BN;
   const int tok = n0 + tid;
   const float mask_t = tok < p.n ? p.mask[tok] : 0.f;
@@ -402,20 +351,20 @@ MJ_DEV void logits_tile16(const LogitsArgs& p, int tm, int tn, char* smem, int t
 #pragma unroll
         for (int r = 0; r < 4; ++r) big = fmaxf(big, fabsf(g.acc[mi][ni][r]));
       if (__all(big * inv_cap <= 0.25f)) {
-        const float c1 = kLog2e * (-1.f / 3.f) * inv_cap2, c2 = kLog2e * (2.f / 15.f) * inv_cap2 * inv_cap2;
-        const float c3 = kLog2e * (-17.f / 315.f) * inv_cap2 * inv_cap2 * inv_cap2;
+        const float c1 = kUnit * (-1.f / 3.f) * inv_cap2, c2 = kUnit * (2.f / 15.f) * inv_cap2 * inv_cap2;
+        const float c3 = kUnit * (-17.f / 315.f) * inv_cap2 * inv_cap2 * inv_cap2;
 #pragma unroll
         for (int mi = 0; mi < G::MI; ++mi)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const float z = g.acc[mi][ni][r], w = z * z;
-            g.acc[mi][ni][r] = z * fmaf(w, fmaf(w, fmaf(w, c3, c2), c1), kLog2e);
+            g.acc[mi][ni][r] = z * fmaf(w, fmaf(w, fmaf(w, c3, c2), c1), kUnit);
           }
       } else {
 #pragma unroll
         for (int mi = 0; mi < G::MI; ++mi)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) g.acc[mi][ni][r] = softcap_apply(g.acc[mi][ni][r], p.cap, inv_cap) * kLog2e;
+          for (int r = 0; r < 4; ++r) g.acc[mi][ni][r] = softcap_apply(g.acc[mi][ni][r], p.cap, inv_cap) * kUnit;
       }
     }
     // an opaque use of the column's 32 accumulators: the register allocator then moves them out of the
@@ -441,8 +390,35 @@ MJ_DEV void logits_tile16(const LogitsArgs& p, int tm, int tn, char* smem, int t
     auto group_off = [&](int mp) {      // kOob when the lane's eight entries lie past V (V % 8 == 0)
       return (keep && (vwave + (2 * mp + (lq & 1)) * 16 + (lq >> 1) * 8) < p.V) ? voff : kOob;
     };
-    float l = 0.f, s = 0.f;
-    if (store) {
+    float l = 0.f, s = 0.f, mx = kNegBig;    // mx: kStatsMax only
+    if constexpr (MODE == kStatsMax) {
+#pragma unroll
+      for (int mi = 0; mi < G::MI; ++mi)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) mx = fmaxf(mx, g.acc[mi][ni][r]);
+      mx = max_rows16(mx);
+      const float mxl = mx * kLog2e;
+#pragma unroll
+      for (int mi = 0; mi < G::MI; ++mi)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float z = g.acc[mi][ni][r];
+          const float e = __builtin_amdgcn_exp2f(fmaf(z, kLog2e, -mxl));
+          l += e;
+          s = fmaf(e, z, s);
+        }
+      if (lq == 0) p.pm[(int64_t)(tm * 2 + wm) * p.ld_p + col] = mx;
+      if (store) {
+#pragma unroll
+        for (int mp = 0; mp < G::MI / 2; ++mp) {
+          const f32x4 u = g.acc[2 * mp][ni], v = g.acc[2 * mp + 1][ni];
+          const auto s0 = __builtin_amdgcn_permlane16_swap(pack_f16(u[0], u[1]), pack_f16(v[0], v[1]), false, false);
+          const auto s1 = __builtin_amdgcn_permlane16_swap(pack_f16(u[2], u[3]), pack_f16(v[2], v[3]), false, false);
+          const u32x4 out = {s0[0], s1[0], s0[1], s1[1]};
+          __builtin_amdgcn_raw_buffer_store_b128(out, zrs, group_off(mp), (uint32_t)(mp * 32) * 2, 0);
+        }
+      }
+    } else if (store) {
 #pragma unroll
       for (int mp = 0; mp < G::MI / 2; ++mp) {
         float v[2][4];
@@ -480,14 +456,14 @@ MJ_DEV void logits_tile16(const LogitsArgs& p, int tm, int tn, char* smem, int t
       // the entropy is that of softmax(z / T) (train_modules/__init__.py:136): its own pair of sums,
       // behind a real scalar branch so that the usual T = 1 pays nothing for it
       asm volatile("");
-      const float kt = (CAP ? 1.f : kLog2e) * p.inv_t;
+      const float kt = kToLog2 * p.inv_t, mxt = mx * kt;
       s = 0.f;
 #pragma unroll
       for (int mi = 0; mi < G::MI; ++mi)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const float z = g.acc[mi][ni][r];
-          const float e = __builtin_amdgcn_exp2f(z * kt);
+          const float e = __builtin_amdgcn_exp2f(MODE == kStatsMax ? fmaf(z, kt, -mxt) : z * kt);
           lt += e;
           s = fmaf(e, z, s);
         }
@@ -495,7 +471,7 @@ MJ_DEV void logits_tile16(const LogitsArgs& p, int tm, int tn, char* smem, int t
     }
     l = sum_rows16(l);
     s = sum_rows16(s);
-    if (CAP) s *= kLn2;                      // sum e * cap(z) in natural units
+    if (CAP && MODE == kStatsExp) s *= kLn2;   // sum e * cap(z) in natural units
     if (lq == 0) {
       const int64_t o = (int64_t)(tm * 2 + wm) * p.ld_p + col;
       p.pl[o] = l;
@@ -514,7 +490,7 @@ MJ_DEV void logits_tile16(const LogitsArgs& p, int tm, int tn, char* smem, int t
         for (int mi = 0; mi < G::MI; ++mi)
 #pragma unroll
           for (int r = 0; r < 4; ++r) zy = (flat == mi * 4 + r) ? g.acc[mi][ni][r] : zy;
-        if (hit) p.zy[col] = CAP ? zy * kLn2 : zy;
+        if (hit) p.zy[col] = CAP && MODE == kStatsExp ? zy * kLn2 : zy;
       }
     }
   }
@@ -540,14 +516,14 @@ __global__ __launch_bounds__(kThreads) void k_logits_stats(LogitsArgs p, TileMap
     if (__builtin_amdgcn_readfirstlane(*p.state) == 0) return;
     const int items = map.items();
     for (int item = blockIdx.x; item < items; item += gridDim.x) {
-      if (map.tile(item, tm, tn, split)) logits_tile<BM, BN, MODE, CAP>(p, tm, tn, smem, opaque_tid());
+      if (map.tile(item, tm, tn, split)) logits_tile16<BM, BN, MODE, CAP>(p, tm, tn, smem, opaque_tid());
       __syncthreads();      // the next tile's first LDS writes must not pass this tile's last reads
     }
   } else {
     if (MODE == kStatsExp && blockIdx.x == 0 && threadIdx.x == 0) *p.state = 0;
     if (!map.tile(blockIdx.x, tm, tn, split)) return;
-    if constexpr (MODE == kStatsExp) logits_tile16<BM, BN, CAP>(p, tm, tn, smem, threadIdx.x);
-    else logits_tile<BM, BN, MODE, CAP>(p, tm, tn, smem, threadIdx.x);
+    if constexpr (MODE == kStatsGrad) logits_tile_grad<BM, BN, CAP>(p, tm, tn, smem, threadIdx.x);
+    else logits_tile16<BM, BN, MODE, CAP>(p, tm, tn, smem, threadIdx.x);
   }
 }
 

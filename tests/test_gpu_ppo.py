@@ -128,6 +128,19 @@ def test_softcap_with_entropy_bonus_across_chunks():
               chunk_tokens=256, old_noise=0.1)
 
 
+@pytest.mark.parametrize("b,l,h,v,cap", [
+    (1, 2, 8, 56, None),            # one token, one slice of K, a fifth of a tile of the vocabulary
+    (1, 257, 64, 128, None),        # exactly a tile of tokens; the second half of the vocabulary tile is empty
+    (1, 258, 72, 136, 30.0),        # one token and eight vocabulary rows over, K not a multiple of a slice
+    (2, 129, 200, 264, None),       # eight rows in a second vocabulary tile
+    (5, 70, 128, 520, 8.0),
+])
+def test_running_maximum_tile_at_its_edges(b, l, h, v, cap):
+    # the entropy bonus takes the logits with a running maximum; the tolerances are this file's: the sums are
+    # float32 whatever the tile, the gradient's 16-bit storage has 2^-9 relative steps
+    _run_case(31 + v, b, l, h, v, entropy_coef=0.1, old_noise=0.1, final_logit_softcap=cap)
+
+
 @pytest.mark.parametrize("splits", [1, 4])
 def test_value_head_gradient_joins_d_hidden_in_the_product(splits):
     """entropy_coef = 0: the E-based backward; dv * value_w is added in the d_hidden product's own
