@@ -1489,12 +1489,12 @@ __global__ __launch_bounds__(kSegThreads, 8) void k_topk_segments(TopKArgs p) {
   __shared__ float s_tau;
   const int tid = threadIdx.x, lane = tid & 63;
   const int r = blockIdx.x / p.segs, seg = blockIdx.x - r * p.segs;
-  const int i0 = min(seg * p.seg_len, p.V), len = min(p.seg_len, p.V - i0);      // len >= 4
+  const int i0 = min(seg * p.seg_len, p.V), len = min(p.seg_len, p.V - i0);      // len >= 64: the host's segments
   const float* base = p.logits + (int64_t)r * p.ld + i0;
   const __amdgpu_buffer_rsrc_t rs = make_rsrc(base, (int64_t)len * 4);
-  // Quad u of the thread starts at element 4 (512 u + tid) of the segment.  Past the end the loads return
-  // zeros; a quad across the end (V % 4 elements of the last segment) is read from len - 4 on instead and
-  // its leading elements, which belong to the quad in front, are skipped.
+  // Quad u of the thread starts at element 4 (512 u + tid) of the segment.  A quad across or past the end is
+  // read from len - 4 on instead; across the end (V % 4 elements of the last segment) its leading elements,
+  // which belong to the quad in front, are skipped, past the end all of them.
   f32x4 x[kSegUnits];
 #pragma unroll
   for (int u = 0; u < kSegUnits; ++u) x[u] = load_b128(rs, (uint32_t)min((u * kSegThreads + tid) * 4, len - 4) * 4, 0);

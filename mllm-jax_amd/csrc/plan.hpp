@@ -190,9 +190,12 @@ inline void sample_tiles(int64_t b, int64_t vocab, int* bn_out, int64_t* tiles_n
 
 // Segments of a row for the top-k draw: as few as hold the row at kDrawSegment elements each, of even
 // length.  segs == 0: the rows are drawn from without them -- short rows (below 4096 elements too few of a
-// segment's groups of threads hold any, and one workgroup has a row in registers' reach anyway), and launches
+// segment's groups of threads hold any, and one workgroup has a row in registers' reach anyway), rows longer
+// than the logits product makes them (kDrawVocabMax; rounding seg_len up to 4 shortens the last segment by
+// up to 4 elements per segment: about 500 of the 16384 at this length, all of them at 4096 segments), and launches
 // with too many workgroups.
 constexpr int kDrawSegment = 16384;
+constexpr int64_t kDrawVocabMax = 1 << 21;
 struct DrawSegments {
   int segs, seg_len;
   size_t counts_at(int64_t b, int k) const { return (size_t)b * segs * k * 8; }
@@ -200,7 +203,7 @@ struct DrawSegments {
 };
 inline DrawSegments draw_segments(int64_t b, int64_t vocab) {
   DrawSegments g = {(int)((vocab + kDrawSegment - 1) / kDrawSegment), 0};
-  if (b * g.segs > (1ll << 30) || g.segs > (1 << 20) || vocab < 4096) g.segs = 0;
+  if (b * g.segs > (1ll << 30) || vocab > kDrawVocabMax || vocab < 4096) g.segs = 0;
   else g.seg_len = (int)rup((vocab + g.segs - 1) / g.segs, 4);
   return g;
 }

@@ -6,7 +6,7 @@
 //   * make_plan: workspace regions are 256-byte aligned, do not overlap, end inside the totals;
 //     the vocab splits of the d_hidden product cover V; chunks cover N;
 //   * the no-alloc chunk search returns the largest chunk that fits, or refuses;
-//   * the sampler's work items cover the vocabulary.
+//   * the sampler's work items cover the vocabulary, and so do the segments of the draw.
 // Prints "ok <checks>" and exits 0, or a message and exits 1.
 #include <algorithm>
 #include <cstdio>
@@ -242,7 +242,33 @@ static void sampler_sweep() {
     }
 }
 
+// Segments of a row for the draw: they cover it, fit a workgroup's registers, and the last one still holds a list
+// of the longest k (the kernel reads whole quads up to the segment's end, so it must hold one at the very least).
+static void draw_sweep() {
+  auto check = [](int64_t b, int64_t v) {
+    const DrawSegments g = draw_segments(b, v);
+    CHECK(g.segs >= 0, "segs %d", g.segs);
+    if (g.segs == 0) {
+      CHECK(g.bytes(b, 50) == 0, "a workspace without segments");
+      return;
+    }
+    const int64_t last = v - (int64_t)(g.segs - 1) * g.seg_len;
+    CHECK(g.seg_len % 4 == 0 && g.seg_len <= kDrawSegment, "vocab %lld: segments of %d", (long long)v, g.seg_len);
+    CHECK(last >= 64 && last <= g.seg_len, "vocab %lld: %d segments of %d, the last one of %lld", (long long)v, g.segs, g.seg_len, (long long)last);
+    CHECK(b * g.segs <= (1ll << 30), "b %lld: %lld workgroups", (long long)b, (long long)(b * g.segs));
+    for (int k : {1, 50, 64}) CHECK(g.bytes(b, k) >= (size_t)b * g.segs * k * 8, "workspace of %zu bytes", g.bytes(b, k));
+  };
+  for (int64_t b : {1, 31, 32, 200, 1 << 16, 1 << 24}) {
+    for (int64_t v = 1; v <= 70000; v += 3) check(b, v);
+    for (int64_t n : {1, 2, 3, 4, 7, 10, 16, 63, 64, 65, 127, 128, 129, 1000, 4095, 4096, 4097, 65535})
+      for (int64_t d = -70; d <= 70; ++d)
+        if (n * kDrawSegment + d > 0) check(b, n * kDrawSegment + d);
+    for (int64_t v : {32000ll, 128256ll, 152064ll, 256000ll, 67092481ll, 67108865ll, 1ll << 21, (1ll << 21) + 1, 1ll << 30}) check(b, v);
+  }
+}
+
 int main() {
+  draw_sweep();
   tile_map_sweep();
   plan_sweep();
   noalloc_sweep();

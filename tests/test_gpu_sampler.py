@@ -192,3 +192,18 @@ def test_one_or_two_rows_on_the_vector_alus(b, h, v, cap):
     out = M.last_position_logits(hid.to(dev)[:, :h], w.to(dev)[:, :v], cap)
     ref = O.lm_head_logits(hid[:, :h].float().numpy(), w[:, :v].float().numpy(), cap)
     np.testing.assert_allclose(out.cpu().numpy(), ref, rtol=1e-5, atol=h * 3.2 * 2.0 ** -24 * 4)
+
+
+def test_a_row_whose_last_segment_would_be_a_single_logit():
+    """4095 * 16384 + 1 logits, all negative, the largest at the very end: cut into 4096 segments the last one
+    would hold one logit.  Distinct values, so the top k of the row is that of torch.topk."""
+    import mllm_jax_amd as M
+    v = 4095 * 16384 + 1
+    row = torch.full((1, v), -5.0, device="cuda:0")
+    at = torch.arange(63, device="cuda:0") * 1000003 + 17
+    row[0, at] = -1.0 - 0.01 * torch.arange(63, device="cuda:0")
+    row[0, v - 1] = -0.5
+    tok, idx, val = M.top_k_sampling_batched(None, row, k=64, t=1.0, return_top_k=True)
+    assert int(tok[0]) == v - 1
+    assert idx[0].tolist() == [v - 1] + at.tolist()
+    assert torch.equal(val[0], row[0, idx[0].long()])
