@@ -1389,9 +1389,12 @@ __global__ __launch_bounds__(64 * kFewWaves) void k_logits_few(LogitsRowsArgs p)
   auto use = [&](int g, const u32x4 (&w)[8]) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-      // sixteen hidden values of row b (clamped: a row past n is computed and not stored, so are k-rows past H)
+      // sixteen hidden values of row b (clamped: a row past n is computed and not stored); k-rows past H are zeros
+      // on this side too, since W's zeros alone would make NaNs of infinities
       const const_quads x = (const_quads)(uintptr_t)(p.hid + (int64_t)min(b, p.n - 1) * p.ld_hid);
-      const u32x4 x0 = x[2 * g], x1 = x[min(2 * g + 1, (p.H >> 3) - 1)];
+      const u32x4 x0 = x[2 * g];
+      u32x4 x1 = {0u, 0u, 0u, 0u};
+      if (2 * g + 1 < (p.H >> 3)) x1 = x[2 * g + 1];
 #pragma unroll
       for (int r = 0; r < 8; ++r) {
         const uint32_t pair = r < 4 ? x0[r] : x1[r - 4];

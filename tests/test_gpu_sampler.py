@@ -207,3 +207,22 @@ def test_a_row_whose_last_segment_would_be_a_single_logit():
     assert int(tok[0]) == v - 1
     assert idx[0].tolist() == [v - 1] + at.tolist()
     assert torch.equal(val[0], row[0, idx[0].long()])
+
+
+@pytest.mark.parametrize("b", [1, 2, 3])
+@pytest.mark.parametrize("h", [8, 24, 40, 136, 144])
+def test_infinities_in_hidden_stay_infinities(b, h):
+    """An infinity in the last eight hidden values gives +-inf logits and no NaN (no entry of W is zero), for
+    lengths that end in the middle of a group of sixteen k-rows and for those that do not; three rows take
+    the matrix form."""
+    import mllm_jax_amd as M
+    dev = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(h)
+    hid = torch.randn(b, h, generator=g).to(torch.bfloat16)
+    w = torch.randn(h, 520, generator=g).to(torch.bfloat16)
+    w[w == 0] = 1.0
+    hid[0, h - 3] = float("inf")
+    out = M.last_position_logits(hid.to(dev), w.to(dev)).cpu()
+    expect = torch.where(w[h - 3] > 0, float("inf"), float("-inf"))
+    assert torch.equal(out[0], expect)
+    assert bool(torch.isfinite(out[1:]).all())
