@@ -623,9 +623,16 @@ int mj_sample_logits(const void* hidden, int64_t ld_hidden, const void* lm_head,
   return check_launch("k_logits_rows");
 }
 
+static int draw_check(int64_t ld_logits, int64_t b, int64_t vocab, int k) {
+  if (b <= 0 || vocab <= 0 || b > (1 << 24) || vocab > (1 << 30) || ld_logits < vocab)
+    return fail(MJ_GRPO_ERR_SHAPE, "sample_top_k: bad shape b=%lld vocab=%lld ld=%lld", (long long)b, (long long)vocab, (long long)ld_logits);
+  if (k < 1 || k > mj::kTopKMax || k > vocab) return fail(MJ_GRPO_ERR_UNSUPPORTED, "sample_top_k: k must be in [1, min(%d, vocab)] (got %d)", mj::kTopKMax, k);
+  return MJ_GRPO_OK;
+}
+
 int mj_sample_draw_workspace_bytes(int64_t b, int64_t vocab, int k, size_t* bytes) {
-  if (b <= 0 || vocab <= 0 || b > (1 << 24) || vocab > (1 << 30) || k < 1 || k > mj::kTopKMax)
-    return fail(MJ_GRPO_ERR_SHAPE, "sample_draw: bad shape b=%lld vocab=%lld k=%d", (long long)b, (long long)vocab, k);
+  int rc;
+  if ((rc = draw_check(vocab, b, vocab, k))) return rc;
   if (bytes) *bytes = draw_segments(b, vocab).bytes(b, k);
   return MJ_GRPO_OK;
 }
@@ -634,9 +641,8 @@ int mj_sample_draw(const float* logits, int64_t ld_logits, int64_t b, int64_t vo
                    const float* noise, int32_t* token, int32_t* top_idx, float* top_val,
                    void* workspace, size_t workspace_bytes, void* stream) {
   if (!logits || !token) return fail(MJ_GRPO_ERR_NULL, "sample_top_k: logits/token is NULL");
-  if (b <= 0 || vocab <= 0 || b > (1 << 24) || vocab > (1 << 30) || ld_logits < vocab)
-    return fail(MJ_GRPO_ERR_SHAPE, "sample_top_k: bad shape b=%lld vocab=%lld ld=%lld", (long long)b, (long long)vocab, (long long)ld_logits);
-  if (k < 1 || k > mj::kTopKMax || k > vocab) return fail(MJ_GRPO_ERR_UNSUPPORTED, "sample_top_k: k must be in [1, min(%d, vocab)] (got %d)", mj::kTopKMax, k);
+  int rc;
+  if ((rc = draw_check(ld_logits, b, vocab, k))) return rc;
   if (!(temperature > 0.f) || !isfinite(temperature)) return fail(MJ_GRPO_ERR_UNSUPPORTED, "sample_top_k: temperature must be > 0");
   mj::TopKArgs a;
   a.logits = logits; a.ld = ld_logits; a.V = (int)vocab; a.k = k; a.t = temperature; a.noise = noise;

@@ -167,6 +167,15 @@ def test_sampler_argument_checks_before_any_launch(lib):
     assert h.mj_sample_top_k(fake, 512, 4, 40, 50, 1.0, None, fake, None, None, None) == 5      # k > vocab
     assert h.mj_sample_top_k(fake, 512, 4, 512, 50, 0.0, None, fake, None, None, None) == 5
     assert h.mj_sample_top_k(fake, 512, 4, 512, 50, 1.0, None, None, None, None, None) == 1
+    # the workspace query refuses what the draw refuses, with the same status and text
+    need = C.c_size_t()
+    for b, v, k in [(4, 512, 65), (4, 512, 0), (4, 40, 50), (0, 512, 50), (4, 1 << 31, 50)]:
+        drawn = h.mj_sample_draw(fake, v, b, v, k, 1.0, None, fake, None, None, None, 0, None)
+        text = h.mj_grpo_last_error()
+        assert drawn == (5 if b == 4 and v < 1000 else 2)
+        assert h.mj_sample_draw_workspace_bytes(b, v, k, C.byref(need)) == drawn
+        assert h.mj_grpo_last_error() == text
+    assert h.mj_sample_draw_workspace_bytes(4, 152064, 50, C.byref(need)) == 0 and need.value > 0
 
 
 def test_skip_masked_flag_enlarges_the_workspace(lib):
