@@ -647,7 +647,7 @@ int mj_sample_draw(const float* logits, int64_t ld_logits, int64_t b, int64_t vo
   mj::TopKArgs a;
   a.logits = logits; a.ld = ld_logits; a.V = (int)vocab; a.k = k; a.t = temperature; a.noise = noise;
   a.token = token; a.top_idx = top_idx; a.top_val = top_val;
-  a.words = nullptr; a.counts = nullptr; a.segs = a.seg_len = 0;
+  a.words = nullptr; a.segs = a.seg_len = 0;
   if (workspace != nullptr) {
     const DrawSegments g = draw_segments(b, vocab);
     if (workspace_bytes < g.bytes(b, k))
@@ -656,7 +656,6 @@ int mj_sample_draw(const float* logits, int64_t ld_logits, int64_t b, int64_t vo
     if (g.segs > 0) {
       a.segs = g.segs; a.seg_len = g.seg_len;
       a.words = (uint64_t*)workspace;
-      a.counts = (uint32_t*)((char*)workspace + g.counts_at(b, k));
       mj::k_topk_segments<<<(unsigned)(b * g.segs), mj::kSegThreads, 0, (hipStream_t)stream>>>(a);
     }
   }

@@ -1453,7 +1453,6 @@ struct TopKArgs {
   float* top_val;        // [b, k] or null (logits / t, descending)
   int segs, seg_len;     // k_topk_segments: pieces of a row and their length (a multiple of 4)
   uint64_t* words;       // [b, segs, k] each segment's largest, descending; null: no segment pass was run
-  uint32_t* counts;      // [b, segs] how many of the k words are there; kSegOverflow: too many near-equal values
 };
 
 MJ_DEV uint32_t topk_key(float f) {   // larger float <=> larger key; -0 and +0 differ only in sign bit order
@@ -1475,22 +1474,32 @@ MJ_DEV float nan_max(float a, float b) { return __builtin_elementwise_maximum(a,
 // 152064 logits is 10 workgroups, the elements stay in registers (8 quads per thread) and are read once.
 // What is left to pay is instructions, so the work per element is a share of its quad's maximum and of one
 // comparison; everything else happens to the few quads that matter, behind an LDS pool.
-// Threshold: the threads form 64 groups of eight; at least k elements reach the k-th largest of the 64 group
-// maxima, `tau`, and few more do (about 100 for k = 50).  x -> key(x / t) is non-decreasing, so the k-th
-// largest key is at least key(tau / t), and an element whose key reaches it has x >= tau up to the rounding
-// of the two quotients: x >= tau_lo, a few ulps below tau.  Elements not below tau_lo (NaNs included:
-// their key is the largest) are ranked by their exact keys.  Groups without elements or with a NaN count as
-// -inf, which only lowers tau; a pool that overflows is reported to k_topk_sample.
+// Threshold: the threads form 128 groups of four; at least k elements reach the k-th largest of the 128 group
+// maxima, `tau`, and few more do (128 ln(128 / (128 - k)) in the mean, 64 for k = 50 and 89 for k = 64; 64 groups
+// gave 97 and, being the smallest of all maxima at k = 64, about 300).  x -> key(x / t) is non-decreasing, so the
+// k-th largest key is at least key(tau / t), and an element whose key reaches it has x >= tau up to the rounding
+// of the two quotients: x >= tau_lo, a few ulps below tau.  Elements not below tau_lo (NaNs included) are
+// ranked by their exact keys.  Groups with a NaN count as -inf, which only lowers tau.
+// Where more elements reach tau_lo than the pool holds, or fewer than k groups hold anything but -inf (blocks of
+// masked tokens and their edges), the threshold is taken once more, from the threads' own maxima.  A segment for
+// which that does not help either (one value everywhere, very many near-equal ones) finds its k-th largest key bit
+// by bit, counting over the registers, so that every list is complete whatever the values are.
+// 80 registers (three workgroups on a CU) without scratch.  128 rows of 152064, k = 50: the draw's two kernels take
+// 21.8 us, one workgroup per row 36.6; 64 rows with a block of 30000 at -inf: 20.3 and 28.0; 16 rows, k = 64: 11.6
+// and 22.6.
 constexpr int kSegThreads = 512, kSegUnits = 8, kSegMax = kSegThreads * kSegUnits * 4, kSegPool = 512;
-constexpr uint32_t kSegOverflow = 0xffffffffu;
-__global__ __launch_bounds__(kSegThreads, 8) void k_topk_segments(TopKArgs p) {
-  __shared__ __attribute__((aligned(16))) float s_max[64];
+constexpr int kSegGroups = kSegThreads / 4;
+static_assert(kSegGroups == 128 && kTopKMax < kSegGroups, "four threads rank one group's maximum among 128");
+__global__ __launch_bounds__(kSegThreads, 6) void k_topk_segments(TopKArgs p) {
+  __shared__ __attribute__((aligned(16))) float s_max[kSegGroups];
+  __shared__ __attribute__((aligned(16))) float s_tau[kSegThreads / 64];
   __shared__ __attribute__((aligned(16))) f32x4 s_quad[kSegPool];
   __shared__ int s_at[kSegPool];                 // row index of the quad's first element, top bits: elements to skip
   __shared__ __attribute__((aligned(16))) uint64_t pool[kSegPool];
-  __shared__ uint32_t s_quads, s_pool;
-  __shared__ float s_tau;
-  const int tid = threadIdx.x, lane = tid & 63;
+  __shared__ __attribute__((aligned(16))) int s_count[2][kSegThreads / 64];
+  __shared__ __attribute__((aligned(16))) int s_ties[4 * kSegUnits][kSegThreads / 64];
+  __shared__ uint32_t s_quads, s_pool, s_chosen;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = blockIdx.x / p.segs, seg = blockIdx.x - r * p.segs;
   const int i0 = min(seg * p.seg_len, p.V), len = min(p.seg_len, p.V - i0);      // len >= 64: the host's segments
   const float* base = p.logits + (int64_t)r * p.ld + i0;
@@ -1508,71 +1517,201 @@ __global__ __launch_bounds__(kSegThreads, 8) void k_topk_segments(TopKArgs p) {
     if ((u * kSegThreads + tid) * 4 + 4 > len) m[u] = -__builtin_inff();    // past or across the end: not a witness for tau
     mx = nan_max(mx, m[u]);
   }
-#pragma unroll
-  for (int o = 1; o < 8; o <<= 1) mx = nan_max(mx, __shfl_xor(mx, o));
-  if ((tid & 7) == 0) s_max[tid >> 3] = mx == mx ? mx : -__builtin_inff();
-  if (tid == 0) { s_quads = 0; s_pool = 0; }
+  mx = nan_max(mx, __shfl_xor(mx, 1));
+  mx = nan_max(mx, __shfl_xor(mx, 2));
+  if ((tid & 3) == 0) s_max[tid >> 2] = mx == mx ? mx : -__builtin_inff();
+  if (tid == 0) { s_quads = 0; s_pool = 0; s_chosen = 0; }
   __syncthreads();
-  if (tid < 64) {
-    const float mine = s_max[lane];
+  {
+    const float mine = s_max[tid >> 2];
     int above = 0;
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const f32x4 o = *(const f32x4*)(s_max + 4 * q);
+    for (int q = 0; q < kSegGroups / 16; ++q) {
+      const f32x4 o = *(const f32x4*)(s_max + 16 * q + 4 * (tid & 3));
 #pragma unroll
       for (int j = 0; j < 4; ++j) above += o[j] > mine ? 1 : 0;
     }
-    float tau = above < p.k ? mine : __builtin_inff();      // the k largest are among these
+    above += __shfl_xor(above, 1);
+    above += __shfl_xor(above, 2);
+    float least = above < p.k ? mine : __builtin_inff();      // the k largest are among these
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) tau = fminf(tau, __shfl_xor(tau, o));
-    if (lane == 0) s_tau = tau;
+    for (int o = 4; o < 64; o <<= 1) least = fminf(least, __shfl_xor(least, o));
+    if (lane == 0) s_tau[wave] = least;
   }
   __syncthreads();
-  const float tau = s_tau;
-  const float tau_lo = tau - fmaxf(fabsf(tau) * 0x1p-20f, 0x1p-100f);
-  // Quads with an element that is not below tau_lo; places by ballots and one LDS atomic per wavefront.
-  uint64_t hit[kSegUnits];
-  int count = 0;
+  float tau = s_tau[0];
 #pragma unroll
-  for (int u = 0; u < kSegUnits; ++u) {
-    const int e = (u * kSegThreads + tid) * 4;
-    hit[u] = __ballot(e < len && (!(m[u] < tau_lo) || e + 4 > len));
-    count += __popcll(hit[u]);
-  }
-  uint32_t first = 0;
-  if (lane == 0 && count > 0) first = atomicAdd(&s_quads, (uint32_t)count);
-  uint32_t at = __builtin_amdgcn_readfirstlane(first);
+  for (int w = 1; w < kSegThreads / 64; ++w) tau = fminf(tau, s_tau[w]);
+  int turn = 0;
+  auto total = [&](int n) {                      // of one number per wavefront; one barrier, alternating slots
+    if (lane == 0) s_count[turn][wave] = n;
+    __syncthreads();
+    int sum = 0;
 #pragma unroll
-  for (int u = 0; u < kSegUnits; ++u) {
-    const uint32_t slot = at + __builtin_amdgcn_mbcnt_hi((uint32_t)(hit[u] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)hit[u], 0));
-    if (((hit[u] >> lane) & 1) && slot < (uint32_t)kSegPool) {
-      const int e = (u * kSegThreads + tid) * 4, s = min(e, len - 4);
-      s_quad[slot] = x[u];
-      s_at[slot] = s | ((e - s) << 28);
+    for (int w = 0; w < kSegThreads / 64; ++w) sum += s_count[turn][w];
+    turn ^= 1;
+    return __builtin_amdgcn_readfirstlane(sum);
+  };
+  uint32_t pooled = 0;
+  bool over;                                     // uniform
+  for (bool again = false;; again = true) {
+    const float tau_lo = tau - fmaxf(fabsf(tau) * 0x1p-20f, 0x1p-100f);
+    const bool narrow = tau > -__builtin_inff();            // uniform; -inf leaves nothing out
+    if (narrow) {
+      // Quads with an element that is not below tau_lo; places by ballots and one LDS atomic per wavefront.
+      uint64_t hit[kSegUnits];
+      int count = 0;
+#pragma unroll
+      for (int u = 0; u < kSegUnits; ++u) {
+        const int e = (u * kSegThreads + tid) * 4;
+        hit[u] = __ballot(e < len && (!(m[u] < tau_lo) || e + 4 > len));
+        count += __popcll(hit[u]);
+      }
+      uint32_t first = 0;
+      if (lane == 0 && count > 0) first = atomicAdd(&s_quads, (uint32_t)count);
+      uint32_t at = __builtin_amdgcn_readfirstlane(first);
+#pragma unroll
+      for (int u = 0; u < kSegUnits; ++u) {
+        const uint32_t slot = at + __builtin_amdgcn_mbcnt_hi((uint32_t)(hit[u] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)hit[u], 0));
+        if (((hit[u] >> lane) & 1) && slot < (uint32_t)kSegPool) {
+          const int e = (u * kSegThreads + tid) * 4, s = min(e, len - 4);
+          s_quad[slot] = x[u];
+          s_at[slot] = s | ((e - s) << 28);
+        }
+        at += __popcll(hit[u]);
+      }
+      __syncthreads();
+      // their elements, one per thread, with the exact key
+      for (uint32_t q = tid; q < min(s_quads, (uint32_t)kSegPool) * 4; q += kSegThreads) {
+        const float v = ((const float*)s_quad)[q];
+        const int s = s_at[q >> 2], j = (int)(q & 3);
+        const bool ok = !(v < tau_lo) && j >= (s >> 28);
+        const uint64_t b = __ballot(ok);
+        uint32_t f = 0;
+        if (ok) {
+          const int leader = __builtin_ctzll(b);
+          if (lane == leader) f = atomicAdd(&s_pool, (uint32_t)__popcll(b));
+          f = __shfl(f, leader) + __builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0));
+          if (f < (uint32_t)kSegPool) pool[f] = topk_word(v, p.t, i0 + (s & 0xfffffff) + j);
+        }
+      }
+      __syncthreads();
     }
-    at += __popcll(hit[u]);
-  }
-  __syncthreads();
-  const uint32_t quads = s_quads;
-  // their elements, one per thread, with the exact key
-  for (uint32_t q = tid; q < min(quads, (uint32_t)kSegPool) * 4; q += kSegThreads) {
-    const float v = ((const float*)s_quad)[q];
-    const int s = s_at[q >> 2], j = (int)(q & 3);
-    const bool ok = !(v < tau_lo) && j >= (s >> 28);
-    const uint64_t b = __ballot(ok);
-    uint32_t f = 0;
-    if (ok) {
-      const int leader = __builtin_ctzll(b);
-      if (lane == leader) f = atomicAdd(&s_pool, (uint32_t)__popcll(b));
-      f = __shfl(f, leader) + __builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0));
-      if (f < (uint32_t)kSegPool) pool[f] = topk_word(v, p.t, i0 + (s & 0xfffffff) + j);
+    pooled = s_pool;
+    over = !narrow || s_quads > (uint32_t)kSegPool || pooled > (uint32_t)kSegPool;
+    if (!over || again) break;
+    // fewer than k groups hold anything above a repeated lowest value (a masked block's edge): the k-th largest
+    // of the 512 threads' own maxima, bit by bit
+    float top = m[0];
+#pragma unroll
+    for (int u = 1; u < kSegUnits; ++u) top = nan_max(top, m[u]);
+    const uint32_t own = topk_key(top == top ? top : -__builtin_inff());
+    const uint32_t floor = topk_key(tau);
+    if (total(__popcll(__ballot(own > floor))) < p.k) break;
+    uint32_t K = 0;
+    for (int bit = 31; bit >= 0; --bit) {
+      const uint32_t c = K | (1u << bit);
+      const int n = total(__popcll(__ballot(own >= c)));
+      if (n >= p.k) K = c;
+      if (n == p.k) break;
     }
+    tau = topk_unkey(K);
+    if (tid == 0) { s_quads = 0; s_pool = 0; }
+    __syncthreads();
   }
-  __syncthreads();
-  const uint32_t pooled = s_pool;
-  const bool over = quads > (uint32_t)kSegPool || pooled > (uint32_t)kSegPool;
-  if (tid == 0) p.counts[blockIdx.x] = over ? kSegOverflow : min(pooled, (uint32_t)p.k);
-  if (over) return;
+  if (over) {
+    // The largest key K that at least k elements reach, from its top bit down; then, of the elements equal to
+    // K, the lowest indices.  The segment is read a second time, element q * 512 + tid in register q (its place
+    // and its bound are then one comparison, and the quads above need not stay alive); past the end: key 0, which
+    // no count asks for.
+    constexpr int kPer = 4 * kSegUnits;
+    uint32_t key[kPer];
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+      const int i = q * kSegThreads + tid;
+      key[q] = __builtin_amdgcn_raw_buffer_load_b32(rs, (uint32_t)min(i, len - 1) * 4, 0, 0);
+    }
+    // one value everywhere (a block of masked tokens): the first k indices
+    bool same = true;
+    const uint32_t front = __builtin_amdgcn_readfirstlane(__float_as_uint(base[0]));
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) same = same && key[q] == front;
+    if (__syncthreads_and(same)) {
+      if (tid < p.k) p.words[(int64_t)blockIdx.x * p.k + tid] = topk_word(__uint_as_float(front), p.t, i0 + tid);
+      return;
+    }
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) key[q] = q * kSegThreads + tid < len ? topk_key(__uint_as_float(key[q]) / p.t) : 0u;
+    auto count = [&](auto&& f) {
+      int c = 0, n = 0;
+#pragma unroll
+      for (int q = 0; q < kPer; ++q) c += f(key[q]) ? 1 : 0;
+#pragma unroll
+      for (int bit = 0; bit < 6; ++bit) n += __popcll(__ballot((c >> bit) & 1)) << bit;      // c <= 32
+      return total(n);
+    };
+    // a block of equal values: the threshold's own key is K
+    uint32_t K = __builtin_amdgcn_readfirstlane(topk_key(tau / p.t));
+    int reach = count([&](uint32_t x) { return x >= K; });     // elements with a key of at least K
+    int more = count([&](uint32_t x) { return x > K; });       // and above K
+    if (reach < p.k || more >= p.k) {
+      K = 0;
+      reach = len;
+      more = 0;
+      for (int bit = 31; bit >= 0 && reach != p.k; --bit) {
+        const uint32_t c = K | (1u << bit);
+        const int n = count([&](uint32_t x) { return x >= c; });
+        if (n >= p.k) { K = c; reach = n; }
+        else more = n;                           // the last such c is K + 1 once all bits are done
+      }
+    }
+    // Elements above K in any order, of those equal to K the first `wanted` by index, which is register by
+    // register and then wavefront by wavefront: their counts per register and wavefront, summed up in front of each.
+    const bool all = reach == p.k;
+    // opaque copies: the comparisons are made anew in each loop, not kept in 64 registers
+    auto opaque = [](int v) { v = __builtin_amdgcn_readfirstlane(v); asm volatile("" : "+s"(v)); return v; };
+    int end = opaque(len), at_K = opaque((int)K);
+    const int wanted = p.k - more;
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+      const int n = __popcll(__ballot(key[q] == (uint32_t)at_K && q * kSegThreads + tid < end));
+      if (lane == 0) s_ties[q][wave] = n;
+    }
+    __syncthreads();
+    if (tid < kPer) {
+      int own[kSegThreads / 64], sum = 0;
+#pragma unroll
+      for (int w = 0; w < kSegThreads / 64; ++w) { own[w] = sum; sum += s_ties[tid][w]; }
+      int before = sum;
+#pragma unroll
+      for (int o = 1; o < kPer; o <<= 1) {
+        const int other = __shfl_up(before, o);
+        if (tid >= o) before += other;
+      }
+#pragma unroll
+      for (int w = 0; w < kSegThreads / 64; ++w) s_ties[tid][w] = before - sum + own[w];
+    }
+    __syncthreads();
+    const int in_front = lane < kPer ? s_ties[lane][wave] : 0;      // lane q: ties in front of register q of this wavefront
+    end = opaque(len);
+    at_K = opaque((int)K);
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+      const int i = q * kSegThreads + tid;
+      const uint64_t ties = __ballot(key[q] == (uint32_t)at_K && i < end);
+      const int before = __builtin_amdgcn_readlane(in_front, q);
+      const bool some = all || before < wanted;
+      if (__ballot(key[q] > (uint32_t)at_K) != 0 || (ties != 0 && some)) {
+        const int rank = before + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(ties >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)ties, 0));
+        if (i < end && (key[q] > (uint32_t)at_K || (key[q] == (uint32_t)at_K && (all || rank < wanted)))) {
+          const uint32_t slot = atomicAdd(&s_chosen, 1u);
+          if (slot < (uint32_t)kSegPool) pool[slot] = ((uint64_t)key[q] << 32) | (uint32_t)~(i0 + i);
+        }
+      }
+    }
+    __syncthreads();
+    pooled = s_chosen;                           // == k
+  }
   const uint32_t padded = (pooled + 7u) & ~7u;
   if ((uint32_t)tid >= pooled && (uint32_t)tid < padded) pool[tid] = 0ull;
   __syncthreads();
@@ -1645,19 +1784,15 @@ __global__ __launch_bounds__(1024) void k_topk_sample(TopKArgs p) {
   constexpr int kRankPool = 1024;
   if (tid == 0) s_pool = 0;
   if (p.words != nullptr) {
-    // The segments' lists hold the top k.  A list's word number ceil(k / segs) - 1 is reached by that
-    // many words of the list, so at least k words reach the smallest of these over the lists: the words
-    // that do -- a few more than k -- are ranked below.  (An incomplete list counts as 0: all qualify.)
+    // The segments' lists of k words each hold the top k.  A list's word number ceil(k / segs) - 1 is reached by
+    // that many words of the list, so at least k words reach the smallest of these over the lists: the words
+    // that do -- a few more than k -- are ranked below.
     const uint64_t* words = p.words + (int64_t)blockIdx.x * p.segs * p.k;
-    const uint32_t* counts = p.counts + (int64_t)blockIdx.x * p.segs;
     if (wave == 0) {
-      const uint32_t place = (uint32_t)((p.k + p.segs - 1) / p.segs);
+      const int place = (p.k + p.segs - 1) / p.segs;
       uint64_t tau = ~0ull;
-      bool full = false;
       for (int q = lane; q < p.segs; q += 64) {
-        const uint32_t c = counts[q];
-        full |= c == kSegOverflow;
-        const uint64_t w = c >= place && c != kSegOverflow ? words[(int64_t)q * p.k + place - 1] : 0ull;
+        const uint64_t w = words[(int64_t)q * p.k + place - 1];
         tau = w < tau ? w : tau;
       }
 #pragma unroll
@@ -1665,20 +1800,16 @@ __global__ __launch_bounds__(1024) void k_topk_sample(TopKArgs p) {
         const uint64_t other = __shfl_xor((unsigned long long)tau, o);
         tau = other < tau ? other : tau;
       }
-      if (__any(full) && lane == 0) s_pool = kRankPool + 1;      // the histogram paths take the row
       if (lane == 0) s_tau_word = tau;
     }
     const int total = p.segs * p.k;
-    auto word = [&](int q) -> uint64_t {         // 0: no such word
-      const int seg = q / p.k;
-      return q < total && (uint32_t)(q - seg * p.k) < min(counts[seg], (uint32_t)p.k) ? words[q] : 0ull;
-    };
+    auto word = [&](int q) -> uint64_t { return q < total ? words[q] : 0ull; };
     const uint64_t first = word(tid);            // requested before the barrier; usually all there is
     __syncthreads();
     const uint64_t tau = s_tau_word;
     for (int q = tid; q < total; q += 1024) {
       const uint64_t w = q == tid ? first : word(q);
-      if (w == 0ull || w < tau) continue;
+      if (w < tau) continue;
       const uint32_t slot = atomicAdd(&s_pool, 1u);
       if (slot < (uint32_t)kRankPool) ranked_word[slot] = w;
     }

@@ -198,8 +198,7 @@ constexpr int kDrawSegment = 16384;
 constexpr int64_t kDrawVocabMax = 1 << 21;
 struct DrawSegments {
   int segs, seg_len;
-  size_t counts_at(int64_t b, int k) const { return (size_t)b * segs * k * 8; }
-  size_t bytes(int64_t b, int k) const { return counts_at(b, k) + (size_t)b * segs * 4; }
+  size_t bytes(int64_t b, int k) const { return (size_t)b * segs * k * 8; }     // k 64-bit words per segment
 };
 inline DrawSegments draw_segments(int64_t b, int64_t vocab) {
   DrawSegments g = {(int)((vocab + kDrawSegment - 1) / kDrawSegment), 0};

@@ -226,3 +226,36 @@ def test_infinities_in_hidden_stay_infinities(b, h):
     expect = torch.where(w[h - 3] > 0, float("inf"), float("-inf"))
     assert torch.equal(out[0], expect)
     assert bool(torch.isfinite(out[1:]).all())
+
+
+@pytest.mark.filterwarnings("ignore:overflow encountered in divide")
+@pytest.mark.parametrize("v,k", [(8200, 64), (16388, 50), (40001, 64), (152064, 64), (152064, 1), (70 * 16384 + 5, 3), (1 << 21, 64)])
+def test_masked_blocks_and_crowded_segments(v, k):
+    """Segments in which more elements reach the threshold than the pool holds: blocks of -inf and of the
+    type's lowest value that fill whole segments, rows with a handful of unmasked logits, one value everywhere,
+    ties in the middle of a segment, two neighbouring floats, NaNs; also more segments than k and than a
+    wavefront has lanes, and lists whose words overflow the draw's pool.  Bit for bit the oracle's choice."""
+    import mllm_jax_amd as M
+    dev = torch.device("cuda:0")
+    rng = np.random.default_rng(v + k)
+    x = rng.normal(0, 2, size=(11, v)).astype(np.float32)
+    low = np.finfo(np.float32).min
+    x[1, v // 4:v // 4 + 40000] = -np.inf
+    x[2, v // 4:v // 4 + 40000] = low
+    x[3] = -np.inf
+    x[3, rng.choice(v, size=40, replace=False)] = rng.normal(0, 2, size=40).astype(np.float32)
+    x[4] = low
+    x[4, v - 30:] = rng.normal(0, 2, size=30).astype(np.float32)
+    x[5] = -1.25
+    x[6, ::3] = 3.0                                                     # a third of the row, larger than most others
+    x[7] = np.where(rng.random(v) < 0.5, np.float32(2.0), np.nextafter(np.float32(2.0), np.float32(3.0)))
+    x[8, 700:] = low                                                    # the edge of a masked block
+    x[9, 1000:] = -np.inf
+    x[9, ::5] = np.round(x[9, ::5])                                     # few distinct values above it
+    x[10, :20000] = np.nan
+    noise = rng.gumbel(size=(11, k)).astype(np.float32)
+    tok, idx, val = M.top_k_sampling_batched(torch.tensor(noise), torch.tensor(x, device=dev), k=k, t=0.9, return_top_k=True)
+    rt, ri, rv = O.top_k_sample(x, k=k, t=0.9, noise=noise)
+    np.testing.assert_array_equal(idx.cpu().numpy(), ri)
+    np.testing.assert_array_equal(val.cpu().numpy().view(np.uint32), rv.view(np.uint32))
+    np.testing.assert_array_equal(tok.cpu().numpy()[:10], rt[:10])       # what argmax makes of NaN scores is not at issue here
