@@ -1467,6 +1467,14 @@ MJ_DEV float topk_unkey(uint32_t key) {
 // One 64-bit word per element whose order is (key descending, index ascending); never 0.
 MJ_DEV uint64_t topk_word(float x, float t, int i) { return ((uint64_t)topk_key(x / t) << 32) | (uint32_t)~i; }
 
+// No element below the result shares the quotient tau / t: a few ulps below tau, or -inf (nothing can be left out)
+// where the quotient is infinite, or so small beside tau that logits far apart share it.
+MJ_DEV float topk_below(float tau, float t) {
+  const float q = fabsf(tau / t);
+  if (!(q < __builtin_inff()) || (t > 1.f && q < 0x1p-126f)) return -__builtin_inff();
+  return tau - fmaxf(fabsf(tau) * 0x1p-20f, 0x1p-100f);
+}
+
 MJ_DEV float nan_max(float a, float b) { return __builtin_elementwise_maximum(a, b); }   // a NaN if either is one
 
 // The k largest of one segment of a row.  One workgroup for a whole row leaves a decode batch of a few
@@ -1478,7 +1486,7 @@ MJ_DEV float nan_max(float a, float b) { return __builtin_elementwise_maximum(a,
 // maxima, `tau`, and few more do (128 ln(128 / (128 - k)) in the mean, 64 for k = 50 and 89 for k = 64; 64 groups
 // gave 97 and, being the smallest of all maxima at k = 64, about 300).  x -> key(x / t) is non-decreasing, so the
 // k-th largest key is at least key(tau / t), and an element whose key reaches it has x >= tau up to the rounding
-// of the two quotients: x >= tau_lo, a few ulps below tau.  Elements not below tau_lo (NaNs included) are
+// of the two quotients: x >= tau_lo (topk_below).  Elements not below tau_lo (NaNs included) are
 // ranked by their exact keys.  Groups with a NaN count as -inf, which only lowers tau.
 // Where more elements reach tau_lo than the pool holds, or fewer than k groups hold anything but -inf (blocks of
 // masked tokens and their edges), the threshold is taken once more, from the threads' own maxima.  A segment for
@@ -1555,8 +1563,8 @@ __global__ __launch_bounds__(kSegThreads, 6) void k_topk_segments(TopKArgs p) {
   uint32_t pooled = 0;
   bool over;                                     // uniform
   for (bool again = false;; again = true) {
-    const float tau_lo = tau - fmaxf(fabsf(tau) * 0x1p-20f, 0x1p-100f);
-    const bool narrow = tau > -__builtin_inff();            // uniform; -inf leaves nothing out
+    const float tau_lo = topk_below(tau, p.t);
+    const bool narrow = tau_lo > -__builtin_inff();         // uniform; -inf leaves nothing out
     if (narrow) {
       // Quads with an element that is not below tau_lo; places by ballots and one LDS atomic per wavefront.
       uint64_t hit[kSegUnits];
@@ -1776,8 +1784,8 @@ __global__ __launch_bounds__(1024) void k_topk_sample(TopKArgs p) {
   // so at least 64 >= k elements reach the smallest of the 64 group maxima, `tau` (a group without
   // elements or with nothing but NaNs leaves tau = -inf, and then every element qualifies).
   // x -> key(x / t) is non-decreasing, so the k-th largest key is at least key(tau / t), and an
-  // element whose key reaches it has x >= tau up to the rounding of the two quotients: x >= tau_lo,
-  // a few ulps below tau.  Second read: elements that are not below tau_lo (NaNs included: their key
+  // element whose key reaches it has x >= tau up to the rounding of the two quotients: x >= tau_lo
+  // (topk_below).  Second read: elements that are not below tau_lo (NaNs included: their key
   // is the largest) go to a pool with their exact keys -- a few hundred for logits of a language
   // model -- where each one's rank under (key descending, index ascending) is counted directly.
   // A pool that overflows (rows of near-equal values) takes the histogram paths below instead.
@@ -1823,7 +1831,7 @@ __global__ __launch_bounds__(1024) void k_topk_sample(TopKArgs p) {
     float tau = s_gmax[lane];
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) tau = fminf(tau, __shfl_xor(tau, o));
-    const float tau_lo = tau - fmaxf(fabsf(tau) * 0x1p-20f, 0x1p-100f);
+    const float tau_lo = topk_below(tau, p.t);
     for_each([&](int i, float x) {
       if (!(x < tau_lo)) {
         const uint32_t slot = atomicAdd(&s_pool, 1u);

@@ -9,6 +9,22 @@ from oracle import grpo_oracle as O
 pytestmark = pytest.mark.gpu
 
 
+def _draw(noise, x, k, t, v=None):
+    """Tokens, indices and values of both forms of the draw, which must agree: mj_sample_draw with its workspace
+    (top_k_sampling_batched: long rows in segments) and mj_sample_top_k (one workgroup per row)."""
+    import mllm_jax_amd as M
+    from mllm_jax_amd import _lib
+    dev = torch.device("cuda:0")
+    lg = torch.tensor(x, device=dev)[:, :v]
+    nz = None if noise is None else torch.tensor(noise, device=dev)
+    tok, idx, val = M.top_k_sampling_batched(nz, lg, k=k, t=t, return_top_k=True)
+    tok1, idx1, val1 = torch.empty_like(tok), torch.empty_like(idx), torch.empty_like(val)
+    _lib.check(_lib.load().mj_sample_top_k(lg.data_ptr(), lg.stride(0), lg.shape[0], lg.shape[1], k, t, None if nz is None else nz.data_ptr(),
+                                           tok1.data_ptr(), idx1.data_ptr(), val1.data_ptr(), torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(tok, tok1) and torch.equal(idx, idx1) and torch.equal(val.view(torch.int32), val1.view(torch.int32))
+    return tok.cpu().numpy(), idx.cpu().numpy(), val.cpu().numpy()
+
+
 def test_last_position_logits_match_float64_product():
     import mllm_jax_amd as M
     dev = torch.device("cuda:0")
@@ -259,3 +275,20 @@ def test_masked_blocks_and_crowded_segments(v, k):
     np.testing.assert_array_equal(idx.cpu().numpy(), ri)
     np.testing.assert_array_equal(val.cpu().numpy().view(np.uint32), rv.view(np.uint32))
     np.testing.assert_array_equal(tok.cpu().numpy()[:10], rt[:10])       # what argmax makes of NaN scores is not at issue here
+
+
+@pytest.mark.filterwarnings("ignore:overflow encountered in divide")
+@pytest.mark.parametrize("v", [3000, 40000])
+@pytest.mark.parametrize("t,scale", [(2e-38, 1.0), (2e-38, 30.0), (3e38, 1e-3), (3e38, 1e-6), (1e20, 1e-25)])
+def test_quotients_that_overflow_or_lose_their_digits(v, t, scale):
+    """logits / t past the largest float (many equal +inf, lower index first) or among the denormals (logits far
+    apart share a quotient, or become zeros): the order is that of the quotients, not of the logits."""
+    rng = np.random.default_rng(v)
+    x = (scale * rng.normal(0, 2, size=(3, v))).astype(np.float32)
+    x[2] = -np.abs(x[2])
+    noise = rng.gumbel(size=(3, 50)).astype(np.float32)
+    tok, idx, val = _draw(noise, x, 50, t)
+    rt, ri, rv = O.top_k_sample(x, k=50, t=t, noise=noise)
+    np.testing.assert_array_equal(idx, ri)
+    np.testing.assert_array_equal(val.view(np.uint32), rv.view(np.uint32))
+    np.testing.assert_array_equal(tok, rt)
