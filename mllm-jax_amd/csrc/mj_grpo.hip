@@ -673,7 +673,6 @@ int mj_sample_top_k(const float* logits, int64_t ld_logits, int64_t b, int64_t v
 // ----------------------------------------------------------------------------- RMSNorm
 namespace {
 constexpr int kNormMaxH = 8192;
-bool norm_streams(int64_t n, int64_t h) { return n * h * 2 > (32ll << 20); }   // see mj_norm_kernels.hpp
 int norm_grid(int64_t n) {   // workgroups of the backward (one row at a time each, rows with this stride): four per CU
   return (int)(n < 1024 ? n : 1024);
 }

@@ -6,12 +6,11 @@
 // Both kernels are HBM-bound row reductions with 16-byte accesses: the forward gives a row to one
 // wavefront (reductions across lanes with shuffles, no LDS traffic), the backward to one workgroup.
 //
-// STREAM: a matrix is larger than the eight L2s together (32 MB), so that nothing of it is left there for the
-// kernel that comes next.  Then the accesses that are made once carry the non-temporal hint: y in the
-// forward, dy, x and dx in the backward.  They stop pushing each other's lines through the 256 MB
-// Infinity Cache.  Backward at 16384 x 3584, 352 MB: 73.5 -> 60 us right behind the forward; forward and
-// backward with the caches flushed in between: 168 -> 139 us, 67 -> 57 at 8000 x 2416, and with a reader of y
-// and a producer of dy in between 213 -> 193.  (A smaller matrix gains nothing, and its reader would miss it.)
+// STREAM (norm_streams, the plan's rule on the matrix's size): the accesses that are made once carry the
+// non-temporal hint -- y in the forward, dy, x and dx in the backward -- so that they do not push each other's
+// lines, and those of the kernels around, through the 256 MB Infinity Cache.  Where three matrices fit it the
+// hint only loses what would have been found there.  16384 x 4096, 128 MB: forward and backward 145 -> 127 us
+// one behind the other, 399 -> 386 with 1.3 GB of other traffic behind them (and that traffic's time).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

@@ -207,5 +207,16 @@ inline DrawSegments draw_segments(int64_t b, int64_t vocab) {
   return g;
 }
 
+// RMSNorm: whether a matrix's single-use accesses carry the non-temporal hint (mj_norm_kernels.hpp).  From 100 MB
+// on: x, dy and dx together are then past the 256 MB Infinity Cache, and what they push out of it costs more than
+// finding a matrix there saves.  Kernels of a forward and a backward, us, with the hint and without, inputs in the
+// caches / after 1.3 GB of other traffic (that traffic's own time included, as it pays for what is left dirty):
+//   38.5 MB (8000 x 2416)  48.3, 44.0 /   -    54.7 MB (8000 x 3584)   63.2, 56.2 /   -
+//   82 MB (12000 x 3584)   88.3, 83.4 / 344, 345     96 MB (14000 x 3584)   97.9, 95.6 / 356, 360
+//   102.5 MB (15000 x 3584)  102.9, 107.2 / 360, 370   112 MB (16384 x 3584)  113.9, 116.9 / 371, 381
+// With a reader of y and a producer of dy in between the sum of all of them differs by less than 1 % either way:
+// the hint costs the backward 8 us at 54.7 and 112 MB and the copies around it gain as much.
+inline bool norm_streams(int64_t n, int64_t h) { return n * h * 2 > (100ll << 20); }
+
 }  // namespace host
 }  // namespace mj

@@ -6,7 +6,8 @@
 //   * make_plan: workspace regions are 256-byte aligned, do not overlap, end inside the totals;
 //     the vocab splits of the d_hidden product cover V; chunks cover N;
 //   * the no-alloc chunk search returns the largest chunk that fits, or refuses;
-//   * the sampler's work items cover the vocabulary, and so do the segments of the draw.
+//   * the sampler's work items cover the vocabulary, and so do the segments of the draw;
+//   * RMSNorm streams only matrices that the Infinity Cache cannot hold.
 // Prints "ok <checks>" and exits 0, or a message and exits 1.
 #include <algorithm>
 #include <cstdio>
@@ -267,8 +268,19 @@ static void draw_sweep() {
   }
 }
 
+// RMSNorm's non-temporal form: only where x, dy and dx together are past the Infinity Cache (256 MB); a matrix that
+// is found there loses by it.
+static void norm_sweep() {
+  for (int64_t h = 8; h <= 8192; h += 8)
+    for (int64_t n : {1, 64, 4100, 4700, 8000, 12000, 16384, 1 << 20}) {
+      if (n * h * 6 <= 256ll << 20) CHECK(!norm_streams(n, h), "%lld x %lld streams", (long long)n, (long long)h);
+      if (n * h * 6 >= 320ll << 20) CHECK(norm_streams(n, h), "%lld x %lld does not stream", (long long)n, (long long)h);
+    }
+}
+
 int main() {
   draw_sweep();
+  norm_sweep();
   tile_map_sweep();
   plan_sweep();
   noalloc_sweep();

@@ -95,10 +95,11 @@ def test_norm_feeds_the_fused_loss_end_to_end():
     assert _rel(wd.grad.float().cpu().numpy(), ref["d_lm_head"]) <= 2e-2
 
 
-@pytest.mark.parametrize("n,h", [(8193, 2048), (4099, 4096), (2051, 8192), (4667, 3600)])
+@pytest.mark.parametrize("n,h", [(8193, 2048), (4099, 4096), (2051, 8192), (4667, 3600),           # larger than the L2s
+                                 (25601, 2048), (12801, 4096), (6401, 8192), (14565, 3600)])        # just past 100 MB: streaming
 def test_matrices_larger_than_the_l2s_stream(n, h):
-    """Just past 32 MB the accesses carry the non-temporal hint: rows are those of a small call bit for
-    bit (a row's arithmetic does not depend on the matrix), dscale is the float64 column sum."""
+    """Past 100 MB the accesses carry the non-temporal hint, in each instantiation: rows are those of a small
+    call bit for bit (a row's arithmetic does not depend on the matrix), dscale is the float64 column sum."""
     import mllm_jax_amd as M
     dev = torch.device("cuda:0")
     g = torch.Generator(device=dev).manual_seed(h)
