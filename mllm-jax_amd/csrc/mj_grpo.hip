@@ -181,8 +181,8 @@ int run(Mode mode, const MjGrpoDesc* d, const void* hidden, const void* lm_head,
     mj::k_sum<<<1, 1024, 0, st>>>(vterm, N, pv->value_loss);
     mj::k_sum<<<1, 1024, 0, st>>>(dvw, N, pv->d_value_b);
     const int vblocks = (N + mj::kValueRows - 1) / mj::kValueRows;
-    mj::k_value_wgrad<<<vblocks, 256, 0, st>>>((const uint16_t*)hidden, d->ld_hidden, N, H, dvw, vpart);
-    mj::k_value_wgrad_reduce<<<(unsigned)((H + 255) / 256), 256, 0, st>>>(vpart, vblocks, H, pv->d_value_w);
+    mj::k_value_wgrad<<<dim3(vblocks, (H + 511) / 512), 256, 0, st>>>((const uint16_t*)hidden, d->ld_hidden, N, H, dvw, vpart);
+    mj::k_value_wgrad_reduce<<<(unsigned)((H + mj::kValueCols - 1) / mj::kValueCols), 256, 0, st>>>(vpart, vblocks, H, pv->d_value_w);
     if ((rc = check_launch("value head kernels"))) return rc;
     dv = dvw;
   }

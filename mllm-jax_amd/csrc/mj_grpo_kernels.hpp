@@ -1181,17 +1181,22 @@ __global__ __launch_bounds__(1024) void k_sum(const float* x, int n, float* out)
   if (threadIdx.x == 0) out[0] = sh[0];
 }
 
-// d_wv[c] = sum_t dv[t] * hidden[t, c]: a workgroup adds up kValueRows rows (8 columns per thread,
-// rows in order), k_value_wgrad_reduce adds the workgroups' partial rows in fixed order.
-// Both are chains of dependent additions behind loads, far from any rate of the chip: short chains in many
-// workgroups, and the loads of eight steps in flight.  2048 x 1536: 21.2 -> 7.1 us and 9.2 -> 4.9 (64 rows each, one
-// load at a time, before).
-constexpr int kValueRows = 16;
+// d_wv[c] = sum_t dv[t] * hidden[t, c], in fixed order.  Both kernels are chains of dependent additions behind
+// loads, far from any rate of the chip, and a long chain in float32 also adds up its roundings.  So: kValueRows rows
+// and 512 columns per workgroup, sixteen rows per wavefront (8 columns per lane, eight loads in flight) added in pairs
+// through LDS; then, sixteen columns per workgroup, a sixteenth of the partial rows per thread, added in pairs again.
+// Up to 16384 tokens no sum is longer than 16 before it is paired.  Both kernels together, us, with one chain of
+// 64 rows and one of all partial rows per column / chains of 16 rows / now: 2048 x 1536 30 / 11.7 / 9.6,
+// 8192 x 3584 71 / 30 / 15, 16384 x 1536 85 / 39 / 13; error at 16384 tokens 4.3, 9.4 and below 4 times 2^-24.
+constexpr int kValueRows = 64;
 __global__ __launch_bounds__(256) void k_value_wgrad(const uint16_t* hid, int64_t ld_hid, int n, int H,
                                                      const float* dv, float* part) {
-  const int r0 = blockIdx.x * kValueRows, r1 = min(r0 + kValueRows, n);
-  for (int c = threadIdx.x * 8; c < H; c += 2048) {
-    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  __shared__ __attribute__((aligned(16))) float sums[4][512];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int r0 = blockIdx.x * kValueRows + wave * (kValueRows / 4), r1 = min(r0 + kValueRows / 4, n);
+  const int c = blockIdx.y * 512 + lane * 8;
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (c < H) {                                   // H % 8 == 0
 #pragma unroll 8
     for (int r = r0; r < r1; ++r) {
       const float d = dv[r];
@@ -1202,19 +1207,34 @@ __global__ __launch_bounds__(256) void k_value_wgrad(const uint16_t* hid, int64_
         acc[2 * j + 1] = fmaf(d, __uint_as_float(v[j] & 0xffff0000u), acc[2 * j + 1]);
       }
     }
-    float* o = part + (int64_t)blockIdx.x * H + c;
-    *(f32x4*)o = f32x4{acc[0], acc[1], acc[2], acc[3]};
-    *(f32x4*)(o + 4) = f32x4{acc[4], acc[5], acc[6], acc[7]};
+  }
+  *(f32x4*)&sums[wave][lane * 8] = f32x4{acc[0], acc[1], acc[2], acc[3]};
+  *(f32x4*)&sums[wave][lane * 8 + 4] = f32x4{acc[4], acc[5], acc[6], acc[7]};
+  __syncthreads();
+#pragma unroll
+  for (int i = threadIdx.x; i < 512; i += 256) {
+    const int col = blockIdx.y * 512 + i;
+    if (col < H) part[(int64_t)blockIdx.x * H + col] = (sums[0][i] + sums[1][i]) + (sums[2][i] + sums[3][i]);
   }
 }
 
+constexpr int kValueCols = 16;                   // columns per workgroup of the reduction
 __global__ __launch_bounds__(256) void k_value_wgrad_reduce(const float* part, int blocks, int H, float* d_wv) {
-  const int c = blockIdx.x * 256 + threadIdx.x;
-  if (c >= H) return;
+  __shared__ float sums[16][kValueCols];
+  const int i = threadIdx.x % kValueCols, slice = threadIdx.x / kValueCols;
+  const int c = blockIdx.x * kValueCols + i;
+  const int per = (blocks + 15) / 16, b0 = slice * per, b1 = min(b0 + per, blocks);
   float a = 0.f;
-#pragma unroll 16
-  for (int b = 0; b < blocks; ++b) a += part[(int64_t)b * H + c];
-  d_wv[c] = a;
+  if (c < H) {
+#pragma unroll 8
+    for (int b = b0; b < b1; ++b) a += part[(int64_t)b * H + c];
+  }
+  sums[slice][i] = a;
+  for (int o = 1; o < 16; o <<= 1) {
+    __syncthreads();
+    if (slice % (2 * o) == 0) sums[slice][i] += sums[slice + o][i];
+  }
+  if (slice == 0 && c < H) d_wv[c] = sums[0][i];
 }
 
 // ----------------------------------------------------------------------------- compaction

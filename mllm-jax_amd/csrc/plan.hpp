@@ -26,7 +26,7 @@ inline int fail(int code, const char* fmt, ...) {
   return code;
 }
 
-constexpr int kValueRows = 16;             // token rows per workgroup of the value head's weight gradient
+constexpr int kValueRows = 64;             // token rows per workgroup of the value head's weight gradient
 constexpr int BM = 256, BN = 256;          // tile of all three contractions
 constexpr int64_t kDefaultChunk = 16384;   // tokens whose logits live in the workspace at once
 constexpr int kRescueGrid = 256;           // workgroups of the rescue pass (one per CU)

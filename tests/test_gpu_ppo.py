@@ -261,3 +261,31 @@ def test_value_head_with_the_rescue_pass():
     assert _rel(hd.grad[:, :-1].reshape(b * t, h).float().cpu().numpy(), ref["d_hidden"]) <= GRAD_RTOL
     assert _rel(wd.grad.float().cpu().numpy(), ref["d_lm_head"]) <= GRAD_RTOL
     assert _rel(wvd.grad.cpu().numpy(), ref["d_value_w"]) <= GRAD_RTOL
+
+
+@pytest.mark.parametrize("tokens,h", [(1, 8), (63, 24), (65, 504), (1025, 520), (16384, 1032)])
+def test_value_weight_gradient_keeps_float32_accuracy(tokens, h):
+    """Rows either side of a wavefront's sixteen, a workgroup's 64 and the reduction's 16 x 64; columns either side
+    of a workgroup's 512.  The reference is the float64 sum of the same products.  A float32 chain of L random terms
+    errs by 2^-24 sqrt(L / 6) of its sum; chains of at most 16, four pairings and a product of three roundings come to
+    about 3 * 2^-24, where one chain of 1024 partial sums alone takes 13."""
+    import mllm_jax_amd as M
+    dev = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(tokens + h)
+    hid = torch.randn(1, tokens + 1, h, generator=g).to(torch.bfloat16)
+    w = (0.1 * torch.randn(h, 64, generator=g)).to(torch.bfloat16)
+    wv = torch.zeros(h)                                   # value predictions exactly 0: dv is -2 R coef / count
+    ret = torch.randn(1, tokens, generator=g)
+    ids = torch.randint(0, 64, (1, tokens + 1), generator=g)
+    labels = torch.ones(1, tokens + 1, dtype=torch.long)
+    wv_dev = wv.to(dev).requires_grad_()
+    hid_dev = hid.to(dev).requires_grad_()
+    module = M.PPOActorCriticModule(lambda input_ids, attention_mask: hid_dev, w.to(dev).requires_grad_(),
+                                    (wv_dev, torch.zeros((), device=dev).requires_grad_()), value_coef=0.5)
+    out = module({"input_ids": ids.to(dev), "attention_mask": labels.to(dev), "labels": labels.to(dev), "returns": ret.to(dev),
+                  "advantages": torch.zeros(1, tokens, device=dev), "total_valid_token_count": float(tokens)})
+    out["loss"].backward()
+    dv = -ret[0].double() / tokens
+    ref = (dv[:, None] * hid[0, :tokens].double()).sum(0)
+    err = float((wv_dev.grad.double().cpu() - ref).norm() / ref.norm())
+    assert err <= 4 * 2.0 ** -24, err
