@@ -216,7 +216,8 @@ int mj_grpo_backward(const MjGrpoDesc* desc, const void* hidden, const void* lm_
  *   MJ_GRPO_ADV_RLOO    r - mean of the others in the group (group mean for singletons); whiten != 0
  *                       then centres and scales over the batch            estimators.py:58-103, :137-157
  *   MJ_GRPO_ADV_DAPO    GRPO + alpha * GLOBAL                             estimators.py:106-134
- * clip_range > 0 clips the result to [-clip_range, clip_range] (estimators.py:28-34). */
+ * clip_range > 0 clips the result to [-clip_range, clip_range] (estimators.py:28-34).
+ * MJ_GRPO_ADV_GLOBAL may be computed in place (advantages == rewards); otherwise the two do not overlap. */
 enum { MJ_GRPO_ADV_GRPO = 0, MJ_GRPO_ADV_GLOBAL = 1, MJ_GRPO_ADV_RLOO = 2, MJ_GRPO_ADV_DAPO = 3 };
 int mj_grpo_advantages(int mode, const float* rewards, const int32_t* group_ids, float* advantages,
                        int64_t b, float eps, float alpha, int whiten, float clip_range, void* stream);

@@ -543,6 +543,10 @@ int mj_grpo_advantages(int mode, const float* rewards, const int32_t* group_ids,
   const bool whitened = mode == mj::kAdvRloo && whiten != 0;
   a.rewards = rewards; a.group_ids = group_ids; a.adv = advantages; a.b = (int)b; a.mode = mode;
   a.eps = eps; a.alpha = alpha; a.clip = whitened ? 0.f : clip_range;
+  if (mode == mj::kAdvGlobal && rewards == advantages) {     // many workgroups would write what others still read
+    mj::k_whiten<<<1, 1024, 0, (hipStream_t)stream>>>(advantages, (int)b, eps, clip_range);
+    return check_launch("k_whiten");
+  }
   const int per = mode == mj::kAdvGlobal ? mj::kAdvThreads : mj::kAdvThreads / mj::kAdvLanes;   // samples per workgroup
   mj::k_advantages<<<(unsigned)((b + per - 1) / per), mj::kAdvThreads, 0, (hipStream_t)stream>>>(a);
   if (whitened) mj::k_whiten<<<1, 1024, 0, (hipStream_t)stream>>>(advantages, (int)b, eps, clip_range);

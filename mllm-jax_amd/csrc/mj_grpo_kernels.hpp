@@ -1187,7 +1187,7 @@ __global__ __launch_bounds__(1024) void k_sum(const float* x, int n, float* out)
 // through LDS; then, sixteen columns per workgroup, a sixteenth of the partial rows per thread, added in pairs again.
 // Up to 16384 tokens no sum is longer than 16 before it is paired.  Both kernels together, us, with one chain of
 // 64 rows and one of all partial rows per column / chains of 16 rows / now: 2048 x 1536 30 / 11.7 / 9.6,
-// 8192 x 3584 71 / 30 / 15, 16384 x 1536 85 / 39 / 13; error at 16384 tokens 4.3, 9.4 and below 4 times 2^-24.
+// 8192 x 3584 71 / 30 / 15, 16384 x 1536 85 / 39 / 13; error at 16384 tokens 5.6, 9.4 and 2.0 times 2^-24.
 constexpr int kValueRows = 64;
 __global__ __launch_bounds__(256) void k_value_wgrad(const uint16_t* hid, int64_t ld_hid, int n, int H,
                                                      const float* dv, float* part) {
@@ -2179,7 +2179,8 @@ __global__ __launch_bounds__(kAdvThreads) void k_advantages(AdvArgs p) {
   if (lane == 0 && sample < p.b) finish(sample, out);
 }
 
-// estimators.py:99-102: the whole batch of leave-one-out advantages centred and scaled, in place; one workgroup
+// The whole batch centred and scaled, in place: leave-one-out advantages (estimators.py:99-102), or rewards that
+// become their global advantages (:52-55).  One workgroup, which has read everything before it writes.
 __global__ __launch_bounds__(1024) void k_whiten(float* adv, int b, float eps, float clip) {
   __shared__ double sh[16];
   float m, sd;

@@ -132,3 +132,15 @@ def test_batches_across_workgroups(b):
                                    O.rloo_advantages(r, gid, whiten=b > 16, clip_range=1.0), **kw)
         np.testing.assert_allclose(M.compute_dapo_advantages_by_group_id(rewards=_d(r), group_ids=_d(gid), clip_range=0.9).cpu().numpy(),
                                    O.dapo_advantages(r, gid, clip_range=0.9), **kw)
+
+
+@pytest.mark.parametrize("b", [1, 200, 256, 257, 1024, 5000, 65536])
+def test_global_advantages_in_place(b):
+    """advantages == rewards, up to the largest batch: what the call gives for separate buffers."""
+    from mllm_jax_amd import _lib
+    rng = np.random.default_rng(b)
+    r = (3.0 + rng.standard_normal(b)).astype(np.float32)
+    x = _d(r)
+    _lib.check(_lib.load().mj_grpo_advantages(1, x.data_ptr(), None, x.data_ptr(), b, 1e-4, 0.0, 0, 1.5,
+                                              torch.cuda.current_stream().cuda_stream))
+    np.testing.assert_allclose(x.cpu().numpy(), O.global_normalized_advantages(r, eps=1e-4, clip_range=1.5), rtol=1e-5, atol=1e-5)
