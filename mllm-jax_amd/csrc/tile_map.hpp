@@ -18,13 +18,15 @@ namespace mj {
 // other, so any 32 consecutive tiles are a block of about 2^lgm x 2^lgn that shares its operand slices
 // in an L2.  The k-splits follow each other in the same list.  Groups of 32 consecutive items go to
 // the eight XCDs in turn (ids congruent mod 8 run on the same XCD): an XCD works on one such block at
-// a time, the eight XCDs on eight neighbouring ones.
+// a time, the eight XCDs on eight neighbouring ones.  Of the last, partial round each XCD gets an
+// eighth: in lots of 32 its tiles would be work for a few XCDs (dW of 512 x 896 x 151936, 2376 tiles: 72 left over,
+// on three XCDs 235.5 us, on all eight 232; a whole pass of 256 x 896 468 -> 452, larger ones the same).
 //
 // The list holds real tiles only and the strips of a grid differ by at most one in width, which
 // is what keeps the XCDs equally loaded: with fixed 4 x 8 blocks and the empty slots of ragged ones as
 // ids of their own, a grid of 9 tile columns walked along N gave every second block one live column out
-// of eight, all of those on the same four XCDs (2049 tokens x 4096 x 128256: logits 2.95 ms against
-// 2.11 ms in this order).
+// of eight, all of those on the same four XCDs (2049 tokens x 4096 x 128256: logits 2.9 ms against
+// 1.85 ms in this order).
 struct TileMap {
   int tiles_m, tiles_n, n_first, lgm, lgn, lgs, splits;
   int width, wide;         // strips: the first `wide` ones are width + 1 tiles across, the others `width`
@@ -39,9 +41,14 @@ struct TileMap {
   MJ_HD int tiles() const { return tiles_m * tiles_n * splits; }
   MJ_HD int items() const { return (tiles() + 255) & ~255; }
   MJ_HD bool tile(int pid, int& tm, int& tn, int& split) const {
-    const int q = pid >> 3;
-    int at = (((q >> 5) * 8 + (pid & 7)) << 5) + (q & 31);      // place in the list of tiles
-    if (at >= tiles()) return false;
+    const int q = pid >> 3, xcd = pid & 7, round = q >> 5, within = q & 31;
+    int at = (round << 8) + xcd * 32 + within;                  // place in the list of tiles
+    const int left = tiles() - (round << 8);
+    if (left < 256) {                                           // the last round: an eighth each
+      const int each = left > 0 ? left >> 3 : 0, more = left > 0 ? left & 7 : 0;
+      if (within >= each + (xcd < more ? 1 : 0)) return false;
+      at = (round << 8) + xcd * each + (xcd < more ? xcd : more) + within;
+    }
     const int per = tiles_m * tiles_n, along = n_first ? tiles_n : tiles_m;
     split = at / per;
     at -= split * per;

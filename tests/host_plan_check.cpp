@@ -38,10 +38,11 @@ static void check_bijection(const TileMap& m, const char* what) {
   std::vector<unsigned char> seen((size_t)tm * tn * sp, 0);
   const int items = m.items();
   CHECK(items % 256 == 0 && items >= 0, "%s: items %d", what, items);
-  long hits = 0;
+  long hits = 0, load[8] = {0};      // tiles per XCD
   for (int id = 0; id < items; ++id) {
     int a = -1, b = -1, s = -1;
     if (!m.tile(id, a, b, s)) continue;
+    ++load[id & 7];
     CHECK(a >= 0 && a < tm && b >= 0 && b < tn && s >= 0 && s < sp, "%s: id %d -> (%d, %d, %d) outside %d x %d x %d",
           what, id, a, b, s, tm, tn, sp);
     unsigned char& cell = seen[((size_t)s * tm + a) * tn + b];
@@ -51,6 +52,8 @@ static void check_bijection(const TileMap& m, const char* what) {
   }
   CHECK(hits == (long)tm * tn * sp, "%s: %ld of %ld tiles produced (tm %d tn %d splits %d lgm %d lgs %d n_first %d)",
         what, hits, (long)tm * tn * sp, tm, tn, sp, m.lgm, m.lgs, m.n_first);
+  const long most = *std::max_element(load, load + 8), least = *std::min_element(load, load + 8);
+  CHECK(most - least <= 1, "%s: %ld tiles on one XCD, %ld on another", what, most, least);
   // ids past the end never yield a tile
   for (int id = items; id < items + 512; ++id) {
     int a, b, s;
