@@ -236,7 +236,7 @@ int run(Mode mode, const MjGrpoDesc* d, const void* hidden, const void* lm_head,
     a.pm = pm; a.pl = pl; a.ps = ps; a.plt = plt; a.inv_t = inv_t; a.ld_p = p.n_pad;
     a.targets = targets + c0; a.zy = zy + c0; a.n_live = n_live; a.c0 = (int)c0;
     a.mask = mask + c0; a.lse = nullptr; a.g = g; a.state = state;
-    const mj::TileMap map = mj::TileMap::pick_shape((V + BM - 1) / BM, (nc + BN - 1) / BN, 1, 1);
+    const mj::TileMap map((V + BM - 1) / BM, (nc + BN - 1) / BN, 1, 1);
 
     mj::FinalizeArgs f;
     f.pm = pm; f.pl = pl; f.ps = ps; f.plt = plt; f.inv_t = inv_t; f.ld_p = p.n_pad; f.parts = (int)p.parts;
@@ -314,7 +314,7 @@ int run(Mode mode, const MjGrpoDesc* d, const void* hidden, const void* lm_head,
       h.dh = (uint16_t*)d_hidden + c0 * ld_dh; h.ld_dh = ld_dh;
       h.part = part; h.n_live = n_live; h.c0 = (int)c0; h.rs = rs; h.state = state;
       h.dv = dv ? dv + c0 : nullptr; h.wv = pv ? pv->value_w : nullptr; h.dead = dead;
-      const mj::TileMap mh = mj::TileMap::pick_shape((nc + BM - 1) / BM, (H + BN - 1) / BN, 0, h.splits);
+      const mj::TileMap mh((nc + BM - 1) / BM, (H + BN - 1) / BN, 0, h.splits);
       {
         Timed t(MJ_GRPO_K_DHIDDEN, st);
         mj::k_dhidden<BM, BN><<<mh.items(), mj::kThreads, lds, st>>>(h, mh);
@@ -338,7 +338,7 @@ int run(Mode mode, const MjGrpoDesc* d, const void* hidden, const void* lm_head,
       w.H = H; w.V = V; w.n = nc;
       w.dw = d_w; w.ld_dw = d->ld_w; w.n_live = n_live; w.c0 = (int)c0; w.dead = dead;
       w.accumulate = (c0 > 0 || (d->flags & MJ_GRPO_FLAG_DW_ACCUMULATE)) ? 1 : 0;
-      const mj::TileMap mw = mj::TileMap::pick_shape((V + BM - 1) / BM, (H + BN - 1) / BN, 0, 1);
+      const mj::TileMap mw((V + BM - 1) / BM, (H + BN - 1) / BN, 0, 1);
       {
         Timed t(MJ_GRPO_K_DW, st);
         if (dw_bf16) mj::k_dw<BM, BN, true><<<mw.items(), mj::kThreads, lds, st>>>(w, mw);
@@ -601,7 +601,6 @@ int mj_sample_logits(const void* hidden, int64_t ld_hidden, const void* lm_head,
   // 60 us at the first shape, but 219 against 207 at 3584 x 152064 and 24 against 18 at the last).
   if (b <= 2) {
     const unsigned grid = (unsigned)((vocab + 255) / 256);
-    a.units = a.items = 0;
     if (b == 1) mj::k_logits_few<1><<<grid, 64 * mj::kFewWaves, 0, st>>>(a);
     else mj::k_logits_few<2><<<grid, 64 * mj::kFewWaves, 0, st>>>(a);
     return check_launch("k_logits_few");
@@ -613,10 +612,8 @@ int mj_sample_logits(const void* hidden, int64_t ld_hidden, const void* lm_head,
   int bn;
   int64_t tiles_n, tile_rows;
   sample_tiles(b, vocab, &bn, &tiles_n, &tile_rows);
-  a.units = (int)((vocab + mj::kRowUnit - 1) / mj::kRowUnit);
-  a.items = (int)((vocab + tile_rows - 1) / tile_rows);
-  if (a.items > a.units) a.items = a.units;
-  const mj::TileMap map = mj::TileMap::pick_shape(a.items, (int)tiles_n, 1, 1);
+  a.cols = mj::RowItems((int)vocab, (int)((vocab + tile_rows - 1) / tile_rows));
+  const mj::TileMap map(a.cols.items, (int)tiles_n, 1, 1);
   if (bn == 128) {
     if ((rc = enable_lds(mj::k_logits_rows<BM, 128>))) return rc;
     mj::k_logits_rows<BM, 128><<<map.items(), mj::kThreads, mj::GemmTN<BM, 128>::kLdsBytes, st>>>(a, map);

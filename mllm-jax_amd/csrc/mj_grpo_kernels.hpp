@@ -184,16 +184,15 @@ MJ_DEV void logits_tile_grad(const LogitsArgs& p, int tm, int tn, char* smem, in
 #pragma unroll
         for (int r = 0; r < 16; ++r) big = fmaxf(big, fabsf(g.acc[mi][ni][r]));
       if (__all(big * inv_cap <= 0.25f)) {
-        // z P(z^2),  P(w) = k (1 - w / (3 c^2) + 2 w^2 / (15 c^4) - 17 w^3 / (315 c^6)),  k = log2(e) or 1
-        const float k0 = 1.f;
-        const float c1 = k0 * (-1.f / 3.f) * inv_cap2, c2 = k0 * (2.f / 15.f) * inv_cap2 * inv_cap2;
-        const float c3 = k0 * (-17.f / 315.f) * inv_cap2 * inv_cap2 * inv_cap2;
+        // z P(z^2),  P(w) = 1 - w / (3 c^2) + 2 w^2 / (15 c^4) - 17 w^3 / (315 c^6)
+        const float c1 = (-1.f / 3.f) * inv_cap2, c2 = (2.f / 15.f) * inv_cap2 * inv_cap2;
+        const float c3 = (-17.f / 315.f) * inv_cap2 * inv_cap2 * inv_cap2;
 #pragma unroll
         for (int mi = 0; mi < G::MI; ++mi)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             const float z = g.acc[mi][ni][r], w = z * z;
-            g.acc[mi][ni][r] = z * fmaf(w, fmaf(w, fmaf(w, c3, c2), c1), k0);
+            g.acc[mi][ni][r] = z * fmaf(w, fmaf(w, fmaf(w, c3, c2), c1), 1.f);
           }
       } else {
 #pragma unroll
@@ -345,7 +344,7 @@ MJ_DEV void logits_tile16(const LogitsArgs& p, int tm, int tn, char* smem, int t
 #pragma unroll
   for (int ni = 0; ni < G::NI; ++ni) {
     const int col = t0 + ni * 16 + l15;
-    // softcap: see logits_tile (series while every logit of the wavefront's block column is small
+    // softcap: see logits_tile_grad (series while every logit of the wavefront's block column is small
     // against the cap; the capped logit is kept in units of log2)
     if (CAP) {
       float big = 0.f;
@@ -862,7 +861,7 @@ template <int BM, int BN>
 __global__ __launch_bounds__(kThreads) void k_dhidden(DhArgs p, TileMap map) {
   using G = GemmTN16<BM, BN, kRowK, kRowK, true, false>;   // rows of dead tokens are not fetched
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  const TileMap live(live_pad(p.n_live, p.c0, p.n_pad) / BM, map.tiles_n, map.n_first, map.lgm, map.splits, map.lgs);
+  const TileMap live(live_pad(p.n_live, p.c0, p.n_pad) / BM, map.tiles_n, map.n_first, map.splits);
   int tm, tn, split;
   if (!live.tile(blockIdx.x, tm, tn, split)) return;
   const int m0 = tm * BM, n0 = tn * BN;
@@ -1326,7 +1325,7 @@ struct LogitsRowsArgs {
   float cap;             // final-logit softcap, 0 = off
   float* out;            // [n, ld_out]
   int64_t ld_out;
-  int units, items;      // the vocabulary in units of kRowUnit columns, spread evenly over `items` work items
+  RowItems cols;         // which columns a work item has (k_logits_rows)
 };
 
 // A decode batch is a few rows against the whole vocabulary matrix: the product is bound by reading
@@ -1337,16 +1336,13 @@ struct LogitsRowsArgs {
 // a k-row is 400 bytes or so out of 300 KB, and a piece that starts in the middle of a 64-byte sector is
 // fetched with the neighbour's bytes around it (128 x 3584 x 152064 in 200-column items: 253 us; in items
 // of 192 and 224 columns: 245).
-constexpr int kRowUnit = 32;
 template <int BM, int BN>
 __global__ __launch_bounds__(kThreads) void k_logits_rows(LogitsRowsArgs p, TileMap map) {
   using G = GemmTN<BM, BN, kKRow, kRowK, (BN < 256 ? 2 : 1)>;   // the narrow tiles wait on memory: three slices in flight
   extern __shared__ __attribute__((aligned(16))) char smem[];
   int tm, tn, split;
   if (!map.tile(blockIdx.x, tm, tn, split)) return;
-  const int base = p.units / p.items, wide = p.units - base * p.items;      // the first `wide` items take one unit more
-  const int m0 = (tm * base + min(tm, wide)) * kRowUnit, n0 = tn * BN;
-  const int m1 = min(p.V, m0 + (base + (tm < wide ? 1 : 0)) * kRowUnit);
+  const int m0 = p.cols.first(tm), m1 = min(p.V, p.cols.first(tm + 1)), n0 = tn * BN;
   G g;
   g.run(p.w + m0, m1 - m0, p.ld_w, p.hid + (int64_t)n0 * p.ld_hid, p.n - n0, p.ld_hid, p.H, smem);
   const int lane = threadIdx.x & 63;

@@ -13,10 +13,11 @@
 namespace mj {
 
 // Maps a linear work-item id to a tile (and a k-split).  The tiles of one k-split are put in a row: the
-// grid of tiles is cut into strips -- 2^lgm tile rows each, walked along N (n_first), or 2^lgn tile
-// columns each, walked along M -- and inside a strip the tiles that lie across it come one after the
-// other, so any 32 consecutive tiles are a block of about 2^lgm x 2^lgn that shares its operand slices
-// in an L2.  The k-splits follow each other in the same list.  Groups of 32 consecutive items go to
+// grid of tiles is cut into strips -- at most kTall tile rows each, walked along N (n_first), or at most kLong
+// tile columns each, walked along M -- and inside a strip the tiles that lie across it come one after the
+// other, so any 32 consecutive tiles are a block of about 4 x 8 (the shape with the fewest operand panels)
+// that shares its operand slices in an L2.  The k-splits follow each other in the same list; where one has fewer
+// than 32 tiles, a group spans several.  Groups of 32 consecutive items go to
 // the eight XCDs in turn (ids congruent mod 8 run on the same XCD): an XCD works on one such block at
 // a time, the eight XCDs on eight neighbouring ones.  Of the last, partial round each XCD gets an
 // eighth: in lots of 32 its tiles would be work for a few XCDs (dW of 512 x 896 x 151936, 2376 tiles: 72 left over,
@@ -28,13 +29,13 @@ namespace mj {
 // of eight, all of those on the same four XCDs (2049 tokens x 4096 x 128256: logits 2.9 ms against
 // 1.85 ms in this order).
 struct TileMap {
-  int tiles_m, tiles_n, n_first, lgm, lgn, lgs, splits;
+  static constexpr int kTall = 4, kLong = 8;
+  int tiles_m, tiles_n, n_first, splits;
   int width, wide;         // strips: the first `wide` ones are width + 1 tiles across, the others `width`
-  // lgs: 2^lgs k-splits of 2^lgm x 2^lgn tiles make a group of 32 (strips are narrower by that much)
-  MJ_HD TileMap(int tm, int tn, int n_first_ = 0, int lgm_ = 2, int splits_ = 1, int lgs_ = 0)
-      : tiles_m(tm), tiles_n(tn), n_first(n_first_), lgm(lgm_), lgn(5 - lgm_ - lgs_), lgs(lgs_), splits(splits_) {
-    const int across = n_first ? tm : tn, lg = n_first ? lgm : lgn;
-    const int strips = across > 0 ? (across + (1 << lg) - 1) >> lg : 1;
+  MJ_HD TileMap(int tm, int tn, int n_first_, int splits_)
+      : tiles_m(tm), tiles_n(tn), n_first(n_first_), splits(splits_) {
+    const int across = n_first ? tm : tn, most = n_first ? kTall : kLong;
+    const int strips = across > 0 ? (across + most - 1) / most : 1;
     width = across / strips;
     wide = across - width * strips;
   }
@@ -68,9 +69,18 @@ struct TileMap {
     tn = n_first ? step : x;
     return true;
   }
-  // The shape with the fewest operand panels per group: 4 x 8 tiles of one k-split.  (Where a split has
-  // fewer than 32 tiles, a group spans several splits by itself.)
-  static TileMap pick_shape(int tm, int tn, int n_first, int splits) { return TileMap(tm, tn, n_first, 2, splits, 0); }
+};
+
+// The columns of the sampler's logits product: whole units of kRowUnit, spread evenly over the work items (the
+// first ones take one unit more where it does not come out even).
+constexpr int kRowUnit = 32;
+struct RowItems {
+  int units, items;
+  MJ_HD RowItems(int vocab = 0, int items_ = 0) : units((vocab + kRowUnit - 1) / kRowUnit), items(items_ < units ? items_ : units) {}
+  MJ_HD int first(int item) const {       // first column of the item; the last item ends at the vocabulary's end
+    const int base = units / items, wide = units - base * items;
+    return (item * base + (item < wide ? item : wide)) * kRowUnit;
+  }
 };
 
 }  // namespace mj

@@ -1,7 +1,7 @@
 // host_plan_check.cpp -- CPU checks of the host-side index arithmetic of the tile kernels, built by
 // tests/test_host_plan_cpu.py with g++ -fsanitize=address,undefined (no HIP, no GPU):
 //   * TileMap: over ids 0 .. items()-1, tile() yields every (tile row, tile column, k-split) of the
-//     problem exactly once and nothing outside it, for every block shape and walk order;
+//     problem exactly once and nothing outside it, in both walk orders, and no XCD gets more than one tile more than another;
 //   * the same for the "live rows" rebuild that k_dhidden makes from a device-side token count;
 //   * make_plan: workspace regions are 256-byte aligned, do not overlap, end inside the totals;
 //     the vocab splits of the d_hidden product cover V; chunks cover N;
@@ -50,8 +50,8 @@ static void check_bijection(const TileMap& m, const char* what) {
     cell = 1;
     ++hits;
   }
-  CHECK(hits == (long)tm * tn * sp, "%s: %ld of %ld tiles produced (tm %d tn %d splits %d lgm %d lgs %d n_first %d)",
-        what, hits, (long)tm * tn * sp, tm, tn, sp, m.lgm, m.lgs, m.n_first);
+  CHECK(hits == (long)tm * tn * sp, "%s: %ld of %ld tiles produced (tm %d tn %d splits %d n_first %d)",
+        what, hits, (long)tm * tn * sp, tm, tn, sp, m.n_first);
   const long most = *std::max_element(load, load + 8), least = *std::min_element(load, load + 8);
   CHECK(most - least <= 1, "%s: %ld tiles on one XCD, %ld on another", what, most, least);
   // ids past the end never yield a tile
@@ -69,19 +69,14 @@ static void tile_map_sweep() {
       if ((long)tm * tn > 20000) continue;
       for (int sp : splits)
         for (int nf = 0; nf < 2; ++nf) {
-          if ((long)tm * tn * sp <= 30000)
-            for (int ls = 0; ls <= 5; ++ls)
-              for (int lm = 0; lm + ls <= 5; ++lm) check_bijection(TileMap(tm, tn, nf, lm, sp, ls), "explicit shape");
-          const TileMap picked = TileMap::pick_shape(tm, tn, nf, sp);
-          CHECK(picked.lgm + picked.lgn + picked.lgs == 5 && picked.lgm >= 0 && picked.lgn >= 0 && picked.lgs >= 0,
-                "pick_shape exponents %d %d %d", picked.lgm, picked.lgn, picked.lgs);
-          check_bijection(picked, "pick_shape");
-          // k_dhidden rebuilds the list for the live rows of tiles (0 .. tm) with the launch's shape; the
+          const TileMap full(tm, tn, nf, sp);
+          check_bijection(full, "every grid");
+          // k_dhidden rebuilds the list for the live rows of tiles (0 .. tm); the
           // launch has items() of the full list, which must cover the rebuilt one
           for (int live = 0; live <= tm; live += (tm > 8 ? tm / 4 + 1 : 1)) {
-            const TileMap lv(live, picked.tiles_n, picked.n_first, picked.lgm, picked.splits, picked.lgs);
+            const TileMap lv(live, full.tiles_n, full.n_first, full.splits);
             check_bijection(lv, "live rebuild");
-            CHECK(lv.items() <= picked.items(), "live list longer than the launch: %d > %d", lv.items(), picked.items());
+            CHECK(lv.items() <= full.items(), "live list longer than the launch: %d > %d", lv.items(), full.items());
           }
         }
     }
@@ -158,9 +153,9 @@ static void check_plan(const MjGrpoDesc& d, bool launches = true) {
     covered += nc;
     // the launches of this chunk: every tile of each product exactly once (spot check at the real shapes)
     if (launches && p.V <= 160000 && p.H <= 4096 && nc <= 32768 && (c0 == 0 || c0 + nc == p.N)) {
-      check_bijection(TileMap::pick_shape((int)((p.V + 255) / 256), (int)((nc + 255) / 256), 1, 1), "logits launch");
-      check_bijection(TileMap::pick_shape((int)((nc + 255) / 256), (int)((p.H + 255) / 256), 0, p.dh_splits), "d_hidden launch");
-      check_bijection(TileMap::pick_shape((int)((p.V + 255) / 256), (int)((p.H + 255) / 256), 0, 1), "d_w launch");
+      check_bijection(TileMap((int)((p.V + 255) / 256), (int)((nc + 255) / 256), 1, 1), "logits launch");
+      check_bijection(TileMap((int)((nc + 255) / 256), (int)((p.H + 255) / 256), 0, p.dh_splits), "d_hidden launch");
+      check_bijection(TileMap((int)((p.V + 255) / 256), (int)((p.H + 255) / 256), 0, 1), "d_w launch");
     }
   }
   CHECK(covered == p.N, "chunks cover %lld of %lld tokens", (long long)covered, (long long)p.N);
@@ -232,17 +227,23 @@ static void noalloc_sweep() {
 }
 
 static void sampler_sweep() {
-  for (int64_t b : {1, 8, 64, 128, 129, 192, 256, 1000})
-    for (int64_t v : {8, 512, 32000, 152064, 256000, 1 << 21}) {
+  for (int64_t b : {1, 3, 8, 64, 128, 129, 192, 256, 257, 1000, 100000})
+    for (int64_t v = 8; v <= 1 << 21; v += v < 5000 ? 8 : (v < 300000 ? 2008 : 100008)) {
       int bn;
       int64_t tiles_n, rows;
       sample_tiles(b, v, &bn, &tiles_n, &rows);
       CHECK((bn == 128 || bn == 256) && tiles_n * bn >= b && (tiles_n - 1) * bn < b, "batch tiles: bn %d x %lld for %lld",
             bn, (long long)tiles_n, (long long)b);
       CHECK(rows >= 8 && rows <= 256 && rows % 8 == 0, "tile_rows %lld", (long long)rows);
-      const int64_t items = (v + rows - 1) / rows;
-      CHECK(items * rows >= v && (items - 1) * rows < v, "vocab items");
-      check_bijection(TileMap::pick_shape((int)items, (int)tiles_n, 1, 1), "sampler launch");
+      // the kernel's columns of each item: they follow each other, are at most a tile wide and end behind the vocabulary
+      const mj::RowItems cols((int)v, (int)((v + rows - 1) / rows));
+      CHECK(cols.items >= 1 && cols.first(0) == 0, "items %d", cols.items);
+      for (int i = 0; i < cols.items; ++i) {
+        const int m0 = cols.first(i), m1 = cols.first(i + 1);
+        CHECK(m0 % 8 == 0 && m0 < v && m1 > m0 && m1 - m0 <= BM, "vocab %lld: item %d of %d has columns %d to %d", (long long)v, i, cols.items, m0, m1);
+      }
+      CHECK(cols.first(cols.items) >= v, "vocab %lld: the last item ends at %d", (long long)v, cols.first(cols.items));
+      if ((long)cols.items * tiles_n <= 20000) check_bijection(TileMap(cols.items, (int)tiles_n, 1, 1), "sampler launch");
     }
 }
 
