@@ -9,20 +9,18 @@ from oracle import grpo_oracle as O
 pytestmark = pytest.mark.gpu
 
 
-def _draw(noise, x, k, t, v=None):
+def _draw(noise, logits, k, t):
     """Tokens, indices and values of both forms of the draw, which must agree: mj_sample_draw with its workspace
     (top_k_sampling_batched: long rows in segments) and mj_sample_top_k (one workgroup per row)."""
     import mllm_jax_amd as M
     from mllm_jax_amd import _lib
-    dev = torch.device("cuda:0")
-    lg = torch.tensor(x, device=dev)[:, :v]
-    nz = None if noise is None else torch.tensor(noise, device=dev)
-    tok, idx, val = M.top_k_sampling_batched(nz, lg, k=k, t=t, return_top_k=True)
+    noise = None if noise is None else noise.to(logits.device)
+    tok, idx, val = M.top_k_sampling_batched(noise, logits, k=k, t=t, return_top_k=True)
     tok1, idx1, val1 = torch.empty_like(tok), torch.empty_like(idx), torch.empty_like(val)
-    _lib.check(_lib.load().mj_sample_top_k(lg.data_ptr(), lg.stride(0), lg.shape[0], lg.shape[1], k, t, None if nz is None else nz.data_ptr(),
+    _lib.check(_lib.load().mj_sample_top_k(logits.data_ptr(), logits.stride(0), *logits.shape, k, t, None if noise is None else noise.data_ptr(),
                                            tok1.data_ptr(), idx1.data_ptr(), val1.data_ptr(), torch.cuda.current_stream().cuda_stream))
     assert torch.equal(tok, tok1) and torch.equal(idx, idx1) and torch.equal(val.view(torch.int32), val1.view(torch.int32))
-    return tok.cpu().numpy(), idx.cpu().numpy(), val.cpu().numpy()
+    return tok, idx, val
 
 
 def test_last_position_logits_match_float64_product():
@@ -45,13 +43,12 @@ def test_last_position_logits_match_float64_product():
 @pytest.mark.parametrize("b,v,k,t", [(3, 1000, 50, 0.9), (64, 152064, 50, 1.0), (7, 129, 64, 0.7), (2, 50, 50, 1.0),
                                      (5, 4097, 1, 1.0)])
 def test_top_k_draw_is_bit_exact(b, v, k, t):
-    import mllm_jax_amd as M
     dev = torch.device("cuda:0")
     g = torch.Generator().manual_seed(b * 1000 + k)
     logits = (3.0 * torch.randn(b, v, generator=g)).float()
     u = torch.rand(b, k, generator=g)
     noise = -torch.log(-torch.log(u))
-    tok, idx, val = M.top_k_sampling_batched(noise.to(dev), logits.to(dev), k=k, t=t, return_top_k=True)
+    tok, idx, val = _draw(noise.to(dev), logits.to(dev), k=k, t=t)
     rt, ri, rv = O.top_k_sample(logits.numpy(), k=k, t=t, noise=noise.numpy())
     np.testing.assert_array_equal(idx.cpu().numpy(), ri)
     np.testing.assert_array_equal(val.cpu().numpy(), rv)
@@ -63,7 +60,6 @@ def test_neighbouring_floats_that_divide_to_the_same_quotient(t):
     """A cluster of adjacent float32 values around the k-th largest: after the division by t > 1
     neighbours collapse into equal quotients and the lower index must win, also for elements that
     sit a few ulps below the kernel's raw-value threshold."""
-    import mllm_jax_amd as M
     dev = torch.device("cuda:0")
     rng = np.random.default_rng(7)
     b, v, k = 4, 70000, 50
@@ -81,7 +77,7 @@ def test_neighbouring_floats_that_divide_to_the_same_quotient(t):
             cluster[j] = c
         x[r, pos] = cluster
     noise = rng.gumbel(size=(b, k)).astype(np.float32)
-    tok, idx, val = M.top_k_sampling_batched(torch.tensor(noise), torch.tensor(x, device=dev), k=k, t=t, return_top_k=True)
+    tok, idx, val = _draw(torch.tensor(noise), torch.tensor(x, device=dev), k=k, t=t)
     rt, ri, rv = O.top_k_sample(x, k=k, t=t, noise=noise)
     np.testing.assert_array_equal(idx.cpu().numpy(), ri)
     np.testing.assert_array_equal(val.cpu().numpy(), rv)
@@ -91,7 +87,6 @@ def test_neighbouring_floats_that_divide_to_the_same_quotient(t):
 def test_signed_zeros_and_nans_follow_the_total_order():
     """Rows of +0 / -0 / tiny values (the k-th place falls among zeros of both signs) and rows with
     NaN and infinities: selection and order are those of the IEEE total order, as in the oracle."""
-    import mllm_jax_amd as M
     dev = torch.device("cuda:0")
     rng = np.random.default_rng(11)
     for v, k in ((50, 34), (129, 64), (5000, 50), (70000, 50)):
@@ -102,7 +97,7 @@ def test_signed_zeros_and_nans_follow_the_total_order():
         x[4, rng.integers(0, v, size=5)] = np.nan
         x[5, rng.integers(0, v, size=3)] = np.inf
         x[5, rng.integers(0, v, size=3)] = -np.inf
-        tok, idx, val = M.top_k_sampling_batched(None, torch.tensor(x, device=dev), k=k, t=1.3, return_top_k=True)
+        tok, idx, val = _draw(None, torch.tensor(x, device=dev), k=k, t=1.3)
         rt, ri, rv = O.top_k_sample(x, k=k, t=1.3, noise=None)
         np.testing.assert_array_equal(idx.cpu().numpy(), ri)
         np.testing.assert_array_equal(val.cpu().numpy().view(np.uint32), rv.view(np.uint32))
@@ -110,7 +105,6 @@ def test_signed_zeros_and_nans_follow_the_total_order():
 
 
 def test_ties_duplicates_and_negative_values():
-    import mllm_jax_amd as M
     dev = torch.device("cuda:0")
     rng = np.random.default_rng(0)
     # few distinct values: the k-th largest is shared by many entries, lower indices must win
@@ -118,7 +112,7 @@ def test_ties_duplicates_and_negative_values():
     x[4] = -7.0                                             # a constant row: indices 0..k-1
     x[5, 100:] = -np.inf
     noise = rng.gumbel(size=(9, 50)).astype(np.float32)
-    tok, idx, val = M.top_k_sampling_batched(torch.tensor(noise), torch.tensor(x, device=dev), k=50, t=1.0, return_top_k=True)
+    tok, idx, val = _draw(torch.tensor(noise), torch.tensor(x, device=dev), k=50, t=1.0)
     rt, ri, rv = O.top_k_sample(x, k=50, t=1.0, noise=noise)
     np.testing.assert_array_equal(idx.cpu().numpy(), ri)
     np.testing.assert_array_equal(val.cpu().numpy(), rv)
@@ -151,7 +145,6 @@ def test_greedy_generator_draws_and_fused_step():
 
 def test_near_equal_logits_overflow_the_pool_and_take_the_slow_path():
     # more than 4096 logits share the 12 leading key bits of the k-th largest: the byte-wise select runs
-    import mllm_jax_amd as M
     dev = torch.device("cuda:0")
     rng = np.random.default_rng(2)
     x = np.full((4, 30000), 1.5, np.float32)
@@ -159,7 +152,7 @@ def test_near_equal_logits_overflow_the_pool_and_take_the_slow_path():
     x[2, ::7] = 9.0                                             # 4286 equal maxima: ties beyond k
     x[3] = rng.integers(0, 3, 30000).astype(np.float32)         # three values
     noise = rng.gumbel(size=(4, 50)).astype(np.float32)
-    tok, idx, val = M.top_k_sampling_batched(torch.tensor(noise), torch.tensor(x, device=dev), k=50, t=1.0, return_top_k=True)
+    tok, idx, val = _draw(torch.tensor(noise), torch.tensor(x, device=dev), k=50, t=1.0)
     rt, ri, rv = O.top_k_sample(x, k=50, t=1.0, noise=noise)
     np.testing.assert_array_equal(idx.cpu().numpy(), ri)
     np.testing.assert_array_equal(val.cpu().numpy(), rv)
@@ -171,7 +164,6 @@ def test_rows_cut_into_segments_draw_like_whole_rows(v, ld):
     """Vocabularies either side of a segment's 16384 elements, rows that are not 16-byte aligned, the
     largest values at the segments' ends, NaNs, ties across segments and a row whose ties overflow a
     segment's pool: bit for bit the oracle's choice."""
-    import mllm_jax_amd as M
     dev = torch.device("cuda:0")
     rng = np.random.default_rng(v)
     k = 64
@@ -184,7 +176,7 @@ def test_rows_cut_into_segments_draw_like_whole_rows(v, ld):
     x[5] = 1.0
     noise = rng.gumbel(size=(6, k)).astype(np.float32)
     lg = torch.tensor(x, device=dev)[:, :v]
-    tok, idx, val = M.top_k_sampling_batched(torch.tensor(noise), lg, k=k, t=0.9, return_top_k=True)
+    tok, idx, val = _draw(torch.tensor(noise), lg, k=k, t=0.9)
     rt, ri, rv = O.top_k_sample(x[:, :v], k=k, t=0.9, noise=noise)
     np.testing.assert_array_equal(idx.cpu().numpy(), ri)
     np.testing.assert_array_equal(val.cpu().numpy().view(np.uint32), rv.view(np.uint32))
@@ -213,13 +205,12 @@ def test_one_or_two_rows_on_the_vector_alus(b, h, v, cap):
 def test_a_row_whose_last_segment_would_be_a_single_logit():
     """4095 * 16384 + 1 logits, all negative, the largest at the very end: cut into 4096 segments the last one
     would hold one logit.  Distinct values, so the top k of the row is that of torch.topk."""
-    import mllm_jax_amd as M
     v = 4095 * 16384 + 1
     row = torch.full((1, v), -5.0, device="cuda:0")
     at = torch.arange(63, device="cuda:0") * 1000003 + 17
     row[0, at] = -1.0 - 0.01 * torch.arange(63, device="cuda:0")
     row[0, v - 1] = -0.5
-    tok, idx, val = M.top_k_sampling_batched(None, row, k=64, t=1.0, return_top_k=True)
+    tok, idx, val = _draw(None, row, k=64, t=1.0)
     assert int(tok[0]) == v - 1
     assert idx[0].tolist() == [v - 1] + at.tolist()
     assert torch.equal(val[0], row[0, idx[0].long()])
@@ -251,7 +242,6 @@ def test_masked_blocks_and_crowded_segments(v, k):
     type's lowest value that fill whole segments, rows with a handful of unmasked logits, one value everywhere,
     ties in the middle of a segment, two neighbouring floats, NaNs; also more segments than k and than a
     wavefront has lanes, and lists whose words overflow the draw's pool.  Bit for bit the oracle's choice."""
-    import mllm_jax_amd as M
     dev = torch.device("cuda:0")
     rng = np.random.default_rng(v + k)
     x = rng.normal(0, 2, size=(11, v)).astype(np.float32)
@@ -270,7 +260,7 @@ def test_masked_blocks_and_crowded_segments(v, k):
     x[9, ::5] = np.round(x[9, ::5])                                     # few distinct values above it
     x[10, :20000] = np.nan
     noise = rng.gumbel(size=(11, k)).astype(np.float32)
-    tok, idx, val = M.top_k_sampling_batched(torch.tensor(noise), torch.tensor(x, device=dev), k=k, t=0.9, return_top_k=True)
+    tok, idx, val = _draw(torch.tensor(noise), torch.tensor(x, device=dev), k=k, t=0.9)
     rt, ri, rv = O.top_k_sample(x, k=k, t=0.9, noise=noise)
     np.testing.assert_array_equal(idx.cpu().numpy(), ri)
     np.testing.assert_array_equal(val.cpu().numpy().view(np.uint32), rv.view(np.uint32))
@@ -287,8 +277,8 @@ def test_quotients_that_overflow_or_lose_their_digits(v, t, scale):
     x = (scale * rng.normal(0, 2, size=(3, v))).astype(np.float32)
     x[2] = -np.abs(x[2])
     noise = rng.gumbel(size=(3, 50)).astype(np.float32)
-    tok, idx, val = _draw(noise, x, 50, t)
+    tok, idx, val = _draw(torch.tensor(noise), torch.tensor(x, device="cuda:0"), k=50, t=t)
     rt, ri, rv = O.top_k_sample(x, k=50, t=t, noise=noise)
-    np.testing.assert_array_equal(idx, ri)
-    np.testing.assert_array_equal(val.view(np.uint32), rv.view(np.uint32))
-    np.testing.assert_array_equal(tok, rt)
+    np.testing.assert_array_equal(idx.cpu().numpy(), ri)
+    np.testing.assert_array_equal(val.cpu().numpy().view(np.uint32), rv.view(np.uint32))
+    np.testing.assert_array_equal(tok.cpu().numpy(), rt)
