@@ -596,13 +596,18 @@ int mj_sample_logits(const void* hidden, int64_t ld_hidden, const void* lm_head,
   a.w = (const __bf16*)lm_head; a.hid = (const __bf16*)hidden; a.ld_w = ld_w; a.ld_hid = ld_hidden;
   a.V = (int)vocab; a.n = (int)b; a.H = (int)h; a.cap = softcap; a.out = logits; a.ld_out = ld_logits;
   hipStream_t st = (hipStream_t)stream;
-  // One or two rows go to the vector ALUs: 57.7 -> 51.0 us at 1 x 896 x 151936, 60.0 -> 52.8 at two rows, 184 -> 177
-  // at 1 x 4096 x 128256, 18.7 -> 14.8 at 1 x 904 x 32008.  With four rows their multiply-adds show (57 against
-  // 60 us at the first shape, but 219 against 207 at 3584 x 152064 and 24 against 18 at the last).
+  // One or two rows go to the vector ALUs: 57.3 -> 47.3 us at 1 x 896 x 152064, 57.8 -> 49.4 at two rows, 221 -> 208
+  // at 1 x 4096 x 152064, 16.1 -> 11.2 at 1 x 896 x 32000 (few_items has the other sizes).  With four rows their
+  // multiply-adds show: 57 against 60 us at 896 x 151936, but 219 against 207 at 3584 x 152064 and 24 against 18 at
+  // 904 x 32008.
   if (b <= 2) {
-    const unsigned grid = (unsigned)((vocab + 255) / 256);
-    if (b == 1) mj::k_logits_few<1><<<grid, 64 * mj::kFewWaves, 0, st>>>(a);
-    else mj::k_logits_few<2><<<grid, 64 * mj::kFewWaves, 0, st>>>(a);
+    const FewItems f = few_items(b, vocab, ld_w);
+    a.cols = mj::RowItems((int)vocab, f.items, f.unit);
+    a.together = f.together;
+    const mj::TileMap map(a.cols.items, 1, 1, 1);
+    auto kernel = f.waves == 8 ? (b == 1 ? mj::k_logits_few<1, 8> : mj::k_logits_few<2, 8>)
+                               : (b == 1 ? mj::k_logits_few<1, 4> : mj::k_logits_few<2, 4>);
+    kernel<<<map.items(), 64 * f.waves, 0, st>>>(a, map);
     return check_launch("k_logits_few");
   }
   // Batch-row tile and vocab columns per work item: the fewest rounds of resident workgroups (one

@@ -1325,7 +1325,8 @@ struct LogitsRowsArgs {
   float cap;             // final-logit softcap, 0 = off
   float* out;            // [n, ld_out]
   int64_t ld_out;
-  RowItems cols;         // which columns a work item has (k_logits_rows)
+  RowItems cols;         // which columns a work item has
+  int together;          // k_logits_few: neighbouring items on one XCD
 };
 
 // A decode batch is a few rows against the whole vocabulary matrix: the product is bound by reading
@@ -1376,17 +1377,19 @@ __global__ __launch_bounds__(kThreads) void k_logits_rows(LogitsRowsArgs p, Tile
 // The same product for one or two batch rows.  A matrix tile is 128 rows wide whatever the batch, and a
 // small model's k loop (14 slices at hidden 896) is over before a tile's pipeline has filled.  With NB <= 2
 // the products are few enough for the vector ALUs, so W streams straight into registers: a
-// workgroup owns 256 columns, a wavefront every fourth group of sixteen k-rows of them (lanes 0..31 the even rows,
-// lanes 32..63 the odd ones, 16 bytes each; the next group requested before the current one is used), hidden
-// comes through the constant cache, and the sums of the wavefronts and of their halves meet in the LDS.
-constexpr int kFewWaves = 4;
-template <int NB>
-__global__ __launch_bounds__(64 * kFewWaves) void k_logits_few(LogitsRowsArgs p) {
-  __shared__ __attribute__((aligned(16))) float part[2 * kFewWaves][256];
+// workgroup owns up to 256 columns (few_items), a wavefront every WAVES-th group of sixteen k-rows of them (lanes
+// 0..31 the even rows, lanes 32..63 the odd ones, 16 bytes each; the next group requested before the current one is
+// used), hidden comes through the constant cache, and the sums of the wavefronts and of their halves meet in the LDS.
+template <int NB, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void k_logits_few(LogitsRowsArgs p, TileMap map) {
+  __shared__ __attribute__((aligned(16))) float part[2 * WAVES][256];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l31 = lane & 31, odd = lane >> 5;
-  const int col0 = blockIdx.x * 256;
-  const bool inside = col0 + l31 * 8 < p.V;                      // V % 8 == 0
+  int item = blockIdx.x, tn, split;
+  if (p.together && !map.tile(blockIdx.x, item, tn, split)) return;
+  if (item >= p.cols.items) return;
+  const int col0 = p.cols.first(item), col1 = min(p.V, p.cols.first(item + 1));
+  const bool inside = col0 + l31 * 8 < col1;                     // both are multiples of 8
   const uint32_t ld2 = (uint32_t)p.ld_w * 2;
   const uint32_t voff = inside ? (uint32_t)l31 * 16 + odd * ld2 : kOob;
   float acc[NB][8];
@@ -1425,11 +1428,11 @@ __global__ __launch_bounds__(64 * kFewWaves) void k_logits_few(LogitsRowsArgs p)
   };
   u32x4 wa[8], wb[8];
   load(wave, wa);
-  for (int g = wave; g < groups; g += 2 * kFewWaves) {
-    load(g + kFewWaves, wb);
+  for (int g = wave; g < groups; g += 2 * WAVES) {
+    load(g + WAVES, wb);
     use(g, wa);
-    load(g + 2 * kFewWaves, wa);
-    if (g + kFewWaves < groups) use(g + kFewWaves, wb);
+    load(g + 2 * WAVES, wa);
+    if (g + WAVES < groups) use(g + WAVES, wb);
   }
   const float inv_cap = p.cap > 0.f ? 1.f / p.cap : 0.f;
 #pragma unroll
@@ -1439,10 +1442,10 @@ __global__ __launch_bounds__(64 * kFewWaves) void k_logits_few(LogitsRowsArgs p)
     *(f32x4*)mine = f32x4{acc[b][0], acc[b][1], acc[b][2], acc[b][3]};
     *(f32x4*)(mine + 4) = f32x4{acc[b][4], acc[b][5], acc[b][6], acc[b][7]};
     __syncthreads();
-    if (b < p.n && col0 + tid < p.V) {
+    if (b < p.n && tid < col1 - col0) {
       float z = 0.f;
 #pragma unroll
-      for (int q = 0; q < 2 * kFewWaves; ++q) z += part[q][tid];
+      for (int q = 0; q < 2 * WAVES; ++q) z += part[q][tid];
       if (p.cap > 0.f) z = softcap_apply(z, p.cap, inv_cap);
       p.out[(int64_t)b * p.ld_out + col0 + tid] = z;
     }

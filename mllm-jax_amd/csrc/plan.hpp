@@ -188,6 +188,37 @@ inline void sample_tiles(int64_t b, int64_t vocab, int* bn_out, int64_t* tiles_n
   *tile_rows_out = tile_rows;
 }
 
+// The same product for one or two rows (k_logits_few): how many workgroups of at most 256 columns, in which units,
+// with how many wavefronts, and in which order they go to the XCDs.  us at hidden 4096 (one row unless it says two):
+// the matrix tile, 256-wide workgroups of four wavefronts in plain order whatever the vocabulary, and this rule:
+//   65000    83.7  97.5  83.7   rows end inside a memory line (anything but a multiple of 256 bytes), and the
+//                               neighbour that needs the other half of it sits on another XCD: kept on one
+//   90000   121   141   116    352 workgroups for 256 CUs: some have two, the others wait.  From one round
+//   200000  271   297   269    on a whole number of rounds, the columns spread evenly
+//   32000    52    65    45    (two rows) half the CUs without a workgroup: up to 256 of at least 64 columns, and eight
+//   36000    51    67    53    (two rows) wavefronts each; up to 176 workgroups for two rows, 144 for one
+//   40000    53    52          (one row: split 55)
+//   152064  221   217   208
+//   256000  362   350   353    lines and rounds come out even: plain order (together it is 4 % slower)
+// In between (45000 to 65536) 256-wide workgroups are as good as any: 50048 74.6, 64.7, 66.5.
+struct FewItems {
+  int items, unit, waves;
+  bool together;          // neighbouring pieces on one XCD
+};
+inline FewItems few_items(int64_t b, int64_t vocab, int64_t ld_w) {
+  const int64_t full = (vocab + 255) / 256;
+  FewItems f = {(int)full, 256, 4, ld_w % 128 != 0};
+  if (full > (b == 1 ? 144 : 176) && full <= 256) return f;
+  f.unit = f.together ? 32 : 64;
+  if (full > 256) f.items = (int)rup(full, 256);
+  else {
+    f.items = (int)((vocab + 63) / 64);
+    if (f.items > 256) f.items = 256;
+    f.waves = 8;
+  }
+  return f;
+}
+
 // Segments of a row for the top-k draw: as few as hold the row at kDrawSegment elements each, of even
 // length.  segs == 0: the rows are drawn from without them -- short rows (below 4096 elements too few of a
 // segment's groups of threads hold any, and one workgroup has a row in registers' reach anyway), rows longer

@@ -71,15 +71,16 @@ struct TileMap {
   }
 };
 
-// The columns of the sampler's logits product: whole units of kRowUnit, spread evenly over the work items (the
-// first ones take one unit more where it does not come out even).
+// The columns of the sampler's logits product: whole units, spread evenly over the work items (the first ones
+// take one unit more where it does not come out even).
 constexpr int kRowUnit = 32;
 struct RowItems {
-  int units, items;
-  MJ_HD RowItems(int vocab = 0, int items_ = 0) : units((vocab + kRowUnit - 1) / kRowUnit), items(items_ < units ? items_ : units) {}
+  int unit, units, items;
+  MJ_HD RowItems(int vocab = 0, int items_ = 0, int unit_ = kRowUnit)
+      : unit(unit_), units((vocab + unit_ - 1) / unit_), items(items_ < units ? items_ : units) {}
   MJ_HD int first(int item) const {       // first column of the item; the last item ends at the vocabulary's end
     const int base = units / items, wide = units - base * items;
-    return (item * base + (item < wide ? item : wide)) * kRowUnit;
+    return (item * base + (item < wide ? item : wide)) * unit;
   }
 };
 

@@ -247,6 +247,29 @@ static void sampler_sweep() {
     }
 }
 
+// One or two rows: pieces of at most 256 columns that follow each other to the end of the vocabulary, begin at whole
+// sectors, and are all there in both orders.
+static void few_sweep() {
+  for (int64_t v = 8; v <= 1 << 21; v += v < 70000 ? 8 : (v < 300000 ? 1000 : 100008))
+    for (int64_t pad : {0, 8, 64, -1}) {
+      const int64_t b = pad < 0 ? 2 : 1;
+      if (pad < 0) pad = 0;
+      const FewItems f = few_items(b, v, v + pad);
+      const mj::RowItems cols((int)v, f.items, f.unit);
+      CHECK(cols.items >= 1 && cols.first(0) == 0 && (f.waves == 4 || f.waves == 8), "items %d waves %d", cols.items, f.waves);
+      CHECK(f.together == ((v + pad) % 128 != 0), "order of %lld", (long long)(v + pad));
+      for (int i = 0; i < cols.items; ++i) {
+        const int m0 = cols.first(i), m1 = cols.first(i + 1);
+        CHECK(m0 % 32 == 0 && m0 < v && m1 > m0 && m1 - m0 <= 256, "vocab %lld: item %d of %d has columns %d to %d", (long long)v, i, cols.items, m0, m1);
+      }
+      CHECK(cols.first(cols.items) >= v, "vocab %lld: the last item ends at %d", (long long)v, cols.first(cols.items));
+      // no CU gets many more columns than another: whole rounds of 256 from one round on
+      if (v > 65536) CHECK(cols.items % 256 == 0, "vocab %lld: %d items", (long long)v, cols.items);
+      const TileMap map(cols.items, 1, 1, 1);
+      CHECK(map.items() >= cols.items, "the grid holds every item");
+    }
+}
+
 // Segments of a row for the draw: they cover it, fit a workgroup's registers, and the last one still holds a list
 // of the longest k (the kernel reads whole quads up to the segment's end, so it must hold one at the very least).
 static void draw_sweep() {
@@ -284,6 +307,7 @@ static void norm_sweep() {
 
 int main() {
   draw_sweep();
+  few_sweep();
   norm_sweep();
   tile_map_sweep();
   plan_sweep();

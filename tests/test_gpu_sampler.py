@@ -185,10 +185,15 @@ def test_rows_cut_into_segments_draw_like_whole_rows(v, ld):
 
 
 @pytest.mark.parametrize("b,h,v,cap", [(1, 8, 8, None), (1, 24, 264, 30.0), (2, 56, 1000, None), (2, 72, 256, 10.0), (1, 136, 2008, None),
-                                       (2, 904, 5000, None)])
+                                       (2, 904, 5000, None),
+                                       # pieces of 64 columns in eight wavefronts, of 64 and 128, whole ones of 256, and even
+                                       # shares of one, two and three rounds; pitches (v + 16) with and without shared lines
+                                       (1, 40, 16368, None), (2, 40, 16376, None), (1, 24, 36848, None), (1, 24, 36880, None), (2, 24, 45040, None),
+                                       (2, 24, 45064, None), (1, 24, 65520, None), (2, 24, 65536, None), (1, 24, 65544, 30.0), (2, 24, 72008, None),
+                                       (1, 24, 131056, None), (2, 136, 131080, None)])
 def test_one_or_two_rows_on_the_vector_alus(b, h, v, cap):
-    """k_logits_few: odd counts of 8-row groups, columns either side of a workgroup's 256, softcap; a row
-    pitch of W and of hidden past their lengths.  The bound is float32 summation: h products of at most
+    """k_logits_few: odd counts of 8-row groups, columns either side of a workgroup's 256 and of each split, softcap;
+    a row pitch of W and of hidden past their lengths.  The bound is float32 summation: h products of at most
     0.2 * 4 * 4 in magnitude, one rounding of 2^-24 of the partial sum each."""
     import mllm_jax_amd as M
     dev = torch.device("cuda:0")
