@@ -374,7 +374,7 @@ int run(Mode mode, const MjGrpoDesc* d, const void* hidden, const void* lm_head,
 
 extern "C" {
 
-int mj_grpo_version(void) { return 300; }   // 0.3.0: MJ_GRPO_FLAG_DW_BF16, d_lm_head as void*
+int mj_grpo_version(void) { return 301; }   // 0.3.1: mj_sample_draw, mj_sample_draw_workspace_bytes
 
 const char* mj_grpo_last_error(void) { return mj::host::g_err; }
 

@@ -19,9 +19,10 @@ namespace mj {
 // that shares its operand slices in an L2.  The k-splits follow each other in the same list; where one has fewer
 // than 32 tiles, a group spans several.  Groups of 32 consecutive items go to
 // the eight XCDs in turn (ids congruent mod 8 run on the same XCD): an XCD works on one such block at
-// a time, the eight XCDs on eight neighbouring ones.  Of the last, partial round each XCD gets an
-// eighth: in lots of 32 its tiles would be work for a few XCDs (dW of 512 x 896 x 151936, 2376 tiles: 72 left over,
-// on three XCDs 235.5 us, on all eight 232; a whole pass of 256 x 896 468 -> 452, larger ones the same).
+// a time, the eight XCDs on eight neighbouring ones.  Of a last round of up to kDealt tiles each XCD gets an
+// eighth: in lots of 32 they would be work for a few XCDs (logits of 246 tokens x 3064, one round and 40, 72, 128
+// or 192 tiles: 175 -> 167 us, 179 -> 169, 181 -> 171, 188 -> 182; a whole pass of 256 x 896 x 151936 468 -> 452).
+// A fuller one keeps its lots (232 tiles: 194 us, 199 in eighths; 242: 197 and 201).
 //
 // The list holds real tiles only and the strips of a grid differ by at most one in width, which
 // is what keeps the XCDs equally loaded: with fixed 4 x 8 blocks and the empty slots of ragged ones as
@@ -29,7 +30,7 @@ namespace mj {
 // of eight, all of those on the same four XCDs (2049 tokens x 4096 x 128256: logits 2.9 ms against
 // 1.85 ms in this order).
 struct TileMap {
-  static constexpr int kTall = 4, kLong = 8;
+  static constexpr int kTall = 4, kLong = 8, kDealt = 192;
   int tiles_m, tiles_n, n_first, splits;
   int width, wide;         // strips: the first `wide` ones are width + 1 tiles across, the others `width`
   MJ_HD TileMap(int tm, int tn, int n_first_, int splits_)
@@ -45,10 +46,12 @@ struct TileMap {
     const int q = pid >> 3, xcd = pid & 7, round = q >> 5, within = q & 31;
     int at = (round << 8) + xcd * 32 + within;                  // place in the list of tiles
     const int left = tiles() - (round << 8);
-    if (left < 256) {                                           // the last round: an eighth each
+    if (left <= kDealt) {                                       // the last round: an eighth each
       const int each = left > 0 ? left >> 3 : 0, more = left > 0 ? left & 7 : 0;
       if (within >= each + (xcd < more ? 1 : 0)) return false;
       at = (round << 8) + xcd * each + (xcd < more ? xcd : more) + within;
+    } else if (at >= tiles()) {
+      return false;
     }
     const int per = tiles_m * tiles_n, along = n_first ? tiles_n : tiles_m;
     split = at / per;
