@@ -345,7 +345,7 @@ MJ_DEV void logits_tile16(const LogitsArgs& p, int tm, int tn, char* smem, int t
   for (int ni = 0; ni < G::NI; ++ni) {
     const int col = t0 + ni * 16 + l15;
     // softcap: see logits_tile_grad (series while every logit of the wavefront's block column is small
-    // against the cap; the capped logit is kept in units of log2)
+    // against the cap; the capped logit is kept in units of log2 in kStatsExp, in natural ones in kStatsMax)
     if (CAP) {
       float big = 0.f;
 #pragma unroll
