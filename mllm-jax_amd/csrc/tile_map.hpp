@@ -19,10 +19,14 @@ namespace mj {
 // that shares its operand slices in an L2.  The k-splits follow each other in the same list; where one has fewer
 // than 32 tiles, a group spans several.  Groups of 32 consecutive items go to
 // the eight XCDs in turn (ids congruent mod 8 run on the same XCD): an XCD works on one such block at
-// a time, the eight XCDs on eight neighbouring ones.  Of a last round of up to kDealt tiles each XCD gets an
-// eighth: in lots of 32 they would be work for a few XCDs (logits of 246 tokens x 3064, one round and 40, 72, 128
-// or 192 tiles: 175 -> 167 us, 179 -> 169, 181 -> 171, 188 -> 182; a whole pass of 256 x 896 x 151936 468 -> 452).
-// A fuller one keeps its lots (232 tiles: 194 us, 199 in eighths; 242: 197 and 201).
+// a time, the eight XCDs on eight neighbouring ones.
+//
+// The last, partial round (dealt()): in lots of 32 its tiles are work for a few XCDs while the others idle, an
+// eighth each uses all of them.  That is better behind up to four full rounds, with 48 to 192 tiles left: logits of
+// 246 x 3064, one round and 72, 128, 192 tiles 179 -> 169 us, 181 -> 171, 188 -> 182; of 507 x 2088, two rounds and
+// 72 174.5 -> 166, four 290 -> 285.  Behind more rounds the XCDs have drifted apart, and the lots let the late
+// ones off: eight rounds and 72 521 us in lots, 533 in eighths, 32 rounds 1996 and 2021.  So do 36 tiles (two rounds:
+// 163 and 165), and a round that is nearly full has nothing to gain (242 tiles: 197 and 201).
 //
 // The list holds real tiles only and the strips of a grid differ by at most one in width, which
 // is what keeps the XCDs equally loaded: with fixed 4 x 8 blocks and the empty slots of ragged ones as
@@ -30,7 +34,7 @@ namespace mj {
 // of eight, all of those on the same four XCDs (2049 tokens x 4096 x 128256: logits 2.9 ms against
 // 1.85 ms in this order).
 struct TileMap {
-  static constexpr int kTall = 4, kLong = 8, kDealt = 192;
+  static constexpr int kTall = 4, kLong = 8;
   int tiles_m, tiles_n, n_first, splits;
   int width, wide;         // strips: the first `wide` ones are width + 1 tiles across, the others `width`
   MJ_HD TileMap(int tm, int tn, int n_first_, int splits_)
@@ -40,14 +44,17 @@ struct TileMap {
     width = across / strips;
     wide = across - width * strips;
   }
+  // whether the `left` tiles behind `round` full rounds are dealt evenly
+  MJ_HD static bool dealt(int round, int left) { return left <= 192 && (round == 0 || (round <= 4 && left > 48)); }
   MJ_HD int tiles() const { return tiles_m * tiles_n * splits; }
   MJ_HD int items() const { return (tiles() + 255) & ~255; }
   MJ_HD bool tile(int pid, int& tm, int& tn, int& split) const {
     const int q = pid >> 3, xcd = pid & 7, round = q >> 5, within = q & 31;
     int at = (round << 8) + xcd * 32 + within;                  // place in the list of tiles
     const int left = tiles() - (round << 8);
-    if (left <= kDealt) {                                       // the last round: an eighth each
-      const int each = left > 0 ? left >> 3 : 0, more = left > 0 ? left & 7 : 0;
+    if (left <= 0) return false;
+    if (dealt(round, left)) {                                   // the last round: an eighth each
+      const int each = left >> 3, more = left & 7;
       if (within >= each + (xcd < more ? 1 : 0)) return false;
       at = (round << 8) + xcd * each + (xcd < more ? xcd : more) + within;
     } else if (at >= tiles()) {

@@ -1,8 +1,8 @@
 // host_plan_check.cpp -- CPU checks of the host-side index arithmetic of the tile kernels, built by
 // tests/test_host_plan_cpu.py with g++ -fsanitize=address,undefined (no HIP, no GPU):
 //   * TileMap: over ids 0 .. items()-1, tile() yields every (tile row, tile column, k-split) of the
-//     problem exactly once and nothing outside it, in both walk orders, and where the last round is not nearly full no XCD gets more than one
-//     tile more than another;
+//     problem exactly once and nothing outside it, in both walk orders, and where the last round is dealt evenly no XCD gets more than one tile
+//     more than another;
 //   * the same for the "live rows" rebuild that k_dhidden makes from a device-side token count;
 //   * make_plan: workspace regions are 256-byte aligned, do not overlap, end inside the totals;
 //     the vocab splits of the d_hidden product cover V; chunks cover N;
@@ -54,7 +54,7 @@ static void check_bijection(const TileMap& m, const char* what) {
   CHECK(hits == (long)tm * tn * sp, "%s: %ld of %ld tiles produced (tm %d tn %d splits %d n_first %d)",
         what, hits, (long)tm * tn * sp, tm, tn, sp, m.n_first);
   const long most = *std::max_element(load, load + 8), least = *std::min_element(load, load + 8);
-  CHECK(most - least <= (hits % 256 <= TileMap::kDealt ? 1 : 32), "%s: %ld tiles on one XCD, %ld on another", what, most, least);
+  CHECK(most - least <= (TileMap::dealt((int)hits / 256, (int)hits % 256) ? 1 : 32), "%s: %ld tiles on one XCD, %ld on another", what, most, least);
   // ids past the end never yield a tile
   for (int id = items; id < items + 512; ++id) {
     int a, b, s;
