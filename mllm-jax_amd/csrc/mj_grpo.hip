@@ -547,6 +547,11 @@ int mj_grpo_advantages(int mode, const float* rewards, const int32_t* group_ids,
     mj::k_whiten<<<1, 1024, 0, (hipStream_t)stream>>>(advantages, (int)b, eps, clip_range);
     return check_launch("k_whiten");
   }
+  if (whitened && b <= mj::kAdvOne) {
+    a.clip = clip_range;
+    mj::k_rloo_whitened<<<1, 1024, 0, (hipStream_t)stream>>>(a);
+    return check_launch("k_rloo_whitened");
+  }
   const int per = mode == mj::kAdvGlobal ? mj::kAdvThreads : mj::kAdvThreads / mj::kAdvLanes;   // samples per workgroup
   mj::k_advantages<<<(unsigned)((b + per - 1) / per), mj::kAdvThreads, 0, (hipStream_t)stream>>>(a);
   if (whitened) mj::k_whiten<<<1, 1024, 0, (hipStream_t)stream>>>(advantages, (int)b, eps, clip_range);
