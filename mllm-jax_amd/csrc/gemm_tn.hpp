@@ -11,7 +11,8 @@
 //           out with one ds_read_b128 per lane;
 //   kKRow : X[k][row], rows contiguous -- LDS image 64 k-rows of 2*ROWS bytes, MFMA fragments
 //           come out of two ds_read_b64_tr_b16 (the LDS transposing read of gfx950).
-// Both give lane l of a fragment the same k order (8*(l/32) + 0..7), so they mix freely.
+// Both give lane l of a fragment the same k order (8*(l/32) + 0..7), so they mix freely.  GemmTN16 also takes
+// its B operand in fragment order (kFrag), which bypasses the LDS.
 //
 // K is walked in slices of 64 through two LDS stages.  A slice travels global memory ->
 // registers (16-byte buffer loads that cover whole 128-byte lines) -> LDS (ds_write_b128) ->
@@ -45,7 +46,7 @@ constexpr int kBK = 64;              // K elements per LDS stage
 constexpr int kSteps = kBK / 16;     // MFMA k-steps per stage
 constexpr uint32_t kOob = 0x7ffffff0u;   // byte offset that every descriptor below rejects
 
-enum Layout { kRowK = 0, kKRow = 1 };
+enum Layout { kRowK = 0, kKRow = 1, kFrag = 2 };
 
 MJ_DEV __amdgpu_buffer_rsrc_t make_rsrc(const void* p, int64_t bytes) {
   // raw buffer (stride 0), 32-bit data format word for gfx9-class descriptors
@@ -492,6 +493,32 @@ struct GemmTN {
   }
 };
 
+// The B operand in fragment order (kFrag): blocks of 16 rows x 32 k, 1 KB each; inside a block lane l's eight k
+// (row l % 16, k = 8 (l / 16) + 0..7) are bytes 16 l .. 16 l + 15, so a wavefront loads a fragment with one
+// contiguous 1 KB access into the registers that the matrix instruction reads.  The row blocks of 32 k lie one after
+// the other, then those of the next 32 k: what a tile reads of a slice is two contiguous pieces (row blocks ahead of k
+// blocks -- a power-of-two pitch at most batch sizes -- cost 3 % at 512 x 4096 x 128256).
+template <int NI>
+struct FragOperand {
+  const char* base;
+  int64_t slice_bytes;
+  int last;              // last slice: requests past it fetch it again
+  __amdgpu_buffer_rsrc_t rsrc;
+  uint32_t off[NI];
+  // p: row block 0 of the tile, k block 0; blocks: row blocks of the matrix; row0: first row of the wavefront
+  MJ_DEV void init(const __bf16* p, int rows_valid, int64_t blocks, int K, int row0, int tid) {
+    base = (const char*)p;
+    slice_bytes = blocks * 2048;
+#pragma unroll
+    for (int j = 0; j < NI; ++j) off[j] = row0 + j * 16 < rows_valid ? (uint32_t)(row0 / 16 + j) * 1024 + (tid & 63) * 16 : kOob;
+    last = max((K + kBK - 1) / kBK - 1, 0);
+  }
+  MJ_DEV void slice_begin(int slice) { rsrc = make_rsrc(base + min(slice, last) * slice_bytes, slice_bytes / 2 + 2 * NI * 1024); }
+  MJ_DEV bf16x8 load(int j, int ks) const {
+    return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off[j], ks * (int)(slice_bytes / 2), 0));
+  }
+};
+
 // The same 256 x 256 tile on v_mfma_f32_16x16x32_bf16, in the order that the instruction rewards.
 // A wavefront's 128 x 128 is 8 x 8 blocks of 16 x 16 and a 64-wide slice is two k-steps of 32.  The
 // two k-steps of a block are issued back to back on the same accumulator: the second instruction
@@ -510,6 +537,14 @@ struct GemmTN {
 // global memory and the LDS (a ring of 24 staging registers with one and a half slices in flight
 // measured 7 % slower: more requests in flight only lengthen each one).
 //
+// With B in fragment order (kFrag) only A goes through the LDS.  Both operands there cost 1500 of a period's 2660
+// cycles of LDS traffic (64 KB written, 128 KB read), a third of the wavefront's memory instructions, and the power that
+// moving the data takes, which is what bounds these products; B straight from the L2 halves that, and the two
+// wavefronts that share a fragment find it in the L1.  The next slice's fragments arrive in a second set of
+// registers while a slice's are in use (the loop is unrolled by two).  dW of 16384 x 3584 x 152064 takes 12.79 ms instead of
+// 13.63, of 4096 x 1536 x 151936 1.50 instead of 1.60, of 2048 x 1536 x 151936 0.83 instead of 0.91; at 512
+// tokens and below, where a tile is mostly its epilogue, the same within 2 %.
+//
 // The matrix instructions are written as assembly so that the result register IS the accumulator
 // operand: with all 256 accumulation registers taken the register allocator otherwise routes some
 // blocks through copies (and the wait states those need).  The first slice starts from the constant
@@ -527,9 +562,10 @@ struct GemmTN16 {
   static constexpr int WM = 128, WN = 128;
   static constexpr int MI = 8, NI = 8;               // 16 x 16 blocks per wavefront
   using OpA = Operand<BM, LAY_A, kThreads, DEAD_A, 16>;
-  using OpB = Operand<BN, LAY_B, kThreads, DEAD_B, 16>;
-  static constexpr int A_LD = OpA::LD, B_LD = OpB::LD, LPS = A_LD + B_LD;
-  static constexpr int kStageBytes = OpA::kBytes + OpB::kBytes;
+  static constexpr bool kFragB = LAY_B == kFrag;     // B goes from memory to the matrix instructions' registers
+  using OpB = Operand<BN, kFragB ? (int)kRowK : LAY_B, kThreads, DEAD_B, 16>;
+  static constexpr int A_LD = OpA::LD, B_LD = kFragB ? 0 : OpB::LD, LPS = A_LD + B_LD;
+  static constexpr int kStageBytes = OpA::kBytes + (kFragB ? 0 : OpB::kBytes);
   static constexpr int kLdsBytes = 2 * kStageBytes;
   // a mask over k-rows comes with a k-major A; it is read once and would serve a k-major B as well
   static constexpr bool kKDead = DEAD_A && LAY_A == kKRow;
@@ -551,14 +587,19 @@ struct GemmTN16 {
     OpA a;
     OpB b;
     a.init(A, rows_a, lda, K, wm * WM, tid, dead_a);
-    b.init(B, rows_b, ldb, K, wn * WN, tid, dead_b);
+    FragOperand<NI> bf;
+    if constexpr (kFragB) {
+      bf.init(B, rows_b, ldb, K, wn * WN, tid);
+    } else {
+      b.init(B, rows_b, ldb, K, wn * WN, tid, dead_b);
+      b.init16(wn * WN, tid);
+    }
     a.init16(wm * WM, tid);
-    b.init16(wn * WN, tid);
     KDead kd;
     if (kKDead) kd.init(dead_a, K, tid);
     auto slices_begin = [&](int slice) {     // in slice order: the mask word of the next slice is requested here
       a.slice_begin(slice);
-      b.slice_begin(slice);
+      if constexpr (!kFragB) b.slice_begin(slice);
       if (kKDead) kd.slice_begin(slice);
     };
 
@@ -577,7 +618,8 @@ struct GemmTN16 {
       if (j < A_LD) a.store_half(stage, j, staged[j], h);
       else b.store_half(stage + OpA::kBytes, j - A_LD, staged[j], h);
     };
-    bf16x8 fa[3][2], fb[NI][2];
+    constexpr int kSets = kFragB ? 2 : 1;             // kFrag: the next slice's fragments arrive while a slice's are in use
+    bf16x8 fa[3][2], fb[kSets * NI][2];
     auto read_a_half = [&](int slice, int i, int ks) {
       const char* stage = smem + (slice & 1) * kStageBytes;
       fa[slot(i)][ks] = a.frag16(stage, i, ks);
@@ -587,32 +629,41 @@ struct GemmTN16 {
       fb[j][0] = b.frag16(stage, j, 0);
       fb[j][1] = b.frag16(stage, j, 1);
     };
+    auto load_b = [&](auto set, int m) {    // kFrag: fragment m / 2, k-step m % 2 of the slice of bf.slice_begin
+      constexpr int S = decltype(set)::value;
+      if constexpr (kFragB) fb[S * NI + m / 2][m % 2] = bf.load(m / 2, m % 2);
+    };
     // first: the k-step 0..31 of block (i, j); second: its k-step 32..63, on the first one's result.
     // The second cannot issue before the first has gone through the matrix unit (16 cycles): a block's
     // memory instruction sits between the two, where the wavefront would otherwise wait.
-    auto first = [&](auto init, auto lead, int i, int j) {
+    auto first = [&](auto init, auto lead, int i, int j) {   // j: of fb
       constexpr bool kInit = decltype(init)::value != 0, kLead = decltype(lead)::value != 0;
       (void)fa; (void)fb; (void)acc;     // named outside the assembly too, so that the lambda captures them
       if constexpr (kInit)
-        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(acc[i][j]) : "v"(fa[slot(i)][0]), "v"(fb[j][0]));
+        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(acc[i][j % NI]) : "v"(fa[slot(i)][0]), "v"(fb[j][0]));
       else if constexpr (kLead)
-        asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(fa[slot(i)][0]), "v"(fb[j][0]));
+        asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j % NI]) : "v"(fa[slot(i)][0]), "v"(fb[j][0]));
       else
-        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(fa[slot(i)][0]), "v"(fb[j][0]));
+        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j % NI]) : "v"(fa[slot(i)][0]), "v"(fb[j][0]));
     };
     auto second = [&](auto settle, int i, int j) {
       constexpr bool kSettle = decltype(settle)::value != 0;
       (void)fa; (void)fb; (void)acc;
       if constexpr (kSettle)
-        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\ts_nop 9" : "+a"(acc[i][j]) : "v"(fa[slot(i)][1]), "v"(fb[j][1]));
+        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\ts_nop 9" : "+a"(acc[i][j % NI]) : "v"(fa[slot(i)][1]), "v"(fb[j][1]));
       else
-        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(fa[slot(i)][1]), "v"(fb[j][1]));
+        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j % NI]) : "v"(fa[slot(i)][1]), "v"(fb[j][1]));
     };
 
     const int KT = (K + kBK - 1) / kBK;
     slices_begin(0);
 #pragma unroll
     for (int j = 0; j < LPS; ++j) load_one(0, j);
+    if constexpr (kFragB) {
+      bf.slice_begin(0);
+#pragma unroll
+      for (int m = 0; m < 2 * NI; ++m) load_b(IntTag<0>(), m);
+    }
     slices_begin(1);
 #pragma unroll
     for (int j = 0; j < LPS; ++j) {
@@ -623,8 +674,10 @@ struct GemmTN16 {
     __builtin_amdgcn_s_barrier();       // slice 0 is in LDS, slice 1 is on its way to the registers
     read_a_half(0, 0, 0);
     read_a_half(0, 0, 1);
+    if constexpr (!kFragB) {
 #pragma unroll
-    for (int j = 0; j < NI; ++j) read_b(0, j);
+      for (int j = 0; j < NI; ++j) read_b(0, j);
+    }
 
     // A period runs from the barrier inside slice s-1 to the one inside slice s: rows 6, 7 of slice
     // s-1, then rows 0..5 of slice s: 64 blocks.  During it slice s+1 moves from the staging registers
@@ -632,6 +685,8 @@ struct GemmTN16 {
     // 8-byte LDS writes and one global load, each in the gap INSIDE a block (between its two matrix
     // instructions, where 12 issue cycles are free anyway), three blocks out of four.  The first
     // period has no rows 6, 7: its 48 blocks carry one memory instruction each.
+    // kFrag: 24 of the blocks carry A's instructions and, in the rows in front, every third one a load of
+    // the next slice's B.
     auto mem_op = [&](int s, int slot, bool first_period) {
       const int q = first_period ? slot - 16 : slot;              // 0..47 or 0..63
       const int c = first_period ? q / 3 : q / 4, r = first_period ? q % 3 : q % 4;
@@ -641,46 +696,58 @@ struct GemmTN16 {
       if (r == 2) load_one(s + 2, c);
     };
     // One block: its two matrix instructions with the period's memory instruction `slot` between them.
-    auto block = [&](auto init, auto lead, auto settle, int i, int j, int s, int slot, bool first_period) {
-      first(init, lead, i, j);
+    auto block = [&](auto init, auto lead, auto settle, auto set, int i, int j, int s, int slot, bool first_period) {
+      constexpr int S = kFragB ? decltype(set)::value : 0;
+      first(init, lead, i, S * NI + j);
       __builtin_amdgcn_sched_barrier(0);
       mem_op(s, slot, first_period);
+      if (kFragB && slot >= 16 && slot % 3 == 2) load_b(IntTag<kFragB ? 1 - S : 0>(), (slot - 16) / 3);
       __builtin_amdgcn_sched_barrier(0);
-      second(settle, i, j);
+      second(settle, i, S * NI + j);
       __builtin_amdgcn_sched_barrier(0);
     };
     // Rows 6 and 7 of slice s-1, column by column, so that the B pairs are released one per two blocks:
     // each is re-read for slice s after its last use (behind the next column's first block; the last
     // one inside row 0).  more: slice s exists (its fragments are read, the period's memory
     // instructions ride along).
-    auto rows_back = [&](auto init, auto more, int s) {
+    auto rows_back = [&](auto init, auto more, auto set, int s) {     // set: of slice s-1
       constexpr bool kMore = decltype(more)::value != 0;
-      if (kMore) slices_begin(s + 2);   // the period's loads
+      if (kMore) {                       // the period's loads
+        slices_begin(s + 2);
+        if constexpr (kFragB) bf.slice_begin(s + 1);
+      }
 #pragma unroll
       for (int j = 0; j < NI; ++j) {
-        if (j == 0) block(init, IntTag<1>(), IntTag<0>(), MI - 2, j, s, kMore ? 2 * j : -1, false);
-        else block(init, IntTag<0>(), IntTag<0>(), MI - 2, j, s, kMore ? 2 * j : -1, false);
+        if (j == 0) block(init, IntTag<1>(), IntTag<0>(), set, MI - 2, j, s, kMore ? 2 * j : -1, false);
+        else block(init, IntTag<0>(), IntTag<0>(), set, MI - 2, j, s, kMore ? 2 * j : -1, false);
         if (kMore) {
           if (j < 2) read_a_half(s, 0, j);
-          if (j > 0) read_b(s, j - 1);
+          if constexpr (!kFragB) {
+            if (j > 0) read_b(s, j - 1);
+          }
           __builtin_amdgcn_sched_barrier(0);
         }
-        if (j == NI - 1) block(init, IntTag<0>(), IntTag<1>(), MI - 1, j, s, kMore ? 2 * j + 1 : -1, false);
-        else block(init, IntTag<0>(), IntTag<0>(), MI - 1, j, s, kMore ? 2 * j + 1 : -1, false);
+        if (j == NI - 1) block(init, IntTag<0>(), IntTag<1>(), set, MI - 1, j, s, kMore ? 2 * j + 1 : -1, false);
+        else block(init, IntTag<0>(), IntTag<0>(), set, MI - 1, j, s, kMore ? 2 * j + 1 : -1, false);
       }
     };
     // Rows 0..5 of slice s; the A pair of row i+1 is read meanwhile (row 5: of rows 6 and 7).
-    auto rows_front = [&](auto init, int s, bool first_period) {
-      if (first_period) slices_begin(s + 2);
+    auto rows_front = [&](auto init, auto set, int s, bool first_period) {
+      if (first_period) {
+        slices_begin(s + 2);
+        if constexpr (kFragB) bf.slice_begin(s + 1);
+      }
 #pragma unroll
       for (int i = 0; i < MI - 2; ++i)
 #pragma unroll
         for (int j = 0; j < NI; ++j) {
-          if (i == MI - 3 && j == NI - 1) block(init, IntTag<0>(), IntTag<1>(), i, j, s, 16 + i * NI + j, first_period);
-          else block(init, IntTag<0>(), IntTag<0>(), i, j, s, 16 + i * NI + j, first_period);
+          if (i == MI - 3 && j == NI - 1) block(init, IntTag<0>(), IntTag<1>(), set, i, j, s, 16 + i * NI + j, first_period);
+          else block(init, IntTag<0>(), IntTag<0>(), set, i, j, s, 16 + i * NI + j, first_period);
           if (j < 2) read_a_half(s, i + 1, j);
           if (i == 5 && (j == 2 || j == 3)) read_a_half(s, 7, j - 2);
-          if (i == 0 && j == 2 && !first_period) read_b(s, NI - 1);   // the last B pair, left over by rows_back
+          if constexpr (!kFragB) {
+            if (i == 0 && j == 2 && !first_period) read_b(s, NI - 1);   // the last B pair, left over by rows_back
+          }
           __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -692,17 +759,38 @@ struct GemmTN16 {
     // Every accumulator is first written at exactly one place (rows 0..5: the first period; rows 6, 7:
     // the second one, which with a single slice reads the zero-filled stage of a slice past K and
     // starts loads that the buffer descriptors reject).
-    rows_front(IntTag<1>(), 0, true);
+    // kFrag: slice s uses the fragments of set s % 2.
+    rows_front(IntTag<1>(), IntTag<0>(), 0, true);
     publish();
-    rows_back(IntTag<1>(), IntTag<1>(), 1);
+    rows_back(IntTag<1>(), IntTag<1>(), IntTag<0>(), 1);
     if (KT > 1) {
-      rows_front(IntTag<0>(), 1, false);
-      for (int s = 2; s < KT; ++s) {
-        publish();
-        rows_back(IntTag<0>(), IntTag<1>(), s);
-        rows_front(IntTag<0>(), s, false);
+      rows_front(IntTag<0>(), IntTag<1>(), 1, false);
+      if constexpr (!kFragB) {
+        for (int s = 2; s < KT; ++s) {
+          publish();
+          rows_back(IntTag<0>(), IntTag<1>(), IntTag<0>(), s);
+          rows_front(IntTag<0>(), IntTag<0>(), s, false);
+        }
+        rows_back(IntTag<0>(), IntTag<0>(), IntTag<0>(), KT);
+      } else {
+        int s = 2;
+        for (; s + 1 < KT; s += 2) {
+          publish();
+          rows_back(IntTag<0>(), IntTag<1>(), IntTag<1>(), s);
+          rows_front(IntTag<0>(), IntTag<0>(), s, false);
+          publish();
+          rows_back(IntTag<0>(), IntTag<1>(), IntTag<0>(), s + 1);
+          rows_front(IntTag<0>(), IntTag<1>(), s + 1, false);
+        }
+        if (s < KT) {
+          publish();
+          rows_back(IntTag<0>(), IntTag<1>(), IntTag<1>(), s);
+          rows_front(IntTag<0>(), IntTag<0>(), s, false);
+          rows_back(IntTag<0>(), IntTag<0>(), IntTag<0>(), KT);
+        } else {
+          rows_back(IntTag<0>(), IntTag<0>(), IntTag<1>(), KT);
+        }
       }
-      rows_back(IntTag<0>(), IntTag<0>(), KT);
     }
   }
 };

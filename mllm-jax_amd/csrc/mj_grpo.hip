@@ -326,12 +326,12 @@ int run(Mode mode, const MjGrpoDesc* d, const void* hidden, const void* lm_head,
                                                                            h.ld_dh, rs, state, h.dv, h.wv);
       }
 
-      // the token-side operand of the dW product, k-contiguous: (rs * hidden)^T while the 16-bit matrix
+      // the token-side operand of the dW product in fragment order: (rs * hidden)^T while the 16-bit matrix
       // holds E, hidden^T once it holds dZ (the state word is final by now)
       {
         Timed t(MJ_GRPO_K_SCALE_HIDDEN, st);
         mj::k_scale_hidden<<<dim3((unsigned)(n_pad / 64), (unsigned)((H + 63) / 64)), 256, 0, st>>>(
-            (const uint16_t*)hid_c, ld_hid, rs, state, nc, n_pad, H, hs);
+            (const uint16_t*)hid_c, ld_hid, rs, state, n_live, (int)c0, nc, n_pad, H, hs);
       }
       mj::DwArgs w;
       w.dzt = (const __bf16*)zt; w.ht = (const __bf16*)hs; w.ld_z = p.ld_z;

@@ -11,7 +11,7 @@
 //   k_dhidden       : dHidden[n,H] = rowscale * (E or dZ) * W^T, optionally split over the vocab into
 //                     fp32 partial sums that k_dhidden_reduce adds up.
 //   k_scale_hidden  : (rs * hidden)^T, or hidden^T behind a kStatsMax pass: the token-side operand of
-//                     the dW product with the tokens contiguous, [H, n_pad] bf16.
+//                     the dW product in fragment order, bf16.
 //   k_dw            : dW^T tile [vocab x hidden] = (E or dZ)^T * (rs * hidden or hidden), written /
 //                     accumulated into dW[H,V] with 16-byte accesses.
 //   k_dz            : only behind a kStatsMax pass: in place, logits -> dZ (bf16).
@@ -683,14 +683,16 @@ __global__ __launch_bounds__(kFinTokens * kFinSlices) void k_finalize(FinalizeAr
   }
 }
 
-// The token-side operand of the dW product, k-contiguous: ht[h, t] = c_t * hidden[t, h] as a
-// [H, n_pad] bf16 matrix, c_t = rs[t] while the 16-bit matrix holds E and 1 once it holds dZ; zeros
-// for t >= n.  One workgroup transposes 64 tokens x 64 columns through the LDS.
+// The token-side operand of the dW product in fragment order (FragOperand: rows = hidden columns, k = tokens):
+// c_t * hidden[t, h], c_t = rs[t] while the 16-bit matrix holds E and 1 once it holds dZ; zeros for tokens that take no
+// part.  One workgroup transposes 64 tokens x 64 columns through the LDS.
 __global__ __launch_bounds__(256) void k_scale_hidden(const uint16_t* hid, int64_t ld_hid, const float* rs,
-                                                  const int* state, int n, int n_pad, int H, uint16_t* ht) {
+                                                  const int* state, const int* n_live, int c0, int n, int n_pad, int H,
+                                                  uint16_t* ht) {
   __shared__ uint16_t tile[64][72];            // [token][column]; 144-byte rows keep the 16-byte writes aligned
   const int t0 = blockIdx.x * 64, h0 = blockIdx.y * 64;
   const bool scaled = *state == 0;
+  if (n_live != nullptr) n = min(n, *n_live - c0);   // tokens past the live ones take no part
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int id = threadIdx.x + 256 * i, row = id >> 3, c = (id & 7) * 8;
@@ -708,12 +710,12 @@ __global__ __launch_bounds__(256) void k_scale_hidden(const uint16_t* hid, int64
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const int id = threadIdx.x + 256 * i, h = id >> 3, c = (id & 7) * 8;
-    if (h0 + h >= H) continue;
+    // block i's column block w of 16 (w: the wavefront), token block i of 32: lane l has column l % 16, tokens 8 (l / 16) on
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63, h = w * 16 + (l & 15), c = i * 32 + (l >> 4) * 8;
     u32x4 out;
 #pragma unroll
     for (int j = 0; j < 4; ++j) out[j] = (uint32_t)tile[c + 2 * j][h] | ((uint32_t)tile[c + 2 * j + 1][h] << 16);
-    *(u32x4*)(ht + (int64_t)(h0 + h) * n_pad + t0 + c) = out;
+    if (h0 + w * 16 < H) *(u32x4*)(ht + ((int64_t)(t0 / 32 + i) * ((H + 15) / 16) + h0 / 16 + w) * 512 + l * 8) = out;
   }
 }
 
@@ -933,7 +935,7 @@ __global__ __launch_bounds__(256) void k_dhidden_reduce(const float* part, int s
 
 struct DwArgs {
   const __bf16* dzt;   // [n, ld_z] E or dZ of the chunk
-  const __bf16* ht;    // [H, n_pad]: k_scale_hidden's matrix, the token-side operand
+  const __bf16* ht;    // k_scale_hidden's matrix, the token-side operand in fragment order
   int64_t ld_z;
   int H, V, n;         // n = tokens of the chunk
   void* dw;            // [H, ld_dw]: f32, or bf16 in the BF16OUT kernel
@@ -945,15 +947,15 @@ struct DwArgs {
 };
 
 // Tile of dW^T: rows = vocab (MFMA row direction), columns = hidden (lanes), on the chained
-// 16 x 16 x 32 engine (GemmTN16).  The token-side operand is k_scale_hidden's [H, n_pad] matrix, so
-// only E / dZ (token-major in memory) goes through the transposing LDS read; the token rows of dead
+// 16 x 16 x 32 engine (GemmTN16).  The token-side operand is k_scale_hidden's matrix in fragment order, so
+// only E / dZ (token-major in memory) goes through the LDS, by the transposing read; the token rows of dead
 // tokens are not fetched.  A lane's four accumulator rows of a block are four consecutive entries of
 // one dW row: one 16-byte access per block in float32; in bf16 the lanes l and l + 16 exchange, two
 // blocks at a time, so that each owns eight consecutive entries (an accumulating call adds in fp32
 // and rounds once).
 template <int BM, int BN, bool BF16OUT>
 __global__ __launch_bounds__(kThreads) void k_dw(DwArgs p, TileMap map) {
-  using G = GemmTN16<BM, BN, kKRow, kRowK, true, false>;
+  using G = GemmTN16<BM, BN, kKRow, kFrag, true, false>;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   int tm, tn, split;
   if (!map.tile(blockIdx.x, tm, tn, split)) return;
@@ -961,7 +963,7 @@ __global__ __launch_bounds__(kThreads) void k_dw(DwArgs p, TileMap map) {
   G g;
   const int n_pad = (p.n + 255) & ~255;
   const int kn = min(p.n, live_pad(p.n_live, p.c0, n_pad));   // tokens past the live ones have dZ = 0
-  g.run(p.dzt + m0, p.V - m0, p.ld_z, p.ht + (int64_t)n0 * n_pad, p.H - n0, n_pad, kn, smem, threadIdx.x, p.dead);
+  g.run(p.dzt + m0, p.V - m0, p.ld_z, p.ht + n0 * 32, p.H - n0, (p.H + 15) / 16, kn, smem, threadIdx.x, p.dead);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform: keeps descriptors in SGPRs
   const int wm = wave & 1, wn = wave >> 1, l15 = lane & 15, lq = lane >> 4;
@@ -1014,6 +1016,11 @@ __global__ __launch_bounds__(kThreads) void k_dw(DwArgs p, TileMap map) {
 #pragma unroll
   for (int ni = 0; ni < G::NI; ++ni) {
     const uint32_t lane_off = (uint32_t)((ni * 16 + l15) * ld4 + lq * 16);
+    // an opaque use of the column's accumulators, as in logits_tile16: none is parked in scratch memory
+#pragma unroll
+    for (int mi = 0; mi < G::MI; ++mi)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) asm volatile("" : "+v"(g.acc[mi][ni][r]));
     // when accumulating, the eight loads of this column of blocks are issued before the first store (a
     // store between two loads would order the second behind it: one memory round trip per 16 bytes)
     f32x4 a[G::MI];

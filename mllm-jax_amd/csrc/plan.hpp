@@ -123,7 +123,7 @@ inline int make_plan(const MjGrpoDesc* d, Plan* p) {
   p->dh_p = take(p->compact ? (size_t)p->N * p->H * 2 : 0);
   p->rs = take((size_t)p->n_pad * 4);
   p->dead = take((size_t)p->n_pad / 8);     // one bit per token of a chunk
-  p->hs = take((size_t)p->n_pad * p->H * 2);
+  p->hs = take((size_t)p->n_pad * rup(p->H, 16) * 2);
   p->zt = take((size_t)p->n_pad * p->ld_z * 2);
   p->part = take(p->dh_splits > 1 ? (size_t)p->dh_splits * p->n_pad * p->H * 4 : 0);
   p->total_bwd = o;

@@ -126,7 +126,7 @@ static void check_plan(const MjGrpoDesc& d, bool launches = true) {
   r.push_back({p.dh_p, p.compact ? (size_t)p.N * p.H * 2 : 0, "dh_p"});
   r.push_back({p.rs, np4, "rs"});
   r.push_back({p.dead, (size_t)p.n_pad / 8, "dead"});
-  r.push_back({p.hs, (size_t)p.n_pad * p.H * 2, "hs"});
+  r.push_back({p.hs, (size_t)p.n_pad * rup(p.H, 16) * 2, "hs"});
   r.push_back({p.zt, (size_t)p.n_pad * p.ld_z * 2, "zt"});
   r.push_back({p.part, p.dh_splits > 1 ? (size_t)p.dh_splits * p.n_pad * p.H * 4 : 0, "part"});
   const size_t bwd_regions = r.size();
