@@ -93,7 +93,9 @@ int mj_grpo_version(void);
 /* Message of the calling thread's last non-zero status ("" if none). */
 const char* mj_grpo_last_error(void);
 
-/* Workspace sizes in bytes for the three entry points below. */
+/* Workspace sizes in bytes for the three entry points below.  The last part of a large forward pass's holds a copy of
+ * a chunk's hidden states in another order (2 bytes x chunk rounded up to 256 x hidden rounded up to 64); mj_grpo_forward
+ * takes a workspace without it too and computes the same bits, up to a tenth slower. */
 int mj_grpo_workspace_bytes(const MjGrpoDesc* desc, size_t* forward_bytes,
                             size_t* forward_backward_bytes);
 

@@ -697,11 +697,12 @@ struct GemmTN16 {
     };
     // One block: its two matrix instructions with the period's memory instruction `slot` between them.
     auto block = [&](auto init, auto lead, auto settle, auto set, int i, int j, int s, int slot, bool first_period) {
-      constexpr int S = kFragB ? decltype(set)::value : 0;
+      constexpr int S = kFragB ? decltype(set)::value & 1 : 0;
+      constexpr bool kNext = kFragB && decltype(set)::value < 2;      // 2: set 0, nothing follows
       first(init, lead, i, S * NI + j);
       __builtin_amdgcn_sched_barrier(0);
       mem_op(s, slot, first_period);
-      if (kFragB && slot >= 16 && slot % 3 == 2) load_b(IntTag<kFragB ? 1 - S : 0>(), (slot - 16) / 3);
+      if (kNext && slot >= 16 && slot % 3 == 2) load_b(IntTag<kFragB ? 1 - S : 0>(), (slot - 16) / 3);
       __builtin_amdgcn_sched_barrier(0);
       second(settle, i, S * NI + j);
       __builtin_amdgcn_sched_barrier(0);
@@ -782,14 +783,19 @@ struct GemmTN16 {
           rows_back(IntTag<0>(), IntTag<1>(), IntTag<0>(), s + 1);
           rows_front(IntTag<0>(), IntTag<1>(), s + 1, false);
         }
+        // an odd number of slices: the last one's fragments change sets, so that the last two rows are one
+        // piece of code (as two, behind a branch, the allocator moved accumulators between registers)
         if (s < KT) {
           publish();
           rows_back(IntTag<0>(), IntTag<1>(), IntTag<1>(), s);
-          rows_front(IntTag<0>(), IntTag<0>(), s, false);
-          rows_back(IntTag<0>(), IntTag<0>(), IntTag<0>(), KT);
-        } else {
-          rows_back(IntTag<0>(), IntTag<0>(), IntTag<1>(), KT);
+          rows_front(IntTag<0>(), IntTag<2>(), s, false);
+#pragma unroll
+          for (int j = 0; j < NI; ++j) {
+            fb[NI + j][0] = fb[j][0];
+            fb[NI + j][1] = fb[j][1];
+          }
         }
+        rows_back(IntTag<0>(), IntTag<0>(), IntTag<1>(), KT);
       }
     }
   }

@@ -47,7 +47,7 @@ bool misaligned(const void* p) { return ((uintptr_t)p & 15u) != 0; }
 // the function on a device: it is set on the first call that launches that kernel on that device,
 // whatever thread makes it (one process-wide table under a mutex), never again afterwards.
 constexpr int kMaxDevices = 64;
-constexpr int kMaxTileKernels = 32;       // tile-kernel instantiations in this file: 15
+constexpr int kMaxTileKernels = 32;       // tile-kernel instantiations in this file: 17
 struct LdsDone {
   const void* fn;
   bool dev[kMaxDevices];
@@ -148,10 +148,20 @@ int run(Mode mode, const MjGrpoDesc* d, const void* hidden, const void* lm_head,
   uint64_t* dead = (uint64_t*)(ws + p.dead);
   // the logits kernels exist with and without the softcap code (a template parameter)
   const bool cap = d->softcap > 0.f;
-  auto k_grad = cap ? mj::k_logits_stats<BM, BN, mj::kStatsGrad, false, true> : mj::k_logits_stats<BM, BN, mj::kStatsGrad, false, false>;
-  auto k_exp = cap ? mj::k_logits_stats<BM, BN, mj::kStatsExp, false, true> : mj::k_logits_stats<BM, BN, mj::kStatsExp, false, false>;
-  auto k_max = cap ? mj::k_logits_stats<BM, BN, mj::kStatsMax, false, true> : mj::k_logits_stats<BM, BN, mj::kStatsMax, false, false>;
-  auto k_max_rescue = cap ? mj::k_logits_stats<BM, BN, mj::kStatsMax, true, true> : mj::k_logits_stats<BM, BN, mj::kStatsMax, true, false>;
+  // hidden in fragment order: one more pass over [n, H], and a workspace that has room for it
+  uint16_t* hid_frag = nullptr;
+  if (mode != kBackwardOnly && fragment_hidden(p.chunk, H, V) && (bwd || ws_bytes >= p.total_fwd_frag)) hid_frag = (uint16_t*)(ws + (bwd ? p.hs : p.hid_frag));
+  using LogitsKernel = void (*)(mj::LogitsArgs, mj::TileMap);
+  const LogitsKernel k_grad = cap ? mj::k_logits_stats<BM, BN, mj::kStatsGrad, false, true, false> : mj::k_logits_stats<BM, BN, mj::kStatsGrad, false, false, false>;
+  const LogitsKernel k_max_rescue = cap ? mj::k_logits_stats<BM, BN, mj::kStatsMax, true, true, false> : mj::k_logits_stats<BM, BN, mj::kStatsMax, true, false, false>;
+  LogitsKernel k_exp, k_max;
+  if (hid_frag != nullptr) {
+    k_exp = cap ? mj::k_logits_stats<BM, BN, mj::kStatsExp, false, true, true> : mj::k_logits_stats<BM, BN, mj::kStatsExp, false, false, true>;
+    k_max = cap ? mj::k_logits_stats<BM, BN, mj::kStatsMax, false, true, true> : mj::k_logits_stats<BM, BN, mj::kStatsMax, false, false, true>;
+  } else {
+    k_exp = cap ? mj::k_logits_stats<BM, BN, mj::kStatsExp, false, true, false> : mj::k_logits_stats<BM, BN, mj::kStatsExp, false, false, false>;
+    k_max = cap ? mj::k_logits_stats<BM, BN, mj::kStatsMax, false, true, false> : mj::k_logits_stats<BM, BN, mj::kStatsMax, false, false, false>;
+  }
   if (mode == kBackwardOnly) {
     if ((rc = enable_lds(k_grad))) return rc;
   } else {
@@ -235,7 +245,7 @@ int run(Mode mode, const MjGrpoDesc* d, const void* hidden, const void* lm_head,
     a.zt = bwd ? zt : nullptr; a.ld_z = p.ld_z;
     a.pm = pm; a.pl = pl; a.ps = ps; a.plt = plt; a.inv_t = inv_t; a.ld_p = p.n_pad;
     a.targets = targets + c0; a.zy = zy + c0; a.n_live = n_live; a.c0 = (int)c0;
-    a.mask = mask + c0; a.lse = nullptr; a.g = g; a.state = state;
+    a.mask = mask + c0; a.lse = nullptr; a.g = g; a.state = state; a.hid_frag = (const __bf16*)hid_frag;
     const mj::TileMap map((V + BM - 1) / BM, (nc + BN - 1) / BN, 1, 1);
 
     mj::FinalizeArgs f;
@@ -259,6 +269,10 @@ int run(Mode mode, const MjGrpoDesc* d, const void* hidden, const void* lm_head,
     z.V = V; z.n = nc; z.cap = d->softcap; z.n_live = n_live; z.c0 = (int)c0; z.state = state; z.rescue = 0;
     const unsigned dz_grid = (unsigned)(nc < 8192 ? nc : 8192);
 
+    if (hid_frag != nullptr) {
+      Timed t(MJ_GRPO_K_SCALE_HIDDEN, st);
+      mj::k_fragment_rows<<<dim3((unsigned)(n_pad / 16), (unsigned)((H + 127) / 128)), 256, 0, st>>>((const uint16_t*)hid_c, ld_hid, nc, H, hid_frag);
+    }
     if (mode == kBackwardOnly) {
       {
         Timed t(MJ_GRPO_K_FINALIZE, st);
@@ -388,7 +402,7 @@ int mj_grpo_workspace_bytes(const MjGrpoDesc* desc, size_t* forward_bytes, size_
   Plan p;
   int rc = make_plan(desc, &p);
   if (rc) return rc;
-  if (forward_bytes) *forward_bytes = p.total_fwd;
+  if (forward_bytes) *forward_bytes = fragment_hidden(p.chunk, p.H, p.V) ? p.total_fwd_frag : p.total_fwd;
   if (forward_backward_bytes) *forward_backward_bytes = p.total_bwd;
   return MJ_GRPO_OK;
 }
@@ -752,14 +766,18 @@ int mj_rmsnorm_backward(const void* dy, int64_t ld_dy, const void* x, int64_t ld
 }  // extern "C"
 
 // Explicit instantiations of the tile kernels used above.
-template __global__ void mj::k_logits_stats<256, 256, mj::kStatsExp, false, false>(mj::LogitsArgs, mj::TileMap);
-template __global__ void mj::k_logits_stats<256, 256, mj::kStatsExp, false, true>(mj::LogitsArgs, mj::TileMap);
-template __global__ void mj::k_logits_stats<256, 256, mj::kStatsMax, false, false>(mj::LogitsArgs, mj::TileMap);
-template __global__ void mj::k_logits_stats<256, 256, mj::kStatsMax, false, true>(mj::LogitsArgs, mj::TileMap);
-template __global__ void mj::k_logits_stats<256, 256, mj::kStatsMax, true, false>(mj::LogitsArgs, mj::TileMap);
-template __global__ void mj::k_logits_stats<256, 256, mj::kStatsMax, true, true>(mj::LogitsArgs, mj::TileMap);
-template __global__ void mj::k_logits_stats<256, 256, mj::kStatsGrad, false, false>(mj::LogitsArgs, mj::TileMap);
-template __global__ void mj::k_logits_stats<256, 256, mj::kStatsGrad, false, true>(mj::LogitsArgs, mj::TileMap);
+template __global__ void mj::k_logits_stats<256, 256, mj::kStatsExp, false, false, false>(mj::LogitsArgs, mj::TileMap);
+template __global__ void mj::k_logits_stats<256, 256, mj::kStatsExp, false, true, false>(mj::LogitsArgs, mj::TileMap);
+template __global__ void mj::k_logits_stats<256, 256, mj::kStatsExp, false, false, true>(mj::LogitsArgs, mj::TileMap);
+template __global__ void mj::k_logits_stats<256, 256, mj::kStatsExp, false, true, true>(mj::LogitsArgs, mj::TileMap);
+template __global__ void mj::k_logits_stats<256, 256, mj::kStatsMax, false, false, false>(mj::LogitsArgs, mj::TileMap);
+template __global__ void mj::k_logits_stats<256, 256, mj::kStatsMax, false, true, false>(mj::LogitsArgs, mj::TileMap);
+template __global__ void mj::k_logits_stats<256, 256, mj::kStatsMax, false, false, true>(mj::LogitsArgs, mj::TileMap);
+template __global__ void mj::k_logits_stats<256, 256, mj::kStatsMax, false, true, true>(mj::LogitsArgs, mj::TileMap);
+template __global__ void mj::k_logits_stats<256, 256, mj::kStatsMax, true, false, false>(mj::LogitsArgs, mj::TileMap);
+template __global__ void mj::k_logits_stats<256, 256, mj::kStatsMax, true, true, false>(mj::LogitsArgs, mj::TileMap);
+template __global__ void mj::k_logits_stats<256, 256, mj::kStatsGrad, false, false, false>(mj::LogitsArgs, mj::TileMap);
+template __global__ void mj::k_logits_stats<256, 256, mj::kStatsGrad, false, true, false>(mj::LogitsArgs, mj::TileMap);
 template __global__ void mj::k_dhidden<256, 256>(mj::DhArgs, mj::TileMap);
 template __global__ void mj::k_dw<256, 256, false>(mj::DwArgs, mj::TileMap);
 template __global__ void mj::k_dw<256, 256, true>(mj::DwArgs, mj::TileMap);

@@ -5,6 +5,7 @@
 //                     place; the epilogue applies the softcap, reduces (sum exp, sum exp*z) per token
 //                     over the tile's vocab rows, picks out the sampled token's logit and (training)
 //                     stores a 16-bit row-major [n, V] matrix for the backward (see StatsMode).
+//   k_fragment_rows : (large products) hidden in fragment order for k_logits_stats.
 //   k_finalize      : adds up the per-tile statistics -> lse, logp, entropy, ratio / clip / min
 //                     surrogate, per-token loss term, dloss/dlogp, the row scale of E and its
 //                     one-hot patch.
@@ -117,6 +118,7 @@ struct LogitsArgs {
   const int* n_live;        // null, or device count of leading tokens (from token c0 on) that need a backward
   int c0;
   const float* mask;        // chunk origin; rows of tokens with mask == 0 are not stored
+  const __bf16* hid_frag;   // hidden of the chunk in fragment order (k_fragment_rows), or nullptr
   const float *lse, *g;     // kStatsGrad: chunk-local saved logsumexp [n] and dloss/dlogp [n_pad]
   int* state;
 };
@@ -300,9 +302,12 @@ MJ_DEV float max_rows16(float x) {
 // accumulators in rotation) until its epilogue was written for this tile's layout: an actor-critic pass of
 // 2048 x 1536 x 151936 takes 3019 us instead of 3121.
 constexpr int kTileExtraLds = 2048;
-template <int BM, int BN, int MODE, bool CAP>
+// FRAG: hidden comes in fragment order, without the LDS (GemmTN16): 14.49 -> 13.07 ms at 16384 x 3584 x 152064, 4.39 ->
+// 4.05 at 5005 tokens, 1.94 -> 1.76 at 2049 x 4096 x 128256; the same sums bit for bit.  Where the copy of hidden is
+// worth its pass: fragment_hidden (plan.hpp).
+template <int BM, int BN, int MODE, bool CAP, bool FRAG>
 MJ_DEV void logits_tile16(const LogitsArgs& p, int tm, int tn, char* smem, int tid) {
-  using G = GemmTN16<BM, BN, kKRow, kRowK>;
+  using G = GemmTN16<BM, BN, kKRow, FRAG ? kFrag : kRowK>;
   static_assert(BN == kThreads, "one token of the tile per thread");
   static_assert(MODE != kStatsGrad, "kStatsGrad runs on logits_tile_grad");
   // CAP: the epilogue's logits are in units of log2 in kStatsExp, in natural units in kStatsMax
@@ -313,7 +318,8 @@ MJ_DEV void logits_tile16(const LogitsArgs& p, int tm, int tn, char* smem, int t
   const float mask_t = tok < p.n ? p.mask[tok] : 0.f;
   const int target_t = tok < p.n ? clamp_target(p.targets[tok], p.V) : -1;
   G g;
-  g.run(p.w + m0, p.V - m0, p.ld_w, p.hid + (int64_t)n0 * p.ld_hid, p.n - n0, p.ld_hid, p.H, smem, tid);
+  if constexpr (FRAG) g.run(p.w + m0, p.V - m0, p.ld_w, p.hid_frag + n0 * 32, p.n - n0, ((p.n + 255) & ~255) / 16, p.H, smem, tid);
+  else g.run(p.w + m0, p.V - m0, p.ld_w, p.hid + (int64_t)n0 * p.ld_hid, p.n - n0, p.ld_hid, p.H, smem, tid);
   float* tile_mask = (float*)(smem + G::kLdsBytes);
   int* tile_target = (int*)(tile_mask + BN);
   tile_mask[tid] = mask_t;
@@ -509,7 +515,7 @@ MJ_DEV int opaque_tid() {
 
 // One workgroup per tile; RESCUE: a small grid that walks the tile list, and leaves at once unless
 // the range check of the kStatsExp pass failed (state != 0).
-template <int BM, int BN, int MODE, bool RESCUE, bool CAP>
+template <int BM, int BN, int MODE, bool RESCUE, bool CAP, bool FRAG>
 __global__ __launch_bounds__(kThreads) void k_logits_stats(LogitsArgs p, TileMap map) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   int tm, tn, split;
@@ -518,15 +524,26 @@ __global__ __launch_bounds__(kThreads) void k_logits_stats(LogitsArgs p, TileMap
     if (__builtin_amdgcn_readfirstlane(*p.state) == 0) return;
     const int items = map.items();
     for (int item = blockIdx.x; item < items; item += gridDim.x) {
-      if (map.tile(item, tm, tn, split)) logits_tile16<BM, BN, MODE, CAP>(p, tm, tn, smem, opaque_tid());
+      if (map.tile(item, tm, tn, split)) logits_tile16<BM, BN, MODE, CAP, FRAG>(p, tm, tn, smem, opaque_tid());
       __syncthreads();      // the next tile's first LDS writes must not pass this tile's last reads
     }
   } else {
     if (MODE == kStatsExp && blockIdx.x == 0 && threadIdx.x == 0) *p.state = 0;
     if (!map.tile(blockIdx.x, tm, tn, split)) return;
     if constexpr (MODE == kStatsGrad) logits_tile_grad<BM, BN, CAP>(p, tm, tn, smem, threadIdx.x);
-    else logits_tile16<BM, BN, MODE, CAP>(p, tm, tn, smem, threadIdx.x);
+    else logits_tile16<BM, BN, MODE, CAP, FRAG>(p, tm, tn, smem, threadIdx.x);
   }
+}
+
+// Rows of a bf16 matrix in fragment order (FragOperand): [n, H] with pitch ld -> blocks of 16 rows x 32 columns, zeros
+// past n and H.  A wavefront writes a block; the four of a workgroup read 256 contiguous bytes of each of 16 rows.
+__global__ __launch_bounds__(256) void k_fragment_rows(const uint16_t* in, int64_t ld, int n, int H, uint16_t* out) {
+  const int kb = blockIdx.y * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int t = blockIdx.x * 16 + (lane & 15), k = kb * 32 + (lane >> 4) * 8;
+  if (kb * 32 >= ((H + kBK - 1) & ~(kBK - 1))) return;
+  u32x4 v = {0u, 0u, 0u, 0u};
+  if (t < n && k < H) v = *(const u32x4*)(in + (int64_t)t * ld + k);
+  *(u32x4*)(out + ((int64_t)kb * gridDim.x + blockIdx.x) * 512 + lane * 8) = v;
 }
 
 // ----------------------------------------------------------------------------- finalize

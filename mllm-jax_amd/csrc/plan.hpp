@@ -39,6 +39,9 @@ struct Plan {
   int64_t dh_k_per_split;
   // byte offsets into the workspace
   size_t zy, term, eterm, pm, pl, ps, plt, g, ge, hent, state, rs, dead, hs, zt, part, total_fwd, total_bwd;
+  // hidden of a chunk in fragment order: behind the regions of a forward pass, which runs without it in a workspace of
+  // total_fwd bytes; in `hs` in a backward pass (the logits product is done with it before hs is written)
+  size_t hid_frag, total_fwd_frag;
   // token compaction (MJ_GRPO_FLAG_SKIP_MASKED): slot-order copies of the inputs and outputs
   bool compact;
   size_t perm, n_live, hid_p, tgt_p, fin_p[5], fout_p[3], dh_p;
@@ -97,6 +100,7 @@ inline int make_plan(const MjGrpoDesc* d, Plan* p) {
   p->dh_k_per_split = rup((p->V + p->dh_splits - 1) / p->dh_splits, 64);
   // pieces are whole 64-wide slices: a small vocabulary has fewer of them than the splits asked for
   p->dh_splits = (int)((p->V + p->dh_k_per_split - 1) / p->dh_k_per_split);
+  const size_t frag_bytes = (size_t)p->n_pad * rup(p->H, 64) * 2;   // also of (rs * hidden)^T in whole 16-row blocks
   size_t o = 0;
   auto take = [&](size_t bytes) { size_t at = o; o = (size_t)rup((int64_t)(o + bytes), 256); return at; };
   p->zy = take((size_t)p->N * 4);
@@ -119,11 +123,12 @@ inline int make_plan(const MjGrpoDesc* d, Plan* p) {
     for (auto& f : p->fin_p) f = take((size_t)p->N * 4);
     for (auto& f : p->fout_p) f = take((size_t)p->N * 4);
   }
-  p->total_fwd = o;
+  p->total_fwd = p->hid_frag = o;
+  p->total_fwd_frag = (size_t)rup((int64_t)(o + frag_bytes), 256);
   p->dh_p = take(p->compact ? (size_t)p->N * p->H * 2 : 0);
   p->rs = take((size_t)p->n_pad * 4);
   p->dead = take((size_t)p->n_pad / 8);     // one bit per token of a chunk
-  p->hs = take((size_t)p->n_pad * rup(p->H, 16) * 2);
+  p->hs = take(frag_bytes);
   p->zt = take((size_t)p->n_pad * p->ld_z * 2);
   p->part = take(p->dh_splits > 1 ? (size_t)p->dh_splits * p->n_pad * p->H * 4 : 0);
   p->total_bwd = o;
@@ -134,6 +139,13 @@ inline int make_plan(const MjGrpoDesc* d, Plan* p) {
   p->total_value = o;
   return MJ_GRPO_OK;
 }
+
+// Whether the logits product reads hidden in fragment order.  The product gains with its size, the pass that writes the
+// copy (k_fragment_rows) is a launch of 5 us at the least.  Product without, with, and the pass, us:
+//   512 x 896 x 151936   181  176  5.4      1024 x 896 x 151936   324  324  5.4     512 x 1536 x 151936  250  253  5.7
+//   512 x 2304 x 152064  343  335  5.4      1024 x 1536 x 151936  479  464  6.8     512 x 4096 x 128256  473  443  6.6
+//   4096 x 1536 x 151936 1739 1687  9.8     5005 x 3584 x 152064 4393 4048 14.2     16384 x 3584 x 152064 14489 13073 38
+inline bool fragment_hidden(int64_t n, int64_t h, int64_t v) { return (double)n * (double)h * (double)v >= 1.6e11; }
 
 // mj_grpo_forward_noalloc: the plan whose forward workspace fits `scratch_bytes`.  chunk_tokens == 0
 // picks the largest chunk (a multiple of 256 tokens, at most 16384) that fits.

@@ -43,3 +43,38 @@ def test_edges_of_blocks_slices_and_tiles(n, h, v, skip):
     # no token and no hidden column of its own is wrong, at the edges in particular
     assert (_rel(dh, ref["d_hidden"], 1)[mask.numpy() != 0] <= 4 * RTOL).all() and not dh[mask.numpy() == 0].any()
     assert (_rel(dw, ref["d_lm_head"], 1) <= 4 * RTOL).all()
+
+
+@pytest.mark.parametrize("n,h,v,cap", [(1100, 1032, 152064, 0.0), (2049, 1000, 80008, 0.0), (300, 4088, 131080, 20.0), (401, 8160, 50000, 0.0)])
+def test_logits_of_hidden_in_fragment_order_are_the_same_bits(n, h, v, cap):
+    """Ragged tokens, hidden sizes that end inside a block of 32 and a slice of 64 with an odd and an even number of
+    slices: a workspace without room for the reordered copy takes the path that reads hidden in place."""
+    import ctypes as C
+
+    from mllm_jax_amd import _lib
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(h)
+    hid = torch.randn(n, h + 8, generator=g, device=dev).to(torch.bfloat16)       # row pitch of its own
+    hid[:, h:] = float("nan")
+    w = (torch.randn(h, v, generator=g, device=dev) / np.sqrt(h)).to(torch.bfloat16)
+    y = torch.randint(0, v, (n,), generator=g, device=dev, dtype=torch.int32)
+    ones = torch.ones(n, device=dev)
+    d = _lib.MjGrpoDesc()
+    d.n_tokens, d.hidden, d.vocab, d.ld_hidden, d.ld_w = n, h, v, h + 8, v
+    d.eps_low = d.eps_high = 0.2
+    d.temperature, d.softcap, d.inv_total_valid_tokens, d.grad_loss_scale = 1.0, cap, 1.0 / n, 1.0
+    full, _ = _lib.workspace_bytes(d)
+    copy = -(-n // 256) * 256 * (-(-h // 64) * 64) * 2
+    runs = []
+    for nbytes in (full, full - copy):
+        ws = torch.full((nbytes,), 255, dtype=torch.uint8, device=dev)             # NaNs wherever it is read unwritten
+        logp, lse, ent, loss = (torch.empty(k, device=dev) for k in (n, n, n, 2))
+        _lib.check(_lib.load().mj_grpo_forward(C.byref(d), hid.data_ptr(), w.data_ptr(), y.data_ptr(), None, ones.data_ptr(), ones.data_ptr(),
+                                               logp.data_ptr(), lse.data_ptr(), ent.data_ptr(), loss.data_ptr(), ws.data_ptr(), nbytes,
+                                               torch.cuda.current_stream().cuda_stream))
+        runs.append((logp, lse, ent, loss))
+    assert all(torch.equal(a, b) for a, b in zip(*runs))
+    z = hid[:, :h].float() @ w.float()
+    z = cap * torch.tanh(z / cap) if cap else z
+    ref = torch.log_softmax(z, -1).gather(1, y.long()[:, None])[:, 0]
+    assert (runs[0][0] - ref).abs().max().item() <= 1e-3
