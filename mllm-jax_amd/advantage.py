@@ -15,6 +15,8 @@ _MODES = {"grpo": 0, "global": 1, "rloo": 2, "dapo": 3}
 
 
 def _rewards(rewards, name="rewards") -> torch.Tensor:
+    if _lib.is_plain_vector(rewards, torch.float32):
+        return rewards
     r = torch.as_tensor(rewards)
     if r.device.type != "cuda":
         raise RuntimeError(f"{name} must be a GPU tensor; the advantage estimators have no CPU path")
@@ -25,6 +27,8 @@ def _rewards(rewards, name="rewards") -> torch.Tensor:
 
 
 def _group_ids(group_ids, r: torch.Tensor) -> torch.Tensor:
+    if _lib.is_plain_vector(group_ids, torch.int32) and group_ids.device == r.device and group_ids.numel() == r.numel():
+        return group_ids
     g = torch.as_tensor(group_ids, device=r.device).reshape(-1)
     if g.numel() != r.numel():
         raise ValueError(f"group_ids must have shape [B] with B={r.numel()}, got size={g.numel()}")
@@ -44,10 +48,8 @@ def _run(mode: str, r: torch.Tensor, g: Optional[torch.Tensor], eps: float, alph
     if float(eps) <= 0:
         raise ValueError("eps must be > 0")
     out = torch.empty_like(r)
-    with torch.cuda.device(r.device):
-        _lib.check(_lib.load().mj_grpo_advantages(
-            _MODES[mode], r.data_ptr(), None if g is None else g.data_ptr(), out.data_ptr(), r.numel(), float(eps),
-            float(alpha), int(bool(whiten)), clip, torch.cuda.current_stream(r.device).cuda_stream))
+    _lib.launch(r.device, "mj_grpo_advantages", _MODES[mode], r.data_ptr(), None if g is None else g.data_ptr(), out.data_ptr(),
+                r.numel(), float(eps), float(alpha), int(bool(whiten)), clip)
     return out
 
 
@@ -108,11 +110,8 @@ def compute_gae_advantages(*, rewards, values, completion_mask, gamma: float = 1
         raise ValueError(f"values and completion_mask must match shape, got {tuple(v.shape)} vs {tuple(m.shape)}")
     v, m = v.contiguous(), m.contiguous()
     adv, ret = torch.empty_like(v), torch.empty_like(v)
-    with torch.cuda.device(r.device):
-        _lib.check(_lib.load().mj_grpo_gae(
-            r.data_ptr(), v.data_ptr(), m.data_ptr(), adv.data_ptr(), ret.data_ptr(), v.shape[0], v.shape[1],
-            float(gamma), float(gae_lambda), int(bool(normalize)), float(eps), _clip(clip_range),
-            torch.cuda.current_stream(r.device).cuda_stream))
+    _lib.launch(r.device, "mj_grpo_gae", r.data_ptr(), v.data_ptr(), m.data_ptr(), adv.data_ptr(), ret.data_ptr(), v.shape[0],
+                v.shape[1], float(gamma), float(gae_lambda), int(bool(normalize)), float(eps), _clip(clip_range))
     return adv, ret
 
 

@@ -218,11 +218,9 @@ class _Prepared:
     def forward(self) -> None:
         fwd, _ = _lib.workspace_bytes(self.desc)
         ws = _workspace(self.device, fwd)
-        with torch.cuda.device(self.device):
-            _lib.check(_lib.load().mj_grpo_forward(
-                C.byref(self.desc), _ptr(self.hidden), _ptr(self.w), _ptr(self.targets), _ptr(self.old),
-                _ptr(self.adv), _ptr(self.mask), _ptr(self.logp), _ptr(self.lse), _ptr(self.ent),
-                _ptr(self.loss), _ptr(ws), ws.numel(), self.stream()))
+        _lib.launch(self.device, "mj_grpo_forward", C.byref(self.desc), _ptr(self.hidden), _ptr(self.w), _ptr(self.targets), _ptr(self.old),
+                    _ptr(self.adv), _ptr(self.mask), _ptr(self.logp), _ptr(self.lse), _ptr(self.ent),
+                    _ptr(self.loss), _ptr(ws), ws.numel())
 
     def forward_backward(self, d_w: Optional[torch.Tensor] = None, value: Optional["_ValueHead"] = None,
                          dw_dtype: torch.dtype = torch.float32):
@@ -243,18 +241,13 @@ class _Prepared:
             self.desc.flags |= _lib.FLAG_DW_BF16
         else:
             self.desc.flags &= ~_lib.FLAG_DW_BF16
-        with torch.cuda.device(self.device):
-            if value is None:
-                _lib.check(_lib.load().mj_grpo_forward_backward(
-                    C.byref(self.desc), _ptr(self.hidden), _ptr(self.w), _ptr(self.targets), _ptr(self.old),
-                    _ptr(self.adv), _ptr(self.mask), _ptr(self.logp), _ptr(self.lse), _ptr(self.ent),
-                    _ptr(self.loss), _ptr(d_h), _ptr(d_w), _ptr(ws), ws.numel(), self.stream()))
-            else:
-                _lib.check(_lib.load().mj_grpo_forward_backward_value(
-                    C.byref(self.desc), C.byref(value.struct(self.n, self.h, self.device)), _ptr(self.hidden),
-                    _ptr(self.w), _ptr(self.targets), _ptr(self.old), _ptr(self.adv), _ptr(self.mask),
-                    _ptr(self.logp), _ptr(self.lse), _ptr(self.ent), _ptr(self.loss), _ptr(d_h), _ptr(d_w),
-                    _ptr(ws), ws.numel(), self.stream()))
+        outputs = (_ptr(self.logp), _ptr(self.lse), _ptr(self.ent), _ptr(self.loss), _ptr(d_h), _ptr(d_w), _ptr(ws), ws.numel())
+        inputs = (_ptr(self.hidden), _ptr(self.w), _ptr(self.targets), _ptr(self.old), _ptr(self.adv), _ptr(self.mask))
+        if value is None:
+            _lib.launch(self.device, "mj_grpo_forward_backward", C.byref(self.desc), *inputs, *outputs)
+        else:
+            _lib.launch(self.device, "mj_grpo_forward_backward_value", C.byref(self.desc),
+                        C.byref(value.struct(self.n, self.h, self.device)), *inputs, *outputs)
         return d_h, d_w[:, : self.v]
 
     def metrics(self, return_token_entropy: bool, sft: bool = False) -> dict:
@@ -269,9 +262,8 @@ class _Prepared:
             # per-sample masked mean entropy (:141-143) and its tokens-4..100 window (:148-157): one kernel
             b, t = self.seq_shape
             stats = torch.empty((2, b), dtype=torch.float32, device=self.device)
-            with torch.cuda.device(self.device):
-                _lib.check(_lib.load().mj_grpo_sequence_entropy(
-                    _ptr(self.ent), _ptr(self.mask), b, t, stats[0].data_ptr(), stats[1].data_ptr(), self.stream()))
+            _lib.launch(self.device, "mj_grpo_sequence_entropy", _ptr(self.ent), _ptr(self.mask), b, t, stats[0].data_ptr(),
+                        stats[1].data_ptr())
             out["entropy"], out["entropy_loss"] = stats[0], stats[1]
         if return_token_entropy:
             out["token_entropy"] = self.ent.reshape(shape)
@@ -401,13 +393,10 @@ def _apply_upstream(grad_loss: torch.Tensor, d_h: torch.Tensor, d_w: Optional[to
     device: when it is 1 -- the loss itself is what gets differentiated -- the launches leave at once
     (no pass over [N,H] or [H,V], no host synchronisation)."""
     g = grad_loss.detach().reshape(-1)[:1].to(torch.float32).contiguous()
-    with torch.cuda.device(d_h.device):
-        _lib.check(_lib.load().mj_grpo_scale_gradients(
-            d_h.data_ptr(), d_h.shape[0], d_h.shape[1], d_h.stride(0),
-            None if d_w is None else d_w.data_ptr(), 0 if d_w is None else d_w.shape[0],
-            0 if d_w is None else d_w.shape[1], 0 if d_w is None else d_w.stride(0),
-            int(d_w is not None and d_w.dtype == torch.bfloat16), g.data_ptr(),
-            torch.cuda.current_stream(d_h.device).cuda_stream))
+    _lib.launch(d_h.device, "mj_grpo_scale_gradients", d_h.data_ptr(), d_h.shape[0], d_h.shape[1], d_h.stride(0),
+                None if d_w is None else d_w.data_ptr(), 0 if d_w is None else d_w.shape[0],
+                0 if d_w is None else d_w.shape[1], 0 if d_w is None else d_w.stride(0),
+                int(d_w is not None and d_w.dtype == torch.bfloat16), g.data_ptr())
 
 
 class _FusedLossFn(torch.autograd.Function):
@@ -595,10 +584,8 @@ class PPOActorCriticModule:
         w = wv.detach().reshape(-1).to(torch.float32).contiguous()
         b = bv.detach().reshape(-1)[:1].to(torch.float32).contiguous()
         out = torch.empty(h2.shape[0], dtype=torch.float32, device=hidden.device)
-        with torch.cuda.device(hidden.device):
-            _lib.check(_lib.load().mj_value_head_forward(
-                h2.data_ptr(), h2.stride(0), w.data_ptr(), b.data_ptr(), out.data_ptr(), h2.shape[0], h2.shape[1],
-                torch.cuda.current_stream(hidden.device).cuda_stream))
+        _lib.launch(hidden.device, "mj_value_head_forward", h2.data_ptr(), h2.stride(0), w.data_ptr(), b.data_ptr(), out.data_ptr(),
+                    h2.shape[0], h2.shape[1])
         return out.reshape(shape)
 
     def value(self, input_ids, attention_mask) -> torch.Tensor:
@@ -679,6 +666,16 @@ def compute_grpo_advantages_by_group_id(*, rewards, group_ids, eps: float = 1e-4
     """Device counterpart of plugins/training/advantage/grpo.py:8-52: float32 advantages [B],
     (r - mean_g) / (std_g + eps) within each group id (population std, variable group sizes).
     `rewards` must be a GPU tensor; `group_ids` is moved beside it."""
+    if not (_lib.is_plain_vector(rewards, torch.float32) and _lib.is_plain_vector(group_ids, torch.int32)
+            and group_ids.device == rewards.device and group_ids.shape == rewards.shape):
+        rewards, group_ids = _advantage_inputs(rewards, group_ids)
+    out = torch.empty_like(rewards)
+    _lib.launch(rewards.device, "mj_grpo_group_advantages", rewards.data_ptr(), group_ids.data_ptr(), out.data_ptr(), rewards.numel(),
+                float(eps))
+    return out
+
+
+def _advantage_inputs(rewards, group_ids):
     rewards = torch.as_tensor(rewards)
     if rewards.device.type != "cuda":
         raise RuntimeError("compute_grpo_advantages_by_group_id needs GPU tensors; there is no CPU path")
@@ -690,13 +687,7 @@ def compute_grpo_advantages_by_group_id(*, rewards, group_ids, eps: float = 1e-4
                          f"{tuple(rewards.shape)}")
     if rewards.numel() == 0:
         raise ValueError("No groups found (empty batch?)")
-    r = rewards.to(torch.float32).contiguous()
-    g = group_ids.to(torch.int32).contiguous()
-    out = torch.empty_like(r)
-    with torch.cuda.device(r.device):
-        _lib.check(_lib.load().mj_grpo_group_advantages(r.data_ptr(), g.data_ptr(), out.data_ptr(), r.numel(),
-                                                        float(eps), torch.cuda.current_stream(r.device).cuda_stream))
-    return out
+    return rewards.to(torch.float32).contiguous(), group_ids.to(torch.int32).contiguous()
 
 
 def loss_and_metrics(module: Callable[[Mapping[str, Any]], dict], inputs: Mapping[str, Any]):

@@ -36,10 +36,7 @@ class _RmsNormFn(torch.autograd.Function):
         s32 = scale.detach().reshape(-1).to(torch.float32).contiguous()
         n, h = x2.shape
         y = torch.empty((n, h), dtype=torch.bfloat16, device=x.device)
-        with torch.cuda.device(x.device):
-            _lib.check(_lib.load().mj_rmsnorm_forward(
-                x2.data_ptr(), x2.stride(0), s32.data_ptr(), y.data_ptr(), h, None, n, h, float(eps),
-                torch.cuda.current_stream(x.device).cuda_stream))
+        _lib.launch(x.device, "mj_rmsnorm_forward", x2.data_ptr(), x2.stride(0), s32.data_ptr(), y.data_ptr(), h, None, n, h, float(eps))
         ctx.save_for_backward(x2, s32)
         ctx.meta = (x.shape, x.dtype, scale.shape, scale.dtype, float(eps))
         return y.reshape(x.shape).to(x.dtype)                    # cast back to the input dtype (llama.py:451)
@@ -61,11 +58,8 @@ class _RmsNormFn(torch.autograd.Function):
         if ws is None:
             _parts.clear()
             ws = _parts[key] = torch.empty(need.value, dtype=torch.uint8, device=x2.device)
-        with torch.cuda.device(x2.device):
-            _lib.check(lib.mj_rmsnorm_backward(
-                dy2.data_ptr(), dy2.stride(0), x2.data_ptr(), x2.stride(0), s32.data_ptr(), dx.data_ptr(), h,
-                ds.data_ptr(), 0, n, h, eps, ws.data_ptr(), ws.numel(),
-                torch.cuda.current_stream(x2.device).cuda_stream))
+        _lib.launch(x2.device, "mj_rmsnorm_backward", dy2.data_ptr(), dy2.stride(0), x2.data_ptr(), x2.stride(0), s32.data_ptr(),
+                    dx.data_ptr(), h, ds.data_ptr(), 0, n, h, eps, ws.data_ptr(), ws.numel())
         return dx.reshape(shape).to(x_dtype), ds.reshape(s_shape).to(s_dtype), None
 
 

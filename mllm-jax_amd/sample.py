@@ -40,10 +40,8 @@ def last_position_logits(hidden_last: torch.Tensor, lm_head: torch.Tensor,
     b, h = hid.shape
     v = w.shape[1]
     out = torch.empty((b, v), dtype=torch.float32, device=hid.device)
-    with torch.cuda.device(hid.device):
-        _lib.check(_lib.load().mj_sample_logits(
-            hid.data_ptr(), hid.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), v, b, h, v,
-            float(final_logit_softcap or 0.0), torch.cuda.current_stream(hid.device).cuda_stream))
+    _lib.launch(hid.device, "mj_sample_logits", hid.data_ptr(), hid.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), v, b, h, v,
+                float(final_logit_softcap or 0.0))
     return out
 
 
@@ -77,11 +75,9 @@ def top_k_sampling_batched(rng: Union[torch.Generator, torch.Tensor, None], logi
     need = C.c_size_t()
     _lib.check(lib.mj_sample_draw_workspace_bytes(b, v, int(k), C.byref(need)))
     ws = torch.empty(need.value, dtype=torch.uint8, device=lg.device)
-    with torch.cuda.device(lg.device):
-        _lib.check(lib.mj_sample_draw(
-            lg.data_ptr(), lg.stride(0), b, v, int(k), float(t), None if noise is None else noise.data_ptr(),
-            token.data_ptr(), None if idx is None else idx.data_ptr(), None if val is None else val.data_ptr(),
-            ws.data_ptr(), ws.numel(), torch.cuda.current_stream(lg.device).cuda_stream))
+    _lib.launch(lg.device, "mj_sample_draw", lg.data_ptr(), lg.stride(0), b, v, int(k), float(t), None if noise is None else noise.data_ptr(),
+                token.data_ptr(), None if idx is None else idx.data_ptr(), None if val is None else val.data_ptr(),
+                ws.data_ptr(), ws.numel())
     return (token, idx, val) if return_top_k else token
 
 

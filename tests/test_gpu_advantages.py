@@ -144,3 +144,24 @@ def test_global_advantages_in_place(b):
     _lib.check(_lib.load().mj_grpo_advantages(1, x.data_ptr(), None, x.data_ptr(), b, 1e-4, 0.0, 0, 1.5,
                                               torch.cuda.current_stream().cuda_stream))
     np.testing.assert_allclose(x.cpu().numpy(), O.global_normalized_advantages(r, eps=1e-4, clip_range=1.5), rtol=1e-5, atol=1e-5)
+
+
+def test_vectors_that_are_read_in_place_give_what_converted_ones_give():
+    """Contiguous float32 rewards and int32 ids go to the kernel as they are; anything else is converted first."""
+    import mllm_jax_amd as M
+    dev = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(3)
+    r = torch.randn(37, generator=g).to(dev)
+    ids = (torch.arange(37, dtype=torch.int32) // 5).to(dev)
+    wide = torch.stack([r, r + 1], 1)
+    for fn in (M.compute_grpo_advantages_by_group_id, M.compute_rloo_advantages_by_group_id, M.compute_dapo_advantages_by_group_id):
+        plain = fn(rewards=r, group_ids=ids)
+        assert plain.data_ptr() != r.data_ptr()
+        for rr, gg in ((r.double(), ids), (wide[:, 0], ids.long()), (r, ids.cpu()), (torch.nn.Parameter(r), ids)):
+            assert torch.equal(plain, fn(rewards=rr, group_ids=gg))
+        with pytest.raises(ValueError):
+            fn(rewards=r, group_ids=ids[:36])
+        with torch.cuda.stream(torch.cuda.Stream()):
+            other = fn(rewards=r, group_ids=ids)
+        torch.cuda.synchronize()
+        assert torch.equal(plain, other)
