@@ -267,7 +267,8 @@ int run(Mode mode, const MjGrpoDesc* d, const void* hidden, const void* lm_head,
     z.lse = (mode == kBackwardOnly ? saved_lse : lse) + c0; z.g = g; z.targets = targets + c0;
     z.ge = bonus ? ge : nullptr; z.hent = bonus ? hent : nullptr; z.mask = mask + c0;
     z.V = V; z.n = nc; z.cap = d->softcap; z.n_live = n_live; z.c0 = (int)c0; z.state = state; z.rescue = 0;
-    const unsigned dz_grid = (unsigned)(nc < 8192 ? nc : 8192);
+    // whole rows, or shares of them where there are few (the rescue, which leaves at once as a rule, takes whole ones)
+    const dim3 dz_grid((unsigned)(nc < 8192 ? nc : 8192), (unsigned)(nc >= 4096 ? 1 : nc >= 2048 ? 4 : 8));
 
     if (hid_frag != nullptr) {
       Timed t(MJ_GRPO_K_SCALE_HIDDEN, st);
@@ -295,15 +296,16 @@ int run(Mode mode, const MjGrpoDesc* d, const void* hidden, const void* lm_head,
       }
       {
         Timed t(MJ_GRPO_K_FINALIZE, st);
-        mj::k_finalize<mj::kStatsExp><<<n_pad / mj::kFinTokens, mj::kFinTokens * mj::kFinSlices, 0, st>>>(f);
+        if (nc < mj::kFinWide) mj::k_finalize<mj::kStatsExp, 16><<<n_pad / 16, 1024, 0, st>>>(f);
+        else mj::k_finalize<mj::kStatsExp, 32><<<n_pad / 32, 1024, 0, st>>>(f);
       }
       // the rescue: the same chunk with a running maximum; every workgroup leaves at once unless the
       // range check in k_finalize failed
       Timed t(MJ_GRPO_K_RESCUE, st);
       f.rescue = 1; z.rescue = 1;
       k_max_rescue<<<kRescueGrid, mj::kThreads, lds, st>>>(a, map);
-      mj::k_finalize<mj::kStatsMax><<<n_pad / mj::kFinTokens, mj::kFinTokens * mj::kFinSlices, 0, st>>>(f);
-      if (bwd) mj::k_dz<<<dz_grid, 256, 0, st>>>(z);
+      mj::k_finalize<mj::kStatsMax, 16><<<n_pad / 16, 1024, 0, st>>>(f);
+      if (bwd) mj::k_dz<<<dz_grid.x, 256, 0, st>>>(z);
     } else {
       {
         Timed t(MJ_GRPO_K_LOGITS_STATS, st);
@@ -311,7 +313,7 @@ int run(Mode mode, const MjGrpoDesc* d, const void* hidden, const void* lm_head,
       }
       {
         Timed t(MJ_GRPO_K_FINALIZE, st);
-        mj::k_finalize<mj::kStatsMax><<<n_pad / mj::kFinTokens, mj::kFinTokens * mj::kFinSlices, 0, st>>>(f);
+        mj::k_finalize<mj::kStatsMax, 16><<<n_pad / 16, 1024, 0, st>>>(f);
       }
       if (bwd) {
         Timed t(MJ_GRPO_K_DZ, st);

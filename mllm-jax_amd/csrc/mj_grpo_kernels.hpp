@@ -576,10 +576,14 @@ struct FinalizeArgs {
 };
 
 // block = (kFinTokens tokens) x (kFinSlices slices of the partial list): few tokens per block keep a
-// small chunk spread over many CUs (a 512-token chunk walks 1188 partials per token)
-constexpr int kFinTokens = 16, kFinSlices = 64;
-template <int MODE>
-__global__ __launch_bounds__(kFinTokens * kFinSlices) void k_finalize(FinalizeArgs p) {
+// small chunk spread over many CUs (a 512-token chunk walks 1188 partials per token), 32 make whole memory lines.  us with
+// one load of an array in flight, 16 tokens and the slices summed by the 16 threads that finish / as it is with 16 / with 32:
+// 512 tokens 13.9 / 10.9 / 11.0, 1113 21.9 / 19.1 / 20.0, 2049 13.8 / 11.0 / 11.8, 4096 18.3 / 18.1 / 17.6, 5005 (no
+// gradient) 28.4 / 24.3 / 13.8, 16384 62.7 / 60.2 / 54.7.
+constexpr int kFinWide = 4096;      // tokens of a chunk from which a block takes 32
+template <int MODE, int kFinTokens>
+__global__ __launch_bounds__(1024) void k_finalize(FinalizeArgs p) {
+  constexpr int kFinSlices = 1024 / kFinTokens;
   __shared__ float sm[kFinSlices][kFinTokens], sl[kFinSlices][kFinTokens], ss[kFinSlices][kFinTokens], st[kFinSlices][kFinTokens];
   if (MODE == kStatsMax) {
     if (p.rescue) {
@@ -592,14 +596,37 @@ __global__ __launch_bounds__(kFinTokens * kFinSlices) void k_finalize(FinalizeAr
   const int t = blockIdx.x * kFinTokens + tx;
   const bool tempered = p.inv_t != 1.f;   // then s and lt are sums under softmax(z / T)
   float m = kNegBig, l = 0.f, s = 0.f, lt = 0.f;
-  if (t < p.n) {
+  if (MODE == kStatsExp && t < p.n) {
+    constexpr int kAhead = 5;                   // loads in flight of each array (ten: the same)
+    for (int q0 = ty; q0 < p.parts; q0 += kAhead * kFinSlices) {
+      float a[kAhead], b[kAhead], c[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const int q = q0 + u * kFinSlices;
+        const int64_t o = (int64_t)q * p.ld_p + t;
+        a[u] = q < p.parts ? p.pl[o] : 0.f;
+        b[u] = q < p.parts ? p.ps[o] : 0.f;
+        c[u] = tempered && q < p.parts ? p.plt[o] : 0.f;
+      }
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        l += a[u];
+        s += b[u];
+        lt += c[u];
+      }
+    }
+    // the wavefront's slices first: fewer entries for the threads that finish
+#pragma unroll
+    for (int o = kFinTokens; o < 64; o <<= 1) {
+      l += __shfl_xor(l, o);
+      s += __shfl_xor(s, o);
+      lt += __shfl_xor(lt, o);
+    }
+  }
+  if (MODE == kStatsMax && t < p.n) {
     for (int q = ty; q < p.parts; q += kFinSlices) {
       const int64_t o = (int64_t)q * p.ld_p + t;
-      if (MODE == kStatsExp) {
-        l += p.pl[o];
-        s += p.ps[o];
-        if (tempered) lt += p.plt[o];
-      } else {
+      {
         const float mq = p.pm[o], lq = p.pl[o], sq = p.ps[o];
         const float mn = fmaxf(m, mq);
         const float a = __expf(m - mn), b = __expf(mq - mn);
@@ -627,7 +654,7 @@ __global__ __launch_bounds__(kFinTokens * kFinSlices) void k_finalize(FinalizeAr
     float M = 0.f, L = 0.f, S = 0.f, LT = 0.f;
     if (MODE == kStatsExp) {
 #pragma unroll
-      for (int i = 0; i < kFinSlices; ++i) {
+      for (int i = 0; i < kFinSlices; i += 64 / kFinTokens) {
         L += sl[i][tx];
         S += ss[i][tx];
         LT += st[i][tx];
@@ -694,9 +721,9 @@ __global__ __launch_bounds__(kFinTokens * kFinSlices) void k_finalize(FinalizeAr
     }
   }
   if (p.dead != nullptr) {
-    // the 16 finalising threads are lanes 0..15 of the block's first wavefront
+    // the finalising threads are the first lanes of the block's first wavefront
     const uint64_t bits = __ballot(dead);
-    if (tx == 0) p.dead[blockIdx.x] = (uint16_t)bits;
+    if (tx < kFinTokens / 16) p.dead[blockIdx.x * (kFinTokens / 16) + tx] = (uint16_t)(bits >> (16 * tx));
   }
 }
 
@@ -820,14 +847,18 @@ struct DzArgs {
   int rescue;          // launched behind a kStatsExp pass: leave unless state != 0
 };
 
-// Streaming, in place, after a kStatsMax pass.  A workgroup takes whole token rows: the per-token
-// constants are loaded once, every thread moves 16 bytes per step and the 256 threads cover 4 KB
-// of the row at a time.
+// Streaming, in place, after a kStatsMax pass: bound by its 4 bytes an entry of traffic.  A workgroup takes a share
+// (blockIdx.y of gridDim.y) of whole token rows: the per-token constants are loaded once, every thread moves 16 bytes
+// per access, and kAhead accesses, 4 KB of the row each, are in flight.  2048 x 151936, a quarter of the rows masked: 206 us
+// in whole rows with one access in flight, 194 so (4.8 TB/s); 256 x 64000 23 and 15.
 __global__ __launch_bounds__(256) void k_dz(DzArgs p) {
   if (p.rescue && __builtin_amdgcn_readfirstlane(*p.state) == 0) return;
+  constexpr int kAhead = 4;
   const int lim = min(p.n, live_pad(p.n_live, p.c0, (p.n + 255) & ~255));
   const float inv_cap2 = p.cap > 0.f ? 1.f / (p.cap * p.cap) : 0.f;
   const bool bonus = p.ge != nullptr;
+  const int share = ((p.V + (int)gridDim.y - 1) / (int)gridDim.y + 2047) & ~2047;
+  const int end = min(p.V, (int)(blockIdx.y + 1) * share);
   for (int t = blockIdx.x; t < lim; t += gridDim.x) {
     const float lse = p.lse[t] * kLog2e, g = p.g[t];
     const float ge = bonus ? p.ge[t] : 0.f, hent = bonus ? p.hent[t] : 0.f;
@@ -835,13 +866,19 @@ __global__ __launch_bounds__(256) void k_dz(DzArgs p) {
     // a token without a gradient: the backward products do not read its row (dead-token bits)
     if (p.mask[t] == 0.f || (!(g != 0.f) && !(ge != 0.f))) continue;
     uint16_t* row = p.zt + (int64_t)t * p.ld_z;
-    for (int v0 = threadIdx.x * 8; v0 < p.V; v0 += 256 * 8) {
-      u32x4 out = {0u, 0u, 0u, 0u};
-      {
-        const u32x4 in = *(const u32x4*)(row + v0);
+    for (int first = blockIdx.y * share + threadIdx.x * 8; first < end; first += kAhead * 2048) {
+      u32x4 in[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u)
+        if (first + u * 2048 < end) in[u] = *(const u32x4*)(row + first + u * 2048);
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const int v0 = first + u * 2048;
+        if (v0 >= end) break;
+        u32x4 out = {0u, 0u, 0u, 0u};
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          const uint32_t w = in[i >> 1];
+          const uint32_t w = in[u][i >> 1];
           const float z = f16_bits_to_f32((uint16_t)((i & 1) ? (w >> 16) : (w & 0xffffu)));
           const float t2 = fmaf(z, kLog2e, -lse);          // log2 p
           const float pr = __builtin_amdgcn_exp2f(t2);
@@ -852,8 +889,8 @@ __global__ __launch_bounds__(256) void k_dz(DzArgs p) {
           const uint32_t b = f32_to_bf16(d);
           if (i & 1) out[i >> 1] |= b << 16; else out[i >> 1] = b;
         }
+        *(u32x4*)(row + v0) = out;
       }
-      *(u32x4*)(row + v0) = out;
     }
   }
 }
