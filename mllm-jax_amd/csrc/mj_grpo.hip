@@ -354,7 +354,11 @@ int run(Mode mode, const MjGrpoDesc* d, const void* hidden, const void* lm_head,
       w.H = H; w.V = V; w.n = nc;
       w.dw = d_w; w.ld_dw = d->ld_w; w.n_live = n_live; w.c0 = (int)c0; w.dead = dead;
       w.accumulate = (c0 > 0 || (d->flags & MJ_GRPO_FLAG_DW_ACCUMULATE)) ? 1 : 0;
-      const mj::TileMap mw((V + BM - 1) / BM, (H + BN - 1) / BN, 0, 1);
+      // In strips of four V tiles walked along H: since the token side bypasses the LDS, the tiles of an XCD in
+      // strips along V (half of H wide) did not stay near enough to share their panels in its L2.  Strips along V
+      // and along H: 46.9 and 25.9 GB fetched at 16384 x 3584 x 152064; us there 12560 and 12150, 1113 tokens
+      // accumulating 1810 and 1733, 512 x 896 249 and 243, 2049 x 4096 x 128256 1827 and 1828.
+      const mj::TileMap mw((V + BM - 1) / BM, (H + BN - 1) / BN, 1, 1);
       {
         Timed t(MJ_GRPO_K_DW, st);
         if (dw_bf16) mj::k_dw<BM, BN, true><<<mw.items(), mj::kThreads, lds, st>>>(w, mw);
