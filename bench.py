@@ -26,7 +26,7 @@ PEAK_HBM_GBS = 8000.0
 # (config index, kernel); None for workloads that were not counted.
 MEASURED_TRAFFIC_BYTES = {          # default chunk (one launch of each kernel per step at configs 0-2 and 4)
     (0, "k_logits_stats"): 0.40e9, (0, "k_dhidden"): 0.42e9, (0, "k_dw"): 0.71e9,
-    (2, "k_logits_stats"): 29.61e9, (2, "k_dhidden"): 23.37e9, (2, "k_dw"): 49.11e9,
+    (2, "k_logits_stats"): 29.61e9, (2, "k_dhidden"): 23.37e9, (2, "k_dw"): 28.10e9,
 }
 TRAFFIC_SOURCE = {0: "profiles/cfg0_qwen05b_fused_fwd_bwd.txt", 2: "profiles/cfg2_qwen7b_fused_fwd_bwd.txt"}
 
